@@ -14,8 +14,9 @@
 //   I2  inverse along axis 1, keeping j < N1:       X2 -> X1
 //   I1  C2R along axis 2, keeping k < N2:           X1 -> B (3N)
 // The kernel K^ is Kernel_Arne (kernel_magnetostatic.go:25-241) integrated
-// on the GPU in FP64 (one lane per destination cell and source direction,
-// same operation order as the Go code, no FMA contraction), transformed in
+// on the GPU in FP64 (one lane per destination cell and source direction, a
+// block for the cells next to the source; same operation order as the Go
+// code, no FMA contraction), transformed in
 // FP64 by the same passes, its real first octant kept and scaled by
 // 1/(P0 P1 P2) (maxwell_convolution.go:135-223,350-388).
 #include <math.h>
@@ -43,9 +44,10 @@ hsdm::Variants& hsdm::variants(int L) {
 }
 
 // ------------------------------------------------------------------ Kernel_Arne (FP64)
-// One lane per (source direction s, destination cell (xw,yw,zw) of the
-// computed octant); images of a periodic axis are visited in the reference's
-// loop order (z outer, then y, then x), kernel_magnetostatic.go:74-183.
+// The field of the charged faces of the source cell (direction s), averaged
+// over the destination cell (xw,yw,zw) of the computed octant; images of a
+// periodic axis are visited in the reference's loop order (z outer, then y,
+// then x), kernel_magnetostatic.go:74-183.
 __device__ __forceinline__ double delta_d(int d) {
     d = d < 0 ? -d : d;
     if (d > 0) d -= 1;
@@ -57,11 +59,75 @@ __device__ __forceinline__ int first_image(int w, int size, int r1) {
     int k = (q >= 0) ? (q + size - 1) / size : -((-q) / size);
     return w + k * size;
 }
-__global__ void __launch_bounds__(64) k_kernel_arne(double* __restrict__ oct, int s0, int s1, int s2, double c0,
-                                                    double c1, double c2, int r10, int r11, int r12, int r20,
-                                                    int r21, int r22, double accuracy) {
+// Integration points of one image at cell displacement (x, y, z): source
+// points (nv, nw) on each charged face, destination points (nx, ny, nz).
+struct ArnePts {
+    int nv, nw, nx, ny, nz;
+    __device__ __forceinline__ long count() const { return (long)nv * nw * nx * ny * nz; }
+};
+__device__ __forceinline__ ArnePts arne_points(const double cs[3], int v, int w, int x, int y, int z,
+                                               double accuracy) {
 #pragma clang fp contract(off)
-    const int h0 = s0 / 2 + 1, h1 = s1 / 2 + 1, h2 = s2 / 2 + 1;
+    double L = cs[0];
+    if (cs[1] < L) L = cs[1];
+    if (cs[2] < L) L = cs[2];
+    double dx = delta_d(x) * cs[0], dy = delta_d(y) * cs[1], dz = delta_d(z) * cs[2];
+    double d = sqrt(dx * dx + dy * dy + dz * dz);
+    if (d == 0) d = L;
+    double maxSize = d / accuracy;
+    ArnePts n;
+    n.nv = 2 * (int)(fmax(cs[v] / maxSize, 1.0) + 0.5);
+    n.nw = 2 * (int)(fmax(cs[w] / maxSize, 1.0) + 0.5);
+    n.nx = (int)(fmax(cs[0] / maxSize, 1.0) + 0.5);
+    n.ny = (int)(fmax(cs[1] / maxSize, 1.0) + 0.5);
+    n.nz = (int)(fmax(cs[2] / maxSize, 1.0) + 0.5);
+    return n;
+}
+// Both faces' charge at source point (i, j) seen at destination point (aa, bb, gg).
+__device__ __forceinline__ void arne_point(const double cs[3], int u, int v, int w, const double R[3],
+                                           const ArnePts& n, double charge, int i, int j, int aa, int bb, int gg,
+                                           double B[3]) {
+#pragma clang fp contract(off)
+    double pole[3];
+    pole[v] = -(cs[v] / 2.) + cs[v] / (double)(2 * n.nv) + (double)i * (cs[v] / (double)n.nv);
+    pole[w] = -(cs[w] / 2.) + cs[w] / (double)(2 * n.nw) + (double)j * (cs[w] / (double)n.nw);
+    const double rx = R[0] - cs[0] / 2 + cs[0] / (double)(2 * n.nx) + (cs[0] / (double)n.nx) * (double)aa;
+    const double ry = R[1] - cs[1] / 2 + cs[1] / (double)(2 * n.ny) + (cs[1] / (double)n.ny) * (double)bb;
+    const double rz = R[2] - cs[2] / 2 + cs[2] / (double)(2 * n.nz) + (cs[2] / (double)n.nz) * (double)gg;
+    pole[u] = cs[u] / 2.;
+    double q0 = rx - pole[0], q1 = ry - pole[1], q2 = rz - pole[2];
+    double r = sqrt(q0 * q0 + q1 * q1 + q2 * q2);
+    double qr = charge / (4 * HS_PI_D * r * r * r);
+    const double bx = q0 * qr, by = q1 * qr, bz = q2 * qr;
+    pole[u] = -(cs[u] / 2.);
+    q0 = rx - pole[0];
+    q1 = ry - pole[1];
+    q2 = rz - pole[2];
+    r = sqrt(q0 * q0 + q1 * q1 + q2 * q2);
+    qr = -charge / (4 * HS_PI_D * r * r * r);
+    B[0] = bx + q0 * qr;
+    B[1] = by + q1 * qr;
+    B[2] = bz + q2 * qr;
+}
+struct ArneP {
+    int s0, s1, s2, r10, r11, r12, r20, r21, r22;
+    double c0, c1, c2, accuracy;
+};
+// An image with more points than this is left to k_kernel_arne_near.
+constexpr long kArneLight = 64;
+// FullTensorIdx (common/index.go:44-47): XX=0 YY=1 ZZ=2 YZ=3 XZ=4 XY=5
+__device__ __forceinline__ int tensor_idx(int a, int b) {
+    const int idx[3][3] = {{0, 5, 4}, {5, 1, 3}, {4, 3, 2}};
+    return idx[a][b];
+}
+
+// Lane (s, cell): its images one after the other while all have few points; a
+// lane that meets one of many puts itself on the list `near` (nnear entries)
+// and leaves its value to k_kernel_arne_near.
+__global__ void __launch_bounds__(64) k_kernel_arne(double* __restrict__ oct, ArneP p, unsigned* __restrict__ near,
+                                                    unsigned* __restrict__ nnear) {
+#pragma clang fp contract(off)
+    const int h0 = p.s0 / 2 + 1, h1 = p.s1 / 2 + 1, h2 = p.s2 / 2 + 1;
     const long noct = (long)h0 * h1 * h2;
     long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= 3 * noct) return;
@@ -70,75 +136,112 @@ __global__ void __launch_bounds__(64) k_kernel_arne(double* __restrict__ oct, in
     const int zw = (int)(I % h2);
     const int yw = (int)((I / h2) % h1);
     const int xw = (int)(I / ((long)h1 * h2));
-    const int size[3] = {s0, s1, s2};
-    const double cs[3] = {c0, c1, c2};
+    const double cs[3] = {p.c0, p.c1, p.c2};
     const int u = s, v = (s + 1) % 3, w = (s + 2) % 3;
-    double L = c0;
-    if (c1 < L) L = c1;
-    if (c2 < L) L = c2;
     double acc[3] = {0, 0, 0};
-    bool any = false;
-    for (int z = first_image(zw, s2, r12); z <= r22; z += s2) {
-        double R2c = (double)z * c2;
-        for (int y = first_image(yw, s1, r11); y <= r21; y += s1) {
-            double R1c = (double)y * c1;
-            for (int x = first_image(xw, s0, r10); x <= r20; x += s0) {
-                any = true;
-                double R[3] = {(double)x * c0, R1c, R2c};
-                double dx = delta_d(x) * c0, dy = delta_d(y) * c1, dz = delta_d(z) * c2;
-                double d = sqrt(dx * dx + dy * dy + dz * dz);
-                if (d == 0) d = L;
-                double maxSize = d / accuracy;
-                int nv = (int)(fmax(cs[v] / maxSize, 1.0) + 0.5);
-                int nw = (int)(fmax(cs[w] / maxSize, 1.0) + 0.5);
-                int nx = (int)(fmax(c0 / maxSize, 1.0) + 0.5);
-                int ny = (int)(fmax(c1 / maxSize, 1.0) + 0.5);
-                int nz = (int)(fmax(c2 / maxSize, 1.0) + 0.5);
-                nv *= 2;
-                nw *= 2;
-                double scale = 1 / (double)((long)nv * nw * nx * ny * nz);
-                double surface = cs[v] * cs[w];
-                double charge = surface * scale;
-                double pu1 = cs[u] / 2.;
-                double pu2 = -pu1;
-                double B[3] = {0, 0, 0};
-                double pole[3];
-                for (int i = 0; i < nv; i++) {
-                    pole[v] = -(cs[v] / 2.) + cs[v] / (double)(2 * nv) + (double)i * (cs[v] / (double)nv);
-                    for (int j = 0; j < nw; j++) {
-                        pole[w] = -(cs[w] / 2.) + cs[w] / (double)(2 * nw) + (double)j * (cs[w] / (double)nw);
-                        for (int aa = 0; aa < nx; aa++) {
-                            double rx = R[0] - c0 / 2 + c0 / (double)(2 * nx) + (c0 / (double)nx) * (double)aa;
-                            for (int bb = 0; bb < ny; bb++) {
-                                double ry = R[1] - c1 / 2 + c1 / (double)(2 * ny) + (c1 / (double)ny) * (double)bb;
-                                for (int gg = 0; gg < nz; gg++) {
-                                    double rz = R[2] - c2 / 2 + c2 / (double)(2 * nz) + (c2 / (double)nz) * (double)gg;
-                                    pole[u] = pu1;
-                                    double q0 = rx - pole[0], q1 = ry - pole[1], q2 = rz - pole[2];
-                                    double r = sqrt(q0 * q0 + q1 * q1 + q2 * q2);
-                                    double qr = charge / (4 * HS_PI_D * r * r * r);
-                                    double bx = q0 * qr, by = q1 * qr, bz = q2 * qr;
-                                    pole[u] = pu2;
-                                    q0 = rx - pole[0]; q1 = ry - pole[1]; q2 = rz - pole[2];
-                                    r = sqrt(q0 * q0 + q1 * q1 + q2 * q2);
-                                    qr = -charge / (4 * HS_PI_D * r * r * r);
-                                    B[0] += (bx + q0 * qr);
-                                    B[1] += (by + q1 * qr);
-                                    B[2] += (bz + q2 * qr);
-                                }
-                            }
-                        }
-                    }
+    bool many = false;
+    for (int z = first_image(zw, p.s2, p.r12); z <= p.r22; z += p.s2)
+        for (int y = first_image(yw, p.s1, p.r11); y <= p.r21; y += p.s1)
+            for (int x = first_image(xw, p.s0, p.r10); x <= p.r20; x += p.s0) {
+                const ArnePts n = arne_points(cs, v, w, x, y, z, p.accuracy);
+                if (n.count() > kArneLight || many) {
+                    many = true;
+                    continue;
                 }
+                const double R[3] = {(double)x * p.c0, (double)y * p.c1, (double)z * p.c2};
+                const double charge = cs[v] * cs[w] * (1 / (double)n.count());
+                double B[3] = {0, 0, 0};
+                for (int i = 0; i < n.nv; i++)
+                    for (int j = 0; j < n.nw; j++)
+                        for (int aa = 0; aa < n.nx; aa++)
+                            for (int bb = 0; bb < n.ny; bb++)
+                                for (int gg = 0; gg < n.nz; gg++) {
+                                    double o[3];
+                                    arne_point(cs, u, v, w, R, n, charge, i, j, aa, bb, gg, o);
+                                    B[0] += o[0];
+                                    B[1] += o[1];
+                                    B[2] += o[2];
+                                }
                 for (int dd = s; dd < 3; dd++) acc[dd] += B[dd];
             }
-        }
+    if (!many)
+        for (int dd = s; dd < 3; dd++) oct[tensor_idx(s, dd) * noct + I] = acc[dd];
+    if (many) near[atomicAdd(nnear, 1u)] = (unsigned)g;
+}
+
+// Block per list entry, all its images in order.  The cells next to the
+// source take up to 10^6 points (24 x 24 x 12 x 12 x 6 for a 4 x 4 x 2 nm
+// cell), whose square roots and divisions in one lane set the time of the
+// whole plan (159 ms of 174 ms at 256x256x8).  Seven waves evaluate the
+// points of one chunk while three lanes of the first wave, one per field
+// component, add up the chunk before it in the order of the loops, so the
+// sums round as in one lane; what is left is the chain of additions (2.8 ms).
+constexpr int kNearThreads = 512, kNearChunk = kNearThreads - 64;
+__global__ void __launch_bounds__(kNearThreads) k_kernel_arne_near(double* __restrict__ oct, ArneP p,
+                                                                   const unsigned* __restrict__ near,
+                                                                   const unsigned* __restrict__ nnear) {
+#pragma clang fp contract(off)
+    __shared__ double val[2][3][kNearChunk];
+    const int h0 = p.s0 / 2 + 1, h1 = p.s1 / 2 + 1, h2 = p.s2 / 2 + 1;
+    const long noct = (long)h0 * h1 * h2;
+    const double cs[3] = {p.c0, p.c1, p.c2};
+    const unsigned cnt = *nnear;
+    const int tid = threadIdx.x;
+    for (unsigned k = blockIdx.x; k < cnt; k += gridDim.x) {
+        const long g = near[k];
+        const int s = (int)(g / noct);
+        const long I = g % noct;
+        const int zw = (int)(I % h2);
+        const int yw = (int)((I / h2) % h1);
+        const int xw = (int)(I / ((long)h1 * h2));
+        const int u = s, v = (s + 1) % 3, w = (s + 2) % 3;
+        double acc = 0;  // lane dd < 3: component dd
+        for (int z = first_image(zw, p.s2, p.r12); z <= p.r22; z += p.s2)
+            for (int y = first_image(yw, p.s1, p.r11); y <= p.r21; y += p.s1)
+                for (int x = first_image(xw, p.s0, p.r10); x <= p.r20; x += p.s0) {
+                    const ArnePts n = arne_points(cs, v, w, x, y, z, p.accuracy);
+                    const long cn = n.count();
+                    const double R[3] = {(double)x * p.c0, (double)y * p.c1, (double)z * p.c2};
+                    const double charge = cs[v] * cs[w] * (1 / (double)cn);
+                    double B = 0;
+                    // chunk c is evaluated in turn c and added in turn c + 1
+                    const long nch = (cn + kNearChunk - 1) / kNearChunk;
+                    for (long c = 0; c <= nch; c++) {
+                        if (tid >= 64) {
+                            const long t = c * kNearChunk + tid - 64;
+                            if (c < nch && t < cn) {
+                                long q = t;
+                                const int gg = (int)(q % n.nz);
+                                q /= n.nz;
+                                const int bb = (int)(q % n.ny);
+                                q /= n.ny;
+                                const int aa = (int)(q % n.nx);
+                                q /= n.nx;
+                                double o[3];
+                                arne_point(cs, u, v, w, R, n, charge, (int)(q / n.nw), (int)(q % n.nw), aa, bb, gg,
+                                           o);
+                                for (int dd = 0; dd < 3; dd++) val[c & 1][dd][tid - 64] = o[dd];
+                            }
+                        } else if (tid < 3 && c > 0) {
+                            const double* o = val[(c - 1) & 1][tid];
+                            const int m = (int)(cn - (c - 1) * kNearChunk < kNearChunk ? cn - (c - 1) * kNearChunk
+                                                                                       : kNearChunk);
+                            int q = 0;
+                            for (; q + 16 <= m; q += 16) {  // sixteen reads in flight, then the chain
+                                double r[16];
+#pragma unroll
+                                for (int e = 0; e < 16; e++) r[e] = o[q + e];
+#pragma unroll
+                                for (int e = 0; e < 16; e++) B += r[e];
+                            }
+                            for (; q < m; q++) B += o[q];
+                        }
+                        __syncthreads();
+                    }
+                    acc += B;
+                }
+        if (tid < 3 && tid >= s) oct[tensor_idx(s, tid) * noct + I] = acc;
     }
-    (void)any;
-    // FullTensorIdx (common/index.go:44-47): XX=0 YY=1 ZZ=2 YZ=3 XZ=4 XY=5
-    const int idx[3][3] = {{0, 5, 4}, {5, 1, 3}, {4, 3, 2}};
-    for (int dd = s; dd < 3; dd++) oct[idx[s][dd] * noct + I] = acc[dd];
-    (void)size;
 }
 
 // Newell demag tensor (A. J. Newell, W. Williams, D. J. Dunlop, J. Geophys.
@@ -905,9 +1008,13 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
         hipLaunchKernelGGL(k_kernel_newell, dim3(hs::div_up(noct, 64)), dim3(64), 0, st, oct, P0, P1, P2, cell[0],
                            cell[1], cell[2], r1[0], r1[1], r1[2], r2[0], r2[1], r2[2], rfar);
     } else {
-        hipLaunchKernelGGL(k_kernel_arne, dim3(hs::div_up(3 * noct, 64)), dim3(64), 0, st, oct, P0, P1, P2, cell[0],
-                           cell[1], cell[2], r1[0], r1[1], r1[2], r2[0], r2[1], r2[2],
-                           (double)(accuracy > 0 ? accuracy : 6));
+        const ArneP ap{P0,    P1,    P2,      r1[0],   r1[1],   r1[2], r2[0],
+                       r2[1], r2[2], cell[0], cell[1], cell[2], (double)(accuracy > 0 ? accuracy : 6)};
+        // the list of near cells (at most 3 noct entries) in the memory of `full`, which is filled after it is read
+        unsigned* near = reinterpret_cast<unsigned*>(full) + 2;
+        hipMemsetAsync(full, 0, sizeof(double), st);
+        hipLaunchKernelGGL(k_kernel_arne, dim3(hs::div_up(3 * noct, 64)), dim3(64), 0, st, oct, ap, near, near - 2);
+        hipLaunchKernelGGL(k_kernel_arne_near, dim3(1024), dim3(kNearThreads), 0, st, oct, ap, near, near - 2);
     }
     hipLaunchKernelGGL(k_kernel_fill, dim3(hs::grid1d(P), 6), dim3(hs::kBlock), 0, st, full, oct, P0, P1, P2);
     // IsZero (maxwell_convolution.go:227-232): components below 1e-12 of the
