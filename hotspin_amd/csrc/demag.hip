@@ -36,12 +36,30 @@
 
 #include "demag_kernels.hpp"
 #include "demag_tune.hpp"
+#include "demag_fused.hpp"
 #include "fft_any.hpp"
 
 hsdm::Variants& hsdm::variants(int L) {
     static std::map<int, hsdm::Variants> reg;
     return reg[L];
 }
+
+namespace fused {
+template <typename T>
+Rows<T>& rows_of(int M) {
+    static std::map<int, Rows<T>> reg;
+    return reg[M];
+}
+template <typename T>
+Mids<T>& mids_of(int Q) {
+    static std::map<int, Mids<T>> reg;
+    return reg[Q];
+}
+template Rows<float>& rows_of<float>(int);
+template Rows<double>& rows_of<double>(int);
+template Mids<float>& mids_of<float>(int);
+template Mids<double>& mids_of<double>(int);
+}  // namespace fused
 
 // ------------------------------------------------------------------ Kernel_Arne (FP64)
 // The field of the charged faces of the source cell (direction s), averaged
@@ -417,6 +435,26 @@ __global__ void __launch_bounds__(256) k_kernel_extract(const cpx<double>* __res
     }
 }
 
+// The fused kernel's table K~(d; j', k) from the tensor transformed along axes
+// 2 and 1 (X: [component][P0][P1][H2p]): the real parts of XX, YY, ZZ, YZ and
+// the imaginary parts of XZ, XY, planes d < N0, times norm = 1/(P1 P2).
+// kt[((k N0 + d) KR + k1 B + k2) 6 + component], j' = k1 + A k2.
+template <typename T>
+__global__ void __launch_bounds__(256) k_kernel_table(const cpx<double>* __restrict__ X, T* __restrict__ kt, int P0,
+                                                      int P1, int H2, int H2p, int N0, int A, int B, int KR,
+                                                      double norm, unsigned zero) {
+    const long n = (long)H2 * N0 * KR;
+    const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int c = blockIdx.y;
+    if (g >= n) return;
+    const int k = (int)(g % H2);  // consecutive lanes read consecutive k
+    const int d = (int)((g / H2) % N0), pos = (int)(g / ((long)H2 * N0));
+    const int j = pos / B + A * (pos % B);
+    const cpx<double> v = X[(((long)c * P0 + d) * P1 + j) * H2p + k];
+    const double r = (c < 4 ? v.x : v.y) * norm;
+    kt[(((long)k * N0 + d) * KR + pos) * 6 + c] = (zero >> c & 1) ? T(0) : T(r);
+}
+
 // ------------------------------------------------------------------ dispatch tables
 template <typename T>
 using r2c_fn = void (*)(const void*, const void*, long, cpx<T>*, long, int, int, const cpx<T>*, const cpx<T>*,
@@ -549,6 +587,10 @@ struct hs_demag {
     // columns (P1), axis 0 (P0); FP32 and FP64 decided separately
     bool genR = false, gen1 = false, gen0 = false, genRd = false, gen1d = false, gen0d = false;
     GenFFT gR{}, g1{}, g0{};
+    // three-kernel convolution (demag_fused.hpp), FP32 and FP64 decided separately
+    bool fz32 = false, fz64 = false;
+    float* kt32 = nullptr;
+    double* kt64 = nullptr;
     cpx<float>* Xzf = nullptr;   // (cap, 3, P0, P1, H2p): the axis-0 spectrum of a run-time-length F3K
     cpx<double>* Xzd = nullptr;  // the same for the FP64 field
 };
@@ -581,6 +623,47 @@ bool sizes_ok(hs_demag* d) {
     const int lim = gen_max_len<double>();
     return d->gR.L <= lim && P1 <= lim && P0 <= lim;
 }
+// Whether the fused kernels take the mesh: open axes 0 and 1 (or one plane),
+// an even padded x length, registered lengths, and a column that fits a block.
+template <typename T>
+bool fused_ok(const hs_demag* d) {
+    const int P1 = d->P[1];
+    if (d->P[2] % 2 || P1 != 2 * d->N[1] || !(d->N[0] == 1 || d->P[0] == 2 * d->N[0])) return false;
+    const auto& m = fused::mids_of<T>(P1);
+    return fused::rows_of<T>(d->M).fwd && m.A && m.pick(d->N[0]) && fused::mid_fits(d->N[0], P1, m.A, m.B, sizeof(cpx<T>));
+}
+
+// rows of the fused kernel's table per column and plane distance
+int fused_table(const hs_demag* d) {
+    const auto& m = fused::mids_of<float>(d->P[1]);
+    return (m.A / 2 + 1) * m.B;
+}
+
+// The fused convolution of nsolve solves (X: nsolve x 3 N0 N1 H2 values).
+template <typename T>
+int run_fused(hs_demag* d, const T* m, const T* msk, double srcMul, T* B, hipStream_t st, cpx<T>* X, const T* kt,
+              const cpx<T>* twM, const cpx<T>* twP2, const cpx<T>* tw1, int nsolve, const int* live) {
+    const int N0 = d->N[0], N1 = d->N[1], N2 = d->N[2], Q = d->P[1], H2 = d->H2;
+    const int rows = 3 * N0 * N1;
+    const long nrows = (long)rows * nsolve;
+    const auto& fr = fused::rows_of<T>(d->M);
+    const auto& fm = fused::mids_of<T>(Q);
+    const Live lrows{live, rows};
+    hs::prof_begin(HS_PROF_F1, st);
+    fr.fwd(m, msk, (long)N0 * N1, X, nrows, rows, N2, T(0.5 * srcMul), twM, twP2, st, lrows);
+    hs::prof_end(HS_PROF_F1, st);
+    hs::prof_begin(HS_PROF_F3K, st);
+    const fused::Mid<T> a{X,      kt, N0, H2, fused::mid_cb(N0, Q, fm.A, fm.B, H2, nsolve, sizeof(cpx<T>)),
+                          nsolve, tw1, live};
+    fm.pick(N0)(a, st);
+    hs::prof_end(HS_PROF_F3K, st);
+    hs::prof_begin(HS_PROF_I1, st);
+    fr.inv(X, B, nrows, rows, N2, twM, twP2, st, lrows);
+    hs::prof_end(HS_PROF_I1, st);
+    HS_LAUNCH_CHECK("hs_demag_field");
+    return hs_last_error();
+}
+
 // FFT table of the row transform: P2/2 points (even P2) or P2 (odd)
 template <typename T>
 const cpx<T>* row_table(const hs_demag* d, const cpx<T>* twM, const cpx<T>* twP2) {
@@ -598,6 +681,8 @@ int run_field32(hs_demag* d, const float* m, const float* msk, double srcMul, fl
         hs::set_error(HS_EINVAL, "hs_demag_field: batch larger than reserved");
         return HS_EINVAL;
     }
+    if (d->fz32)
+        return run_fused<float>(d, m, msk, srcMul, B, st, X1, d->kt32, d->twMf, d->twP2f, d->tw1f, nsolve, live);
     const long nrows = 3L * N0 * N1 * nsolve;
     Geo g1 = {(long)N1 * H2p, 0, H2p, 1};
     Geo g2 = {(long)P1 * H2p, 0, H2p, 1};
@@ -716,6 +801,7 @@ void tune32(hs_demag* d, hipStream_t st) {
     d->row32 = d->rowi32 = (d->genR || vr.rows.empty()) ? hsdm::RowV{} : vr.rows[0];
     d->col32 = (d->gen1 || vc.cols.empty()) ? hsdm::ColV{} : vc.cols[0];
     d->z32 = (d->gen0 || vz.z.empty()) ? hsdm::ZV{} : vz.z[0];
+    if (d->fz32) return;  // none of these passes runs
     // a plan with a run-time-length pass keeps the first variant of its
     // compiled passes (no timing)
     if (!d->row32.r2c || !d->col32.fwd || !d->z32.fn) return;
@@ -867,6 +953,8 @@ int run_field(hs_demag* d, const T* m, const T* msk, double srcMul, T* B, hipStr
               const cpx<T>* tw0) {
     const int N0 = d->N[0], N1 = d->N[1], N2 = d->N[2], P1 = d->P[1], P0 = d->P[0], P2 = d->P[2];
     const int H2 = d->H2, H2p = d->H2p, M = d->M;
+    if constexpr (sizeof(T) == 8)
+        if (d->fz64) return run_fused<T>(d, m, msk, srcMul, B, st, X1, d->kt64, twM, twP2, tw1, 1, nullptr);
     auto r2c = d->genRd ? nullptr : pick_r2c<T, T>(M);
     auto c2r = d->genRd ? nullptr : pick_c2r<T, T>(M);
     auto f1 = d->gen1d ? nullptr : pick_cols<T, -1>(P1);
@@ -966,8 +1054,14 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     hipMalloc(&d->kern32, sizeof(float) * 6 * nk32);
     if (d->kern32) hipMemsetAsync(d->kern32, 0, sizeof(float) * 6 * nk32, st);
     hipMalloc(&d->X1f, sizeof(cpx<float>) * 3L * N[0] * N[1] * H2p);
-    hipMalloc(&d->X2f, sizeof(cpx<float>) * 3L * N[0] * P1 * H2p);
-    if (d->gen0) hipMalloc(&d->Xzf, sizeof(cpx<float>) * 3L * P0 * P1 * H2p);
+    // HS_DEMAG_FORCE asks for particular five-pass variants
+    d->fz32 = !getenv("HS_DEMAG_FORCE") && fused_ok<float>(d);
+    d->fz64 = fused_ok<double>(d);
+    if (!d->fz32) hipMalloc(&d->X2f, sizeof(cpx<float>) * 3L * N[0] * P1 * H2p);
+    if (!d->fz32 && d->gen0) hipMalloc(&d->Xzf, sizeof(cpx<float>) * 3L * P0 * P1 * H2p);
+    const long nt = (d->fz32 || d->fz64) ? 6L * N[0] * fused_table(d) * H2 : 0;
+    if (d->fz32) hipMalloc(&d->kt32, sizeof(float) * nt);
+    if (d->fz64) hipMalloc(&d->kt64, sizeof(double) * nt);
     // ---- Kernel_Arne on the device (FP64)
     int r1[3], r2[3];
     for (int c = 0; c < 3; c++) {
@@ -990,7 +1084,8 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     hipMalloc(&full, sizeof(double) * 6 * P);
     hipMalloc(&X, sizeof(cpx<double>) * 6L * P0 * P1 * H2p);
     hipMalloc(&maxbits, 2 * kExtractLanes * sizeof(unsigned long long));
-    if (!oct || !full || !X || !maxbits || !d->kern64 || !d->kern32 || !d->X1f || !d->X2f || (d->gen0 && !d->Xzf)) {
+    if (!oct || !full || !X || !maxbits || !d->kern64 || !d->kern32 || !d->X1f ||
+        (!d->fz32 && (!d->X2f || (d->gen0 && !d->Xzf))) || (d->fz32 && !d->kt32) || (d->fz64 && !d->kt64)) {
         hs::set_error(HS_ENOMEM, "hs_demag_create: out of device memory");
         hipFree(oct); hipFree(full); hipFree(X); hipFree(maxbits);
         hs_demag_destroy(d);
@@ -1039,6 +1134,21 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
         gen::cols<double, -1>(X, X, ga1, ga1, 6 * P0, P1, P1, H2, d->g1, d->tw1d, st, all);
     else
         pick_cols<double, -1>(P1)(X, X, ga1, ga1, 6 * P0, P1, P1, H2, d->tw1d, st);
+    if (d->fz32 || d->fz64) {
+        const auto& fm = fused::mids_of<float>(P1);
+        const int KR = fused_table(d);
+        const dim3 g(hs::grid1d((long)H2 * N[0] * KR), 6);
+        unsigned zero = 0;
+        for (int c = 0; c < 6; c++)
+            if (gmax > 0 && cmax[c] / gmax < 1e-12) zero |= 1u << c;
+        const double norm = 1.0 / ((double)P1 * P2);
+        if (d->fz32)
+            hipLaunchKernelGGL(k_kernel_table<float>, g, dim3(hs::kBlock), 0, st, X, d->kt32, P0, P1, H2, H2p, N[0],
+                               fm.A, fm.B, KR, norm, zero);
+        if (d->fz64)
+            hipLaunchKernelGGL(k_kernel_table<double>, g, dim3(hs::kBlock), 0, st, X, d->kt64, P0, P1, H2, H2p, N[0],
+                               fm.A, fm.B, KR, norm, zero);
+    }
     Geo ga0 = {(long)P0 * P1 * H2p, (long)H2p, (long)P1 * H2p, P1};
     if (auto f0 = pick_cols<double, -1>(P0))
         f0(X, X, ga0, ga0, 6 * P1, P0, P0, H2, d->tw0d, st);
@@ -1088,7 +1198,7 @@ extern "C" hs_demag* hs_demag_create_newell(const int N[3], const double cell[3]
 
 extern "C" void hs_demag_destroy(hs_demag* d) {
     if (!d) return;
-    void* ps[] = {d->kern64, d->kern32, d->X1f, d->X2f, d->X1d, d->X2d, d->twMf, d->twP2f,
+    void* ps[] = {d->kt32,   d->kt64,   d->kern64, d->kern32, d->X1f, d->X2f, d->X1d, d->X2d, d->twMf, d->twP2f,
                   d->tw1f,   d->tw0f,   d->twMd, d->twP2d, d->tw1d, d->tw0d, d->Xzf, d->Xzd};
     for (void* p : ps)
         if (p) hipFree(p);
@@ -1149,9 +1259,9 @@ extern "C" int hs_demag_field_f64(hs_demag* d, const double* m, const double* ms
     }
     if (!d->X1d) {
         hipMalloc(&d->X1d, sizeof(cpx<double>) * 3L * d->N[0] * d->N[1] * d->H2p);
-        hipMalloc(&d->X2d, sizeof(cpx<double>) * 3L * d->N[0] * d->P[1] * d->H2p);
-        if (d->gen0d) hipMalloc(&d->Xzd, sizeof(cpx<double>) * 3L * d->P[0] * d->P[1] * d->H2p);
-        if (!d->X1d || !d->X2d || (d->gen0d && !d->Xzd)) {
+        if (!d->fz64) hipMalloc(&d->X2d, sizeof(cpx<double>) * 3L * d->N[0] * d->P[1] * d->H2p);
+        if (!d->fz64 && d->gen0d) hipMalloc(&d->Xzd, sizeof(cpx<double>) * 3L * d->P[0] * d->P[1] * d->H2p);
+        if (!d->X1d || (!d->fz64 && (!d->X2d || (d->gen0d && !d->Xzd)))) {
             hs::set_error(HS_ENOMEM, "hs_demag_field_f64: out of device memory");
             return HS_ENOMEM;
         }
@@ -1239,9 +1349,9 @@ extern "C" int hs_demag_reserve(hs_demag* d, int nsolve) {
     if (nsolve <= d->cap) return 0;
     cpx<float>*X1 = nullptr, *X2 = nullptr, *Xz = nullptr;
     hipMalloc(&X1, sizeof(cpx<float>) * 3L * d->N[0] * d->N[1] * d->H2p * nsolve);
-    hipMalloc(&X2, sizeof(cpx<float>) * 3L * d->N[0] * d->P[1] * d->H2p * nsolve);
-    if (d->gen0) hipMalloc(&Xz, sizeof(cpx<float>) * 3L * d->P[0] * d->P[1] * d->H2p * nsolve);
-    if (!X1 || !X2 || (d->gen0 && !Xz)) {
+    if (!d->fz32) hipMalloc(&X2, sizeof(cpx<float>) * 3L * d->N[0] * d->P[1] * d->H2p * nsolve);
+    if (!d->fz32 && d->gen0) hipMalloc(&Xz, sizeof(cpx<float>) * 3L * d->P[0] * d->P[1] * d->H2p * nsolve);
+    if (!X1 || (!d->fz32 && (!X2 || (d->gen0 && !Xz)))) {
         hipFree(X1);
         hipFree(X2);
         hipFree(Xz);
@@ -1263,9 +1373,11 @@ long hs_demag_ncell(const hs_demag* d) { return d->ncell; }
 long hs_demag_footprint(const hs_demag* d) {
     const long nk = (long)d->K[0] * d->K[1] * d->K[2];
     long b = 6 * nk * (sizeof(double) + sizeof(float));
-    b += (long)sizeof(cpx<float>) * 3L * d->N[0] * (d->N[1] + d->P[1]) * d->H2p * d->cap;
+    b += (long)sizeof(cpx<float>) * 3L * d->N[0] * (d->N[1] + (d->fz32 ? 0 : d->P[1])) * d->H2p * d->cap;
+    if (d->kt32) b += 6L * d->N[0] * fused_table(d) * d->H2 * (long)sizeof(float);
+    if (d->kt64) b += 6L * d->N[0] * fused_table(d) * d->H2 * (long)sizeof(double);
     b += 6L * d->K[0] * d->K[1] * (d->KP - d->H2) * (long)sizeof(float);
-    if (d->X1d) b += (long)sizeof(cpx<double>) * 3L * d->N[0] * (d->N[1] + d->P[1]) * d->H2p;
+    if (d->X1d) b += (long)sizeof(cpx<double>) * 3L * d->N[0] * (d->N[1] + (d->fz64 ? 0 : d->P[1])) * d->H2p;
     if (d->Xzf) b += (long)sizeof(cpx<float>) * 3L * d->P[0] * d->P[1] * d->H2p * d->cap;
     if (d->Xzd) b += (long)sizeof(cpx<double>) * 3L * d->P[0] * d->P[1] * d->H2p;
     b += (long)(sizeof(cpx<float>) + sizeof(cpx<double>)) * (d->M + d->P[2] + d->P[1] + d->P[0]);

@@ -1,0 +1,71 @@
+"""The three-kernel demag convolution (column tiles in LDS, axis 0 convolved
+directly) against the FP64 oracle, at the sizes where its tiling can go wrong:
+plane counts below, at and beyond one axis-0 item (1..8 planes, then blocks of
+6 and 8 with a remainder), column counts that leave a partial tile, row counts
+that leave a partial row block, each length family, masks and batches.
+
+Bars: FP64 1e-12 of max|B| (as the five-pass convolution); FP32 2e-6, the
+round-off of FP32 transforms of up to 2048 points and sums of up to 3 N0
+products (eps (log2 P1 P2 + N0) ~ 6e-8 (20 + 33) = 3e-6 at worst, rms 1/10)."""
+import numpy as np
+import pytest
+
+from hotspin_amd.api import Demag
+from hotspin_amd._lib import check
+from oracle import pyoracle as po
+from tests.gpu_util import P, dev, empty, host, relerr, require_gpu, torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _gpu():
+    require_gpu()
+    yield
+    check("demag fused")
+
+
+SHAPES = ([(n0, 8, 16) for n0 in range(1, 10)] +           # planes per item, first of the blocked form
+          [(10, 8, 16), (12, 4, 8), (13, 8, 8), (16, 16, 8), (17, 4, 16), (33, 8, 8)] +
+          [(2, 5, 10), (3, 6, 12), (2, 10, 20), (1, 12, 24), (3, 24, 48), (2, 20, 40), (4, 80, 10)] +
+          [(1, 32, 128), (8, 256, 8), (2, 512, 8), (1, 384, 16), (5, 64, 512)])
+
+
+@pytest.mark.parametrize("N", SHAPES)
+def test_fields_match_oracle(N):
+    cell = (2e-9, 3e-9, 2.5e-9)
+    rng = np.random.default_rng(sum(N))
+    n = N[0] * N[1] * N[2]
+    m = rng.standard_normal((3, n))
+    msk = rng.random(n)
+    d, o = Demag(N, cell), po.Demag(N, cell)
+    for w in (None, msk):
+        want = o.B(m, w, 8e5).reshape(3, n)
+        dm, dw = dev(m), None if w is None else dev(w)
+        B = empty((3, n))
+        d.field_f64(P(dm), P(dw), 8e5, P(B))
+        assert relerr(host(B), want) <= 1e-12
+        dm, dw = dev(m, np.float32), None if w is None else dev(w, np.float32)
+        B = empty((3, n), torch.float32)
+        d.field_f32(P(dm), P(dw), 8e5, P(B))
+        assert relerr(host(B), want) <= 2e-6
+    d.close()
+
+
+@pytest.mark.parametrize("N", [(2, 8, 16), (9, 6, 24)])
+def test_periodic_x_and_the_other_axes(N):
+    """A periodic x axis keeps the three kernels (rows without padding); a
+    periodic axis 0 or 1 takes the five passes.  Both match the oracle."""
+    cell = (2e-9, 3e-9, 2.5e-9)
+    n = N[0] * N[1] * N[2]
+    m = np.random.default_rng(3).standard_normal((3, n))
+    for pbc in ((0, 0, 1), (0, 1, 0), (1, 0, 0), (1, 1, 1)):
+        d = Demag(N, cell, pbc)
+        want = po.Demag(N, cell, pbc).B(m, None, 8e5).reshape(3, n)
+        dm, B = dev(m), empty((3, n))
+        d.field_f64(P(dm), None, 8e5, P(B))
+        assert relerr(host(B), want) <= 1e-12
+        dm, B = dev(m, np.float32), empty((3, n), torch.float32)
+        d.field_f32(P(dm), None, 8e5, P(B))
+        assert relerr(host(B), want) <= 2e-6
+        d.close()
