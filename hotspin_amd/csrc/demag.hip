@@ -435,24 +435,44 @@ __global__ void __launch_bounds__(256) k_kernel_extract(const cpx<double>* __res
     }
 }
 
-// The fused kernel's table K~(d; j', k) from the tensor transformed along axes
-// 2 and 1 (X: [component][P0][P1][H2p]): the real parts of XX, YY, ZZ, YZ and
-// the imaginary parts of XZ, XY, planes d < N0, times norm = 1/(P1 P2).
-// kt[((k N0 + d) KR + k1 B + k2) 6 + component], j' = k1 + A k2.
+// The fused kernel's table K~(d; j', k), planes d < N0, from the octant of the
+// transformed tensor: the inverse transform along axis 0, real and even in d
+// for XX, YY, ZZ, YZ, i kappa and odd for XZ, XY (tw0: w_P0^t); XX is kept
+// negated, as the fused kernel uses it.
+// kt[((tc N0 + d) KR + pos) 6 + component]: without folding tc = k and
+// pos = k1 B + k2 holds row j' = k1 + A k2; folded by R, tc = k (R/2 + 1) + s
+// and pos the row j' = R (k1 + A k2) + s.
+constexpr int kTabD = 8;  // planes a thread forms at a time
 template <typename T>
-__global__ void __launch_bounds__(256) k_kernel_table(const cpx<double>* __restrict__ X, T* __restrict__ kt, int P0,
-                                                      int P1, int H2, int H2p, int N0, int A, int B, int KR,
-                                                      double norm, unsigned zero) {
-    const long n = (long)H2 * N0 * KR;
+__global__ void __launch_bounds__(256) k_kernel_table(const double* __restrict__ kern, T* __restrict__ kt, int N0,
+                                                      int P0, int P1, int H2, int K0, int K1, int R, int A, int B,
+                                                      int KR, const cpx<double>* __restrict__ tw0) {
+    const int TC = fused::table_cols(R);
+    const long n = (long)H2 * TC * KR;
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const int c = blockIdx.y;
     if (g >= n) return;
     const int k = (int)(g % H2);  // consecutive lanes read consecutive k
-    const int d = (int)((g / H2) % N0), pos = (int)(g / ((long)H2 * N0));
-    const int j = pos / B + A * (pos % B);
-    const cpx<double> v = X[(((long)c * P0 + d) * P1 + j) * H2p + k];
-    const double r = (c < 4 ? v.x : v.y) * norm;
-    kt[(((long)k * N0 + d) * KR + pos) * 6 + c] = (zero >> c & 1) ? T(0) : T(r);
+    const int s = (int)((g / H2) % TC), pos = (int)(g / ((long)H2 * TC));
+    const int j = R * (pos / B + A * (pos % B)) + s;
+    const bool mir = 2 * j > P1;
+    const double sg = mir && (c == 3 || c == 5) ? -1.0 : 1.0;  // YZ and XY are odd along axis 1
+    const double* q = kern + ((long)c * K0 * K1 + (mir ? P1 - j : j)) * H2 + k;
+    T* o = kt + (((long)k * TC + s) * N0 * KR + pos) * 6 + c;
+    for (int d0 = 0; d0 < N0; d0 += kTabD) {
+        double acc[kTabD];
+        for (int u = 0; u < kTabD; u++) acc[u] = 0.0;
+        for (int i = 0; i < K0; i++) {
+            const double v = sg * q[(long)i * K1 * H2] * ((i == 0 || 2 * i == P0) ? 1.0 : 2.0);
+#pragma unroll
+            for (int u = 0; u < kTabD; u++) {
+                const cpx<double> w = tw0[(int)((long)i * (d0 + u) % P0)];
+                acc[u] += v * (c < 4 ? w.x : -w.y);
+            }
+        }
+        for (int u = 0; u < kTabD; u++)
+            if (d0 + u < N0) o[(long)(d0 + u) * KR * 6] = T(c == 0 ? -acc[u] : acc[u]);
+    }
 }
 
 // ------------------------------------------------------------------ dispatch tables
@@ -587,8 +607,9 @@ struct hs_demag {
     // columns (P1), axis 0 (P0); FP32 and FP64 decided separately
     bool genR = false, gen1 = false, gen0 = false, genRd = false, gen1d = false, gen0d = false;
     GenFFT gR{}, g1{}, g0{};
-    // three-kernel convolution (demag_fused.hpp), FP32 and FP64 decided separately
-    bool fz32 = false, fz64 = false;
+    // three-kernel convolution (demag_fused.hpp): the fold of axis 1, 0 = not
+    // taken, FP32 and FP64 decided separately; kt64 may be filled on first use
+    int fold32 = 0, fold64 = 0;
     float* kt32 = nullptr;
     double* kt64 = nullptr;
     cpx<float>* Xzf = nullptr;   // (cap, 3, P0, P1, H2p): the axis-0 spectrum of a run-time-length F3K
@@ -623,42 +644,55 @@ bool sizes_ok(hs_demag* d) {
     const int lim = gen_max_len<double>();
     return d->gR.L <= lim && P1 <= lim && P0 <= lim;
 }
-// Whether the fused kernels take the mesh: open axes 0 and 1 (or one plane),
-// an even padded x length, registered lengths, and a column that fits a block.
+// Fold R of axis 1 with which the fused kernels take the mesh (mid_fold), 0 if
+// they do not: open axes 0 and 1 (or one plane), an even padded x length,
+// registered lengths.
 template <typename T>
-bool fused_ok(const hs_demag* d) {
-    const int P1 = d->P[1];
-    if (d->P[2] % 2 || P1 != 2 * d->N[1] || !(d->N[0] == 1 || d->P[0] == 2 * d->N[0])) return false;
-    const auto& m = fused::mids_of<T>(P1);
-    return fused::rows_of<T>(d->M).fwd && m.A && m.pick(d->N[0]) && fused::mid_fits(d->N[0], P1, m.A, m.B, sizeof(cpx<T>));
+int fused_fold(const hs_demag* d) {
+    const int P1 = d->P[1], N0 = d->N[0];
+    if (d->P[2] % 2 || P1 != 2 * d->N[1] || !(N0 == 1 || d->P[0] == 2 * N0)) return 0;
+    return fused::mid_fold(N0, P1, sizeof(cpx<T>), [&](int R) {
+        const auto& m = fused::mids_of<T>(P1 / R);
+        return fused::rows_of<T>(d->M).fwd[fused::fold_index(R)] && m.A && m.pick(N0, R > 1) &&
+               fused::mid_fits(N0, P1 / R, m.A, m.B, sizeof(cpx<T>));
+    });
+}
+// values of the fused spectrum (per solve) and of its kernel table
+long fused_spectrum(const hs_demag* d, int R) { return 3L * d->N[0] * (R > 1 ? d->P[1] : d->N[1]) * d->H2p; }
+int fused_rows(const hs_demag* d, int R) { return fused::table_rows_of(d->P[1] / R, R > 1); }
+long fused_table(const hs_demag* d, int R) {
+    return 6L * d->N[0] * fused_rows(d, R) * fused::table_cols(R) * d->H2;
+}
+// Fills the table of fold R from the FP64 octant.
+template <typename T>
+void fill_table(const hs_demag* d, T* kt, int R, hipStream_t st) {
+    const auto& m = fused::mids_of<T>(d->P[1] / R);
+    const int KR = fused_rows(d, R);
+    hipLaunchKernelGGL(k_kernel_table<T>, dim3(hs::grid1d((long)d->H2 * fused::table_cols(R) * KR), 6),
+                       dim3(hs::kBlock), 0, st, d->kern64, kt, d->N[0], d->P[0], d->P[1], d->H2, d->K[0], d->K[1], R,
+                       m.A, m.B, KR, d->tw0d);
 }
 
-// rows of the fused kernel's table per column and plane distance
-int fused_table(const hs_demag* d) {
-    const auto& m = fused::mids_of<float>(d->P[1]);
-    return (m.A / 2 + 1) * m.B;
-}
-
-// The fused convolution of nsolve solves (X: nsolve x 3 N0 N1 H2 values).
+// The fused convolution of nsolve solves (X: nsolve x fused_spectrum values).
 template <typename T>
 int run_fused(hs_demag* d, const T* m, const T* msk, double srcMul, T* B, hipStream_t st, cpx<T>* X, const T* kt,
-              const cpx<T>* twM, const cpx<T>* twP2, const cpx<T>* tw1, int nsolve, const int* live) {
-    const int N0 = d->N[0], N1 = d->N[1], N2 = d->N[2], Q = d->P[1], H2 = d->H2;
-    const int rows = 3 * N0 * N1;
-    const long nrows = (long)rows * nsolve;
+              int R, const cpx<T>* twM, const cpx<T>* twP2, const cpx<T>* tw1, int nsolve, const int* live) {
+    const int N0 = d->N[0], N1 = d->N[1], Q = d->P[1] / R, f = fused::fold_index(R);
     const auto& fr = fused::rows_of<T>(d->M);
     const auto& fm = fused::mids_of<T>(Q);
-    const Live lrows{live, rows};
+    const fused::RowP g{3 * N0 * N1, N1, Q, 3 * N0, nsolve, d->N[2], (long)N0 * N1};
+    const Live lrows{live, g.rows};
     hs::prof_begin(HS_PROF_F1, st);
-    fr.fwd(m, msk, (long)N0 * N1, X, nrows, rows, N2, T(0.5 * srcMul), twM, twP2, st, lrows);
+    fr.fwd[f](m, msk, X, g, T(0.5 * srcMul), twM, twP2, tw1, st, lrows);
     hs::prof_end(HS_PROF_F1, st);
     hs::prof_begin(HS_PROF_F3K, st);
-    const fused::Mid<T> a{X,      kt, N0, H2, fused::mid_cb(N0, Q, fm.A, fm.B, H2, nsolve, sizeof(cpx<T>)),
-                          nsolve, tw1, live};
-    fm.pick(N0)(a, st);
+    const int ncol = d->H2 * R;
+    const fused::Mid<T> a{X,    kt,     N0, ncol, fused::mid_cb(N0, Q, fm.A, fm.B, ncol, nsolve, sizeof(cpx<T>)),
+                          nsolve, R, tw1, live};
+    fm.pick(N0, R > 1)(a, st);
     hs::prof_end(HS_PROF_F3K, st);
     hs::prof_begin(HS_PROF_I1, st);
-    fr.inv(X, B, nrows, rows, N2, twM, twP2, st, lrows);
+    fr.inv[f](X, B, g, twM, twP2, tw1, st, lrows);
     hs::prof_end(HS_PROF_I1, st);
     HS_LAUNCH_CHECK("hs_demag_field");
     return hs_last_error();
@@ -681,8 +715,9 @@ int run_field32(hs_demag* d, const float* m, const float* msk, double srcMul, fl
         hs::set_error(HS_EINVAL, "hs_demag_field: batch larger than reserved");
         return HS_EINVAL;
     }
-    if (d->fz32)
-        return run_fused<float>(d, m, msk, srcMul, B, st, X1, d->kt32, d->twMf, d->twP2f, d->tw1f, nsolve, live);
+    if (d->fold32)
+        return run_fused<float>(d, m, msk, srcMul, B, st, X1, d->kt32, d->fold32, d->twMf, d->twP2f, d->tw1f, nsolve,
+                                live);
     const long nrows = 3L * N0 * N1 * nsolve;
     Geo g1 = {(long)N1 * H2p, 0, H2p, 1};
     Geo g2 = {(long)P1 * H2p, 0, H2p, 1};
@@ -801,7 +836,7 @@ void tune32(hs_demag* d, hipStream_t st) {
     d->row32 = d->rowi32 = (d->genR || vr.rows.empty()) ? hsdm::RowV{} : vr.rows[0];
     d->col32 = (d->gen1 || vc.cols.empty()) ? hsdm::ColV{} : vc.cols[0];
     d->z32 = (d->gen0 || vz.z.empty()) ? hsdm::ZV{} : vz.z[0];
-    if (d->fz32) return;  // none of these passes runs
+    if (d->fold32) return;  // none of these passes runs
     // a plan with a run-time-length pass keeps the first variant of its
     // compiled passes (no timing)
     if (!d->row32.r2c || !d->col32.fwd || !d->z32.fn) return;
@@ -954,7 +989,8 @@ int run_field(hs_demag* d, const T* m, const T* msk, double srcMul, T* B, hipStr
     const int N0 = d->N[0], N1 = d->N[1], N2 = d->N[2], P1 = d->P[1], P0 = d->P[0], P2 = d->P[2];
     const int H2 = d->H2, H2p = d->H2p, M = d->M;
     if constexpr (sizeof(T) == 8)
-        if (d->fz64) return run_fused<T>(d, m, msk, srcMul, B, st, X1, d->kt64, twM, twP2, tw1, 1, nullptr);
+        if (d->fold64)
+            return run_fused<T>(d, m, msk, srcMul, B, st, X1, d->kt64, d->fold64, twM, twP2, tw1, 1, nullptr);
     auto r2c = d->genRd ? nullptr : pick_r2c<T, T>(M);
     auto c2r = d->genRd ? nullptr : pick_c2r<T, T>(M);
     auto f1 = d->gen1d ? nullptr : pick_cols<T, -1>(P1);
@@ -1009,6 +1045,19 @@ int run_field(hs_demag* d, const T* m, const T* msk, double srcMul, T* B, hipStr
 }
 }  // namespace
 
+namespace {
+// static scratch of hs_demag_field_f64_noalloc (below)
+constexpr size_t kScratchBytes = size_t(64) << 20;
+// FP64 spectra of one solve of the plan's mesh: X1, then X2 and (run-time
+// axis-0 length only) Xz, each from a 256-byte boundary
+size_t x_bytes(const hs_demag* d, int rows) { return sizeof(cpx<double>) * 3ull * rows * d->P[1] * d->H2p; }
+size_t up256(size_t b) { return (b + 255) / 256 * 256; }
+size_t noalloc_bytes(const hs_demag* d) {
+    const size_t x1 = sizeof(cpx<double>) * 3ull * d->N[0] * d->N[1] * d->H2p;
+    return up256(x1) + up256(x_bytes(d, d->N[0])) + (d->gen0d ? x_bytes(d, d->P[0]) : 0);
+}
+}  // namespace
+
 // kernel: 0 = Kernel_Arne at `accuracy`, 1 = Newell
 static hs_demag* demag_create(const int N[3], const double cell[3], const int pbc[3], int accuracy, int kernel,
                               CUstream stream) {
@@ -1053,15 +1102,16 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     const long nk32 = (long)d->K[0] * d->K[1] * d->KP;
     hipMalloc(&d->kern32, sizeof(float) * 6 * nk32);
     if (d->kern32) hipMemsetAsync(d->kern32, 0, sizeof(float) * 6 * nk32, st);
-    hipMalloc(&d->X1f, sizeof(cpx<float>) * 3L * N[0] * N[1] * H2p);
     // HS_DEMAG_FORCE asks for particular five-pass variants
-    d->fz32 = !getenv("HS_DEMAG_FORCE") && fused_ok<float>(d);
-    d->fz64 = fused_ok<double>(d);
-    if (!d->fz32) hipMalloc(&d->X2f, sizeof(cpx<float>) * 3L * N[0] * P1 * H2p);
-    if (!d->fz32 && d->gen0) hipMalloc(&d->Xzf, sizeof(cpx<float>) * 3L * P0 * P1 * H2p);
-    const long nt = (d->fz32 || d->fz64) ? 6L * N[0] * fused_table(d) * H2 : 0;
-    if (d->fz32) hipMalloc(&d->kt32, sizeof(float) * nt);
-    if (d->fz64) hipMalloc(&d->kt64, sizeof(double) * nt);
+    d->fold32 = getenv("HS_DEMAG_FORCE") ? 0 : fused_fold<float>(d);
+    d->fold64 = fused_fold<double>(d);
+    hipMalloc(&d->X1f, sizeof(cpx<float>) * fused_spectrum(d, d->fold32));
+    if (!d->fold32) hipMalloc(&d->X2f, sizeof(cpx<float>) * 3L * N[0] * P1 * H2p);
+    if (!d->fold32 && d->gen0) hipMalloc(&d->Xzf, sizeof(cpx<float>) * 3L * P0 * P1 * H2p);
+    if (d->fold32) hipMalloc(&d->kt32, sizeof(float) * fused_table(d, d->fold32));
+    // the FP64 table now where hs_demag_field_f64_noalloc takes the mesh (it cannot allocate), else on first use
+    const bool tab64 = d->fold64 && noalloc_bytes(d) <= kScratchBytes;
+    if (tab64) hipMalloc(&d->kt64, sizeof(double) * fused_table(d, d->fold64));
     // ---- Kernel_Arne on the device (FP64)
     int r1[3], r2[3];
     for (int c = 0; c < 3; c++) {
@@ -1085,7 +1135,7 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     hipMalloc(&X, sizeof(cpx<double>) * 6L * P0 * P1 * H2p);
     hipMalloc(&maxbits, 2 * kExtractLanes * sizeof(unsigned long long));
     if (!oct || !full || !X || !maxbits || !d->kern64 || !d->kern32 || !d->X1f ||
-        (!d->fz32 && (!d->X2f || (d->gen0 && !d->Xzf))) || (d->fz32 && !d->kt32) || (d->fz64 && !d->kt64)) {
+        (!d->fold32 && (!d->X2f || (d->gen0 && !d->Xzf))) || (d->fold32 && !d->kt32) || (tab64 && !d->kt64)) {
         hs::set_error(HS_ENOMEM, "hs_demag_create: out of device memory");
         hipFree(oct); hipFree(full); hipFree(X); hipFree(maxbits);
         hs_demag_destroy(d);
@@ -1134,21 +1184,6 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
         gen::cols<double, -1>(X, X, ga1, ga1, 6 * P0, P1, P1, H2, d->g1, d->tw1d, st, all);
     else
         pick_cols<double, -1>(P1)(X, X, ga1, ga1, 6 * P0, P1, P1, H2, d->tw1d, st);
-    if (d->fz32 || d->fz64) {
-        const auto& fm = fused::mids_of<float>(P1);
-        const int KR = fused_table(d);
-        const dim3 g(hs::grid1d((long)H2 * N[0] * KR), 6);
-        unsigned zero = 0;
-        for (int c = 0; c < 6; c++)
-            if (gmax > 0 && cmax[c] / gmax < 1e-12) zero |= 1u << c;
-        const double norm = 1.0 / ((double)P1 * P2);
-        if (d->fz32)
-            hipLaunchKernelGGL(k_kernel_table<float>, g, dim3(hs::kBlock), 0, st, X, d->kt32, P0, P1, H2, H2p, N[0],
-                               fm.A, fm.B, KR, norm, zero);
-        if (d->fz64)
-            hipLaunchKernelGGL(k_kernel_table<double>, g, dim3(hs::kBlock), 0, st, X, d->kt64, P0, P1, H2, H2p, N[0],
-                               fm.A, fm.B, KR, norm, zero);
-    }
     Geo ga0 = {(long)P0 * P1 * H2p, (long)H2p, (long)P1 * H2p, P1};
     if (auto f0 = pick_cols<double, -1>(P0))
         f0(X, X, ga0, ga0, 6 * P1, P0, P0, H2, d->tw0d, st);
@@ -1162,6 +1197,8 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
             hipMemsetAsync(d->kern32 + c * nk32, 0, sizeof(float) * nk32, st);
         }
     }
+    if (d->fold32) fill_table<float>(d, d->kt32, d->fold32, st);
+    if (tab64) fill_table<double>(d, d->kt64, d->fold64, st);
     unsigned long long mb[2 * kExtractLanes];
     hipMemcpyAsync(mb, maxbits, sizeof(mb), hipMemcpyDeviceToHost, st);
     hipStreamSynchronize(st);
@@ -1258,12 +1295,26 @@ extern "C" int hs_demag_field_f64(hs_demag* d, const double* m, const double* ms
         return HS_EINVAL;
     }
     if (!d->X1d) {
-        hipMalloc(&d->X1d, sizeof(cpx<double>) * 3L * d->N[0] * d->N[1] * d->H2p);
-        if (!d->fz64) hipMalloc(&d->X2d, sizeof(cpx<double>) * 3L * d->N[0] * d->P[1] * d->H2p);
-        if (!d->fz64 && d->gen0d) hipMalloc(&d->Xzd, sizeof(cpx<double>) * 3L * d->P[0] * d->P[1] * d->H2p);
-        if (!d->X1d || (!d->fz64 && (!d->X2d || (d->gen0d && !d->Xzd)))) {
+        hipMalloc(&d->X1d, sizeof(cpx<double>) * fused_spectrum(d, d->fold64));
+        if (!d->fold64) hipMalloc(&d->X2d, sizeof(cpx<double>) * 3L * d->N[0] * d->P[1] * d->H2p);
+        if (!d->fold64 && d->gen0d) hipMalloc(&d->Xzd, sizeof(cpx<double>) * 3L * d->P[0] * d->P[1] * d->H2p);
+        const bool tab = d->fold64 && !d->kt64;
+        if (tab) hipMalloc(&d->kt64, sizeof(double) * fused_table(d, d->fold64));
+        if (!d->X1d || (!d->fold64 && (!d->X2d || (d->gen0d && !d->Xzd))) || (d->fold64 && !d->kt64)) {
+            void* ps[] = {d->X1d, d->X2d, d->Xzd};
+            for (void* p : ps)
+                if (p) hipFree(p);
+            d->X1d = d->X2d = d->Xzd = nullptr;
+            if (tab && d->kt64) {
+                hipFree(d->kt64);
+                d->kt64 = nullptr;
+            }
             hs::set_error(HS_ENOMEM, "hs_demag_field_f64: out of device memory");
             return HS_ENOMEM;
+        }
+        if (tab) {  // ready for calls on any stream
+            fill_table<double>(d, d->kt64, d->fold64, hs::S(stream));
+            hipStreamSynchronize(hs::S(stream));
         }
     }
     return run_field<double>(d, m, msk, HS_MU0 * msat0T0Mul, B, hs::S(stream), d->X1d, d->X2d, d->Xzd, d->kern64,
@@ -1277,7 +1328,6 @@ extern "C" int hs_demag_field_f64(hs_demag* d, const double* m, const double* ms
 // threads) race.  No pass reads a spectrum element that the same call has
 // not written first, so the contents left by an earlier call do not matter.
 namespace {
-constexpr size_t kScratchBytes = size_t(64) << 20;
 constexpr int kMaxDevices = 64;
 }  // namespace
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -1301,14 +1351,6 @@ void* scratch_address() {
     return g_scratch[dev];
 }
 
-// FP64 spectra of one solve of the plan's mesh: X1, then X2 and (run-time
-// axis-0 length only) Xz, each from a 256-byte boundary
-size_t x_bytes(const hs_demag* d, int rows) { return sizeof(cpx<double>) * 3ull * rows * d->P[1] * d->H2p; }
-size_t up256(size_t b) { return (b + 255) / 256 * 256; }
-size_t noalloc_bytes(const hs_demag* d) {
-    const size_t x1 = sizeof(cpx<double>) * 3ull * d->N[0] * d->N[1] * d->H2p;
-    return up256(x1) + up256(x_bytes(d, d->N[0])) + (d->gen0d ? x_bytes(d, d->P[0]) : 0);
-}
 }  // namespace
 
 extern "C" int hs_demag_field_f64_noalloc(hs_demag* d, const double* m, const double* msk, double msat0T0Mul,
@@ -1348,10 +1390,10 @@ extern "C" int hs_demag_reserve(hs_demag* d, int nsolve) {
     if (!d || nsolve < 1) return HS_EINVAL;
     if (nsolve <= d->cap) return 0;
     cpx<float>*X1 = nullptr, *X2 = nullptr, *Xz = nullptr;
-    hipMalloc(&X1, sizeof(cpx<float>) * 3L * d->N[0] * d->N[1] * d->H2p * nsolve);
-    if (!d->fz32) hipMalloc(&X2, sizeof(cpx<float>) * 3L * d->N[0] * d->P[1] * d->H2p * nsolve);
-    if (!d->fz32 && d->gen0) hipMalloc(&Xz, sizeof(cpx<float>) * 3L * d->P[0] * d->P[1] * d->H2p * nsolve);
-    if (!X1 || (!d->fz32 && (!X2 || (d->gen0 && !Xz)))) {
+    hipMalloc(&X1, sizeof(cpx<float>) * fused_spectrum(d, d->fold32) * nsolve);
+    if (!d->fold32) hipMalloc(&X2, sizeof(cpx<float>) * 3L * d->N[0] * d->P[1] * d->H2p * nsolve);
+    if (!d->fold32 && d->gen0) hipMalloc(&Xz, sizeof(cpx<float>) * 3L * d->P[0] * d->P[1] * d->H2p * nsolve);
+    if (!X1 || (!d->fold32 && (!X2 || (d->gen0 && !Xz)))) {
         hipFree(X1);
         hipFree(X2);
         hipFree(Xz);
@@ -1373,11 +1415,13 @@ long hs_demag_ncell(const hs_demag* d) { return d->ncell; }
 long hs_demag_footprint(const hs_demag* d) {
     const long nk = (long)d->K[0] * d->K[1] * d->K[2];
     long b = 6 * nk * (sizeof(double) + sizeof(float));
-    b += (long)sizeof(cpx<float>) * 3L * d->N[0] * (d->N[1] + (d->fz32 ? 0 : d->P[1])) * d->H2p * d->cap;
-    if (d->kt32) b += 6L * d->N[0] * fused_table(d) * d->H2 * (long)sizeof(float);
-    if (d->kt64) b += 6L * d->N[0] * fused_table(d) * d->H2 * (long)sizeof(double);
+    b += (long)sizeof(cpx<float>) * (fused_spectrum(d, d->fold32) + (d->X2f ? 3L * d->N[0] * d->P[1] * d->H2p : 0)) *
+         d->cap;
+    if (d->kt32) b += fused_table(d, d->fold32) * (long)sizeof(float);
+    if (d->kt64) b += fused_table(d, d->fold64) * (long)sizeof(double);
     b += 6L * d->K[0] * d->K[1] * (d->KP - d->H2) * (long)sizeof(float);
-    if (d->X1d) b += (long)sizeof(cpx<double>) * 3L * d->N[0] * (d->N[1] + (d->fz64 ? 0 : d->P[1])) * d->H2p;
+    if (d->X1d)
+        b += (long)sizeof(cpx<double>) * (fused_spectrum(d, d->fold64) + (d->X2d ? 3L * d->N[0] * d->P[1] * d->H2p : 0));
     if (d->Xzf) b += (long)sizeof(cpx<float>) * 3L * d->P[0] * d->P[1] * d->H2p * d->cap;
     if (d->Xzd) b += (long)sizeof(cpx<double>) * 3L * d->P[0] * d->P[1] * d->H2p;
     b += (long)(sizeof(cpx<float>) + sizeof(cpx<double>)) * (d->M + d->P[2] + d->P[1] + d->P[0]);

@@ -21,11 +21,12 @@
 // zero-padded FFT pair (36 N0 flop against about 10 P0 log2 P0 per output),
 // no padding, and any N0.  Its components XX, YY, ZZ and YZ are real and even
 // in d; XZ and XY (odd along axis 0) are imaginary and odd, K~ = i kappa.
-// With u = i x_x in place of x_x and v = i y_x in place of y_x the tensor is
-// real:  v   =  Kxx u - kxy x_y - kxz x_z
+// With u = i x_x in place of x_x and v = -i y_x in place of y_x the tensor is
+// real and symmetric:
+//        v   = -Kxx u + kxy x_y + kxz x_z
 //        y_y =  kxy u + Kyy x_y + Kyz x_z
-//        y_z =  kxz u + Kyz x_y + Kzz x_z,
-// and -d transposes it.  A mirrored row P1 - j' has Kyz and kxy negated.
+//        y_z =  kxz u + Kyz x_y + Kzz x_z;
+// at -d kxy and kxz are negated, in a mirrored row P1 - j' kxy and Kyz.
 #pragma once
 
 #include <algorithm>
@@ -57,15 +58,18 @@ constexpr Split2 split_even(int L) {
 template <typename T>
 struct Mid {
     cpx<T>* X;
-    const T* kt;  // [column][d][KR][6]: XX, YY, ZZ, YZ, kappa XZ, kappa XY
-    int N0, ncol, CB, nsolve;
-    const cpx<T>* tw;  // w_Q^t, t < Q
+    const T* kt;  // [column][d][KR][6]: -XX, YY, ZZ, YZ, kappa XZ, kappa XY
+    int N0, ncol, CB, nsolve, R;
+    const cpx<T>* tw;  // w_P1^t, P1 = Q R
     const int* live;   // per-solve flags or null
 };
 
 // Table rows of K~ for a Q-point axis 1: frequency q = k1 + A k2 sits in slot
 // k1 B + k2; rows q and Q - q share |K|, and the slots k1 <= A/2 cover both.
-constexpr int table_rows(int Q) { return (split_even(Q).A / 2 + 1) * split_even(Q).B; }
+// A folded column (see k_frows) has all Q rows; its mirror is another column.
+constexpr int table_rows(int Q, bool fold) { return fold ? Q : (split_even(Q).A / 2 + 1) * split_even(Q).B; }
+// K~ columns per x frequency: 1, or the residues s <= R/2 of a folded axis 1
+constexpr int table_cols(int R) { return R > 1 ? R / 2 + 1 : 1; }
 
 // the tensor at one distance and row (six values from an 8- or 16-byte boundary)
 template <typename T>
@@ -79,18 +83,40 @@ struct Coef {
 };
 __device__ __forceinline__ float fmaT(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fmaT(double a, double b, double c) { return __builtin_fma(a, b, c); }
-// axis-0 items per thread: 3 IB values each, at most kEpt in all
+// axis-0 items per thread: 3 IB values each, at most 24 in all
 constexpr int mid_itm(int IB) { return 8 / IB; }
+
+// The table entry (distance 0) of column tc's slot; sj = -1 for a mirrored row.
+template <typename T, int Q, bool FOLD>
+__device__ __forceinline__ const T* table_row(const Mid<T>& a, int tc, int slot, T& sj) {
+    constexpr int A = split_even(Q).A, B = split_even(Q).B;
+    bool mir;
+    int row;
+    if constexpr (FOLD) {  // column k R + s: frequencies R q + s, mirrored at R (Q - 1 - q) + R - s
+        const int k = tc / a.R, s = tc % a.R;
+        mir = 2 * s > a.R;
+        row = mir ? Q - 1 - slot : slot;
+        tc = k * (a.R / 2 + 1) + (mir ? a.R - s : s);
+    } else {
+        const int k1 = slot / B, k2 = slot % B;
+        mir = k1 > A / 2;
+        row = mir ? (A - k1) * B + (B - 1 - k2) : slot;
+    }
+    sj = mir ? T(-1) : T(1);
+    constexpr int KR = table_rows(Q, FOLD);
+    return a.kt + ((long)tc * a.N0 * KR + row) * 6;
+}
 
 // One block: CB columns of one solve, 3 N0 pencils of Q points each, held in
 // LDS as lds[pencil * A (B+1) + k1 (B+1) + k2] (the odd row pitch keeps both
 // phases free of bank conflicts).  blockDim.x = elements / kEpt, rounded up
 // to whole waves.
-template <typename T, int Q, int IB, bool MULTI>
+// Axis 0 in items of IB planes (MULTI: N0 > IB).
+template <typename T, int Q, int IB, bool MULTI, bool FOLD>
 __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
-    constexpr int A = split_even(Q).A, B = split_even(Q).B, BP = B + 1, PL = A * BP, AIN = A / 2;
+    constexpr int A = split_even(Q).A, B = split_even(Q).B, BP = B + 1, PL = A * BP, AIN = FOLD ? A : A / 2;
     constexpr int UA = (kEpt + A - 1) / A, UB = (kEpt + B - 1) / B, ITM = mid_itm(IB);
-    constexpr int KR = (A / 2 + 1) * B, N1 = Q / 2;
+    constexpr int KR = table_rows(Q, FOLD), N1 = FOLD ? Q : Q / 2;
     static_assert(A * B == Q && A % 2 == 0, "two-level split");
     extern __shared__ __align__(16) unsigned char mid_smem[];
     cpx<T>* tws = reinterpret_cast<cpx<T>*>(mid_smem);
@@ -102,7 +128,7 @@ __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
     const int N0 = a.N0, col0 = tile * a.CB, ncb = min(a.CB, a.ncol - col0);
     const int PC = 3 * N0, NP = PC * ncb;
     cpx<T>* X = a.X + ((long)sol * a.ncol + col0) * (long)(PC * N1);
-    {  // phase 1: A-point DFTs over n1 of the rows j = B n1 + n2 < N1
+    {  // phase 1: A-point DFTs over n1 of the rows j = B n1 + n2 < N1 (the upper half is padding unless folded)
         cpx<T> v[UA][A];
 #pragma unroll
         for (int u = 0; u < UA; u++) {
@@ -112,7 +138,7 @@ __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
 #pragma unroll
             for (int n1 = 0; n1 < AIN; n1++) v[u][n1] = xp[B * n1];
         }
-        for (int t = tid; t < Q; t += NT) tws[t] = a.tw[t];
+        for (int t = tid; t < Q; t += NT) tws[t] = a.tw[FOLD ? t * a.R : t];
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < UA; u++) {
@@ -159,12 +185,9 @@ __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
             for (int q = 0; q < IB; q++) y[it][0][q] = y[it][1][q] = y[it][2][q] = {T(0), T(0)};
             if (e < items) {
                 const int slot = e % Q, r = e / Q, ib = MULTI ? r % NIB : 0, col = MULTI ? r / NIB : r;
-                const int k1 = slot / B, k2 = slot % B;
-                const bool mir = k1 > A / 2;
-                const int row = mir ? (A - k1) * B + (B - 1 - k2) : slot;
-                const T sj = mir ? T(-1) : T(1);
-                const T* kb = a.kt + ((long)(col0 + col) * N0 * KR + row) * 6;
-                const cpx<T>* xs = lds + col * PC * PL + k1 * BP + k2;
+                T sj;
+                const T* kb = table_row<T, Q, FOLD>(a, col0 + col, slot, sj);
+                const cpx<T>* xs = lds + col * PC * PL + slot / B * BP + slot % B;
                 // K~ at plane distance ad >= 0 for this row
                 auto coef = [&](int ad, Coef<T>& w) {
                     w.load(kb + (long)ad * (6 * KR));
@@ -177,8 +200,8 @@ __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
                     cpx<T>&a0 = y[it][0][q], &a1 = y[it][1][q], &a2 = y[it][2][q];
                     // chained into the accumulators: three fma each (a sum of products
                     // added afterwards takes a fourth instruction)
-                    a0.x = fmaT(-xz, x2.x, fmaT(-xy, x1.x, fmaT(w.xx, x0.x, a0.x)));
-                    a0.y = fmaT(-xz, x2.y, fmaT(-xy, x1.y, fmaT(w.xx, x0.y, a0.y)));
+                    a0.x = fmaT(xz, x2.x, fmaT(xy, x1.x, fmaT(w.xx, x0.x, a0.x)));
+                    a0.y = fmaT(xz, x2.y, fmaT(xy, x1.y, fmaT(w.xx, x0.y, a0.y)));
                     a1.x = fmaT(w.yz, x2.x, fmaT(w.yy, x1.x, fmaT(xy, x0.x, a1.x)));
                     a1.y = fmaT(w.yz, x2.y, fmaT(w.yy, x1.y, fmaT(xy, x0.y, a1.y)));
                     a2.x = fmaT(w.zz, x2.x, fmaT(w.yz, x1.x, fmaT(xz, x0.x, a2.x)));
@@ -273,9 +296,9 @@ __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
                 for (int k1 = 0; k1 < A; k1++) v[k1] = lds[p * PL + k1 * BP + n2];
                 dft_reg<T, A, +1>(v);
                 cpx<T>* xp = X + p * N1 + n2;
-                if (p % PC < N0) {  // y_x = -i v
+                if (p % PC < N0) {  // y_x = i v
 #pragma unroll
-                    for (int n1 = 0; n1 < AIN; n1++) xp[B * n1] = {v[n1].y, -v[n1].x};
+                    for (int n1 = 0; n1 < AIN; n1++) xp[B * n1] = {-v[n1].y, v[n1].x};
                 } else {
 #pragma unroll
                     for (int n1 = 0; n1 < AIN; n1++) xp[B * n1] = v[n1];
@@ -299,20 +322,71 @@ constexpr int frow_lds() {
     return (W * A * (B + 1) > W * row_pitch<M, W>()) ? W * A * (B + 1) : W * row_pitch<M, W>();
 }
 
-// R2C of rows [row0, row0 + W) of x times 2 half (rows of n2 reals; the mask
-// repeats every mrows rows), out column-major: out[(sol (M+1) + k) rows + row].
-template <typename T, int M, int W, int NT = W * split2(M).B>
-__global__ void __launch_bounds__(NT) k_frows(const T* __restrict__ x, const T* __restrict__ msk, long mrows,
-                                              cpx<T>* __restrict__ out, long nrows, int rows, int n2,
-                                              T half, const cpx<T>* __restrict__ twM,
-                                              const cpx<T>* __restrict__ twP, Live lv) {
+// Rows of a block.  R = 1: W consecutive rows.  R > 1 (axis 1 folded by R):
+// where a whole column, 3 N0 P1 points, is too large for LDS, the first radix
+// R of axis 1 is done here: P1 = R Q, and the block takes the rows j' + Q m,
+// m < R/2 (the others are padding), of W / (R/2) consecutive j' of one pencil:
+//   x_s[j'] = w_P1^(s j') sum_m w_R^(s m) x[j' + Q m],  s < R,
+// whose Q-point transforms are the frequencies R q + s.  The spectrum then has
+// R columns per x frequency, [solve][k][s][c][i][j' < Q].
+struct RowP {
+    int rows, N1, Q, PC;  // rows and pencils (3 N0) of a solve
+    int nsolve, n2;
+    long mrows;           // rows of the mask
+};
+template <int W, int R>
+struct RowMap {
+    static constexpr int RH = R > 1 ? R / 2 : 1, WA = W / RH;
+    long row0;      // R = 1: first row; R > 1: first row of the pencil
+    int j0, sol, pen;
+    __device__ __forceinline__ RowMap(const RowP& g) {
+        const int b = xcd_swizzle(blockIdx.x, gridDim.x);
+        if constexpr (R == 1) {
+            row0 = (long)b * W;
+            j0 = sol = pen = 0;
+        } else {
+            const int ng = (g.Q + WA - 1) / WA;
+            row0 = (long)(b / ng) * g.N1;
+            j0 = b % ng * WA;
+            sol = b / ng / g.PC;
+            pen = b / ng - sol * g.PC;
+        }
+    }
+    // row of slot p (p = m WA + a), and whether it exists
+    __device__ __forceinline__ long row(const RowP& g, int p, bool& in) const {
+        if constexpr (R == 1) {
+            in = row0 + p < (long)g.rows * g.nsolve;
+            return in ? row0 + p : row0;
+        } else {
+            const int j = j0 + p % WA;
+            in = j < g.Q;
+            return row0 + (in ? j : 0) + (long)g.Q * (p / WA);
+        }
+    }
+    __device__ __forceinline__ bool dead(const RowP& g, const Live& lv) const {
+        if constexpr (R == 1) {
+            const long last = (long)g.rows * g.nsolve - 1;
+            return all_dead(lv, row0, row0 + W - 1 < last ? row0 + W - 1 : last);
+        } else {
+            return lv.flag && !lv.flag[sol];
+        }
+    }
+};
+
+// R2C of a block's rows of x times 2 half (rows of n2 reals; the mask repeats
+// every mrows rows), written column by column.
+template <typename T, int M, int W, int R, int NT = W * split2(M).B>
+__global__ void __launch_bounds__(NT) k_frows(const T* __restrict__ x, const T* __restrict__ msk,
+                                              cpx<T>* __restrict__ out, RowP g, T half,
+                                              const cpx<T>* __restrict__ twM, const cpx<T>* __restrict__ twP,
+                                              const cpx<T>* __restrict__ tw1, Live lv) {
     constexpr int A = split2(M).A, B = split2(M).B, BP = B + 1, PM = row_pitch<M, W>();
     static_assert(A * B == M && A <= B, "two-level split");
     __shared__ cpx<T> lds[frow_lds<M, W>()];
     __shared__ cpx<T> tws[M + 1];
-    const int tid = threadIdx.x;
-    const long row0 = (long)xcd_swizzle(blockIdx.x, gridDim.x) * W;
-    if (all_dead(lv, row0, (row0 + W <= nrows ? row0 + W : nrows) - 1)) return;
+    const int tid = threadIdx.x, n2 = g.n2;
+    const RowMap<W, R> rm(g);
+    if (rm.dead(g, lv)) return;
     constexpr int TA = (M + NT - 1) / NT, TB = (M + 1 + NT - 1) / NT;
     cpx<T> ta[TA], tb[TB];
 #pragma unroll
@@ -321,11 +395,10 @@ __global__ void __launch_bounds__(NT) k_frows(const T* __restrict__ x, const T* 
     for (int q = 0; q < TB; q++) tb[q] = twP[tid + q * NT <= M ? tid + q * NT : 0];
     {
         const int nb = tid % B, p = tid / B;
-        const long r = row0 + p;
-        const bool rin = r < nrows;
-        const long rc = rin ? r : row0;
+        bool rin;
+        const long rc = rm.row(g, p, rin);
         const T* xr = x + rc * n2;
-        const T* mr = msk ? msk + (rc % mrows) * n2 : nullptr;
+        const T* mr = msk ? msk + (rc % g.mrows) * n2 : nullptr;
         cpx<T> v[A];
         if ((n2 & 1) == 0) {  // uniform
             using V2 = typename std::conditional<sizeof(T) == 4, float2, double2>::type;
@@ -394,57 +467,114 @@ __global__ void __launch_bounds__(NT) k_frows(const T* __restrict__ x, const T* 
         for (int k2 = 0; k2 < B; k2++) lds[p2 * PM + k1 + A * k2] = u[k2];
     }
     __syncthreads();
-    // split X[k] = E + w^k O: lanes walk the W rows first, so that a column's W values leave together
-    const int p = tid % W, kk = tid / W;
-    const long r = row0 + p;
-    if (r < nrows) {
-        const long sol = r / rows;
-        cpx<T>* o = out + sol * (M + 1) * (long)rows + (r - sol * rows);
-        auto split = [&](int k) {
-            const cpx<T> zk = lds[p * PM + (k == M ? 0 : k)];
-            const cpx<T> zm = lds[p * PM + (k == 0 ? 0 : M - k)];
-            const cpx<T> E = {half * (zk.x + zm.x), half * (zk.y - zm.y)};
-            const cpx<T> O = {half * (zk.y + zm.y), half * (zm.x - zk.x)};
-            o[(long)k * rows] = cadd(E, cmul(tws[k], O));
-        };
+    // split X[k] = E + w^k O
+    auto split = [&](int p, int k) {
+        const cpx<T> zk = lds[p * PM + (k == M ? 0 : k)];
+        const cpx<T> zm = lds[p * PM + (k == 0 ? 0 : M - k)];
+        const cpx<T> E = {half * (zk.x + zm.x), half * (zk.y - zm.y)};
+        const cpx<T> O = {half * (zk.y + zm.y), half * (zm.x - zk.x)};
+        return cadd(E, cmul(tws[k], O));
+    };
+    if constexpr (R == 1) {  // lanes walk the W rows first, so that a column's W values leave together
+        const int p = tid % W, kk = tid / W;
+        bool in;
+        const long r = rm.row(g, p, in);
+        if (in) {
+            const long sol = r / g.rows;
+            cpx<T>* o = out + sol * (M + 1) * (long)g.rows + (r - sol * g.rows);
 #pragma unroll
-        for (int q = 0; q < A; q++) split(kk + B * q);
-        if (kk == 0) split(M);
+            for (int q = 0; q < A; q++) o[(long)(kk + B * q) * g.rows] = split(p, kk + B * q);
+            if (kk == 0) o[(long)M * g.rows] = split(p, M);
+        }
+    } else {  // ... the WA values of j' first
+        constexpr int RH = R / 2, WA = W / RH, KS = NT / WA;
+        const int a = tid % WA, kk = tid / WA, j = rm.j0 + a;
+        if (j < g.Q) {
+            cpx<T> wj[R];
+#pragma unroll
+            for (int s = 1; s < R; s++) wj[s] = tw1[s * j];
+            const long cs = (long)g.PC * g.Q;
+            cpx<T>* o = out + rm.sol * (long)(M + 1) * R * cs + (long)rm.pen * g.Q + j;
+            for (int k = kk; k <= M; k += KS) {
+                cpx<T> f[R];
+#pragma unroll
+                for (int m = 0; m < R; m++) f[m] = m < RH ? split(m * WA + a, k) : cpx<T>{T(0), T(0)};
+                dft_reg<T, R, -1>(f);
+#pragma unroll
+                for (int s = 0; s < R; s++) o[((long)k * R + s) * cs] = s ? cmul(f[s], wj[s]) : f[s];
+            }
+        }
     }
 }
 
-// C2R of rows [row0, row0 + W) from the column-major spectrum.
-template <typename T, int M, int W, int NT = W * split2(M).B>
-__global__ void __launch_bounds__(NT) k_irows(const cpx<T>* __restrict__ in, T* __restrict__ x, long nrows, int rows,
-                                              int n2, const cpx<T>* __restrict__ twM,
-                                              const cpx<T>* __restrict__ twP, Live lv) {
+// C2R of a block's rows from the column-major spectrum; R > 1: the last radix
+// of axis 1 first, x[j' + Q m] = sum_s w_R^(-s m) w_P1^(-s j') z_s[j'].
+template <typename T, int M, int W, int R, int NT = W * split2(M).B>
+__global__ void __launch_bounds__(NT) k_irows(const cpx<T>* __restrict__ in, T* __restrict__ x, RowP g,
+                                              const cpx<T>* __restrict__ twM, const cpx<T>* __restrict__ twP,
+                                              const cpx<T>* __restrict__ tw1, Live lv) {
     constexpr int A = split2(M).A, B = split2(M).B, BP = B + 1, PM = row_pitch<M, W>();
     static_assert(A * B == M && A <= B, "two-level split");
     __shared__ cpx<T> lds[frow_lds<M, W>()];
     __shared__ cpx<T> tws[M];
     __shared__ cpx<T> twp[M];
-    const int tid = threadIdx.x;
-    const long row0 = (long)xcd_swizzle(blockIdx.x, gridDim.x) * W;
-    if (all_dead(lv, row0, (row0 + W <= nrows ? row0 + W : nrows) - 1)) return;
+    const int tid = threadIdx.x, n2 = g.n2;
+    const RowMap<W, R> rm(g);
+    if (rm.dead(g, lv)) return;
     {
-        const int p = tid % W, kk = tid / W;
-        const long r = row0 + p < nrows ? row0 + p : row0;  // a valid row for the lanes past the end
-        const long sol = r / rows;
-        const cpx<T>* q0 = in + sol * (M + 1) * (long)rows + (r - sol * rows);
         constexpr int TA = (M + NT - 1) / NT;
-        cpx<T> g[A], gm, ta[TA], tb[TA];
-#pragma unroll
-        for (int q = 0; q < A; q++) g[q] = q0[(long)(kk + B * q) * rows];
-        gm = q0[(long)M * rows];
+        cpx<T> ta[TA], tb[TA];
 #pragma unroll
         for (int q = 0; q < TA; q++) {
             const int e = tid + q * NT;
             ta[q] = twM[e < M ? e : 0];
             tb[q] = twP[e < M ? e : 0];
         }
+        if constexpr (R == 1) {
+            const int p = tid % W, kk = tid / W;
+            bool ok;
+            const long r = rm.row(g, p, ok);
+            const long sol = r / g.rows;
+            const cpx<T>* q0 = in + sol * (M + 1) * (long)g.rows + (r - sol * g.rows);
+            cpx<T> v[A], vm;
 #pragma unroll
-        for (int q = 0; q < A; q++) lds[p * PM + kk + B * q] = g[q];
-        if (kk == 0) lds[p * PM + M] = gm;
+            for (int q = 0; q < A; q++) v[q] = q0[(long)(kk + B * q) * g.rows];
+            vm = q0[(long)M * g.rows];
+#pragma unroll
+            for (int q = 0; q < A; q++) lds[p * PM + kk + B * q] = v[q];
+            if (kk == 0) lds[p * PM + M] = vm;
+        } else {
+            constexpr int RH = R / 2, WA = W / RH, KS = NT / WA, U = 16 / R > 1 ? 16 / R : 1;
+            const int a = tid % WA, kk = tid / WA, j = rm.j0 + a < g.Q ? rm.j0 + a : 0;
+            cpx<T> wj[R];
+#pragma unroll
+            for (int s = 1; s < R; s++) {
+                wj[s] = tw1[s * j];
+                wj[s].y = -wj[s].y;
+            }
+            const long cs = (long)g.PC * g.Q;
+            const cpx<T>* q0 = in + rm.sol * (long)(M + 1) * R * cs + (long)rm.pen * g.Q + j;
+            for (int k0 = kk; k0 <= M; k0 += U * KS) {  // U frequencies of R loads in flight
+                cpx<T> f[U][R];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const long k = k0 + u * KS <= M ? k0 + u * KS : M;
+#pragma unroll
+                    for (int s = 0; s < R; s++) f[u][s] = q0[(k * R + s) * cs];
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int k = k0 + u * KS;
+                    if (k <= M) {
+#pragma unroll
+                        for (int s = 1; s < R; s++) f[u][s] = cmul(f[u][s], wj[s]);
+                        dft_reg<T, R, +1>(f[u]);
+#pragma unroll
+                        for (int m = 0; m < RH; m++) lds[(m * WA + a) * PM + k] = f[u][m];
+                    }
+                }
+            }
+        }
 #pragma unroll
         for (int q = 0; q < TA; q++) {
             const int e = tid + q * NT;
@@ -480,12 +610,13 @@ __global__ void __launch_bounds__(NT) k_irows(const cpx<T>* __restrict__ in, T* 
     __syncthreads();
     if (tid < W * A) {
         const int k1 = tid % A, p2 = tid / A;
-        const long r = row0 + p2;
+        bool rin;
+        const long r = rm.row(g, p2, rin);
         cpx<T> u[B];
 #pragma unroll
         for (int m = 0; m < B; m++) u[m] = lds[(p2 * A + k1) * BP + m];
         dft_reg<T, B, +1>(u);
-        if (r < nrows) {
+        if (rin) {
             using V2 = typename std::conditional<sizeof(T) == 4, float2, double2>::type;
             T* xr = x + r * n2;
 #pragma unroll
@@ -528,10 +659,41 @@ inline int mid_nt(int N0, int Q, int CB) {
 inline bool mid_fits(int N0, int Q, int A, int B, size_t cs) {
     return mid_nt(N0, Q, 1) <= kMidMax && mid_lds(Q, A, B, N0, 1, cs) <= (size_t)kLds;
 }
-// Columns per block: about 6144 elements (three blocks a CU), fewer while the
-// launch would leave CUs idle.  A column's arithmetic does not depend on it.
+// Tile elements (complex) of a block that leave a CU six blocks (half of it,
+// three).  Small tiles hide each other's phases: 3072 against 6144 elements
+// take 24.7 against 30.8 us at 32 solves of 128x128x2, 13.5 against 14.7 at
+// 64x64x4.
+constexpr long kTile = 3072;
+// The direct convolution's N0^2 products pass the zero-padded FFTs of the five
+// passes between 32 planes (three kernels 98 us, five passes 160 at 32 solves
+// of 32x32x32) and 64 (54 against 43 us at 64x64x64).
+constexpr int kPlanes = 32;
+inline long mid_elems(size_t cs) { return kTile * 8 / (long)cs; }
+// Fold R of axis 1 for N0 planes and P1 points (fits(R): registered and a
+// column fits a block), 0 if none.  No folding up to 6144 elements a column
+// (FP64: 3072).  Beyond, a column leaves too few blocks a CU, and folding
+// until it has 3072 elements is best while the rows still leave in 64-byte
+// pieces (R <= 4: 42.4 us a field at 256x256x8 against 45.7 with R = 2 and
+// 48.3 without), else until it has 6144 (R = 8 at 512x512x16: 298 us, R = 16
+// with 16-byte pieces 334; five passes 317).  FP64 stops at R = 4: beyond, the
+// five passes are faster (512x512x16: 1050 us against 1127 with R = 16).
+template <typename F>
+int mid_fold(int N0, int P1, size_t cs, F fits) {
+    const long el = kTile;
+    if (N0 > kPlanes) return 0;
+    auto ok = [&](int R, long most) { return P1 % R == 0 && 3L * N0 * (P1 / R) <= most && fits(R); };
+    if (ok(1, cs == 8 ? 2 * el : el)) return 1;
+    for (int R = 2; R <= 4; R *= 2)
+        if (ok(R, el)) return R;
+    if (cs == 8)
+        for (int R = 2; R <= 8; R *= 2)
+            if (ok(R, 2 * el)) return R;
+    return ok(1, 1L << 40) ? 1 : 0;
+}
+// Columns per block: about kTile elements, fewer while the launch would leave
+// CUs idle.  A column's arithmetic does not depend on it.
 inline int mid_cb(int N0, int Q, int A, int B, int ncol, int nsolve, size_t cs) {
-    int cb = std::max(1, 6144 * 8 / (int)cs / (3 * N0 * Q));
+    int cb = (int)std::max(1L, mid_elems(cs) / (3L * N0 * Q));
     cb = std::min(cb, ncol);
     while (cb > 1 && ((long)((ncol + cb - 1) / cb) * nsolve < 512 || mid_nt(N0, Q, cb) > kMidMax ||
                       mid_lds(Q, A, B, N0, cb, cs) > (size_t)kLds))
@@ -540,77 +702,113 @@ inline int mid_cb(int N0, int Q, int A, int B, int ncol, int nsolve, size_t cs) 
 }
 // ---- registry ---------------------------------------------------------------
 template <typename T>
-using frows_t = void (*)(const T*, const T*, long, cpx<T>*, long, int, int, T, const cpx<T>*, const cpx<T>*,
+using frows_t = void (*)(const T*, const T*, cpx<T>*, const RowP&, T, const cpx<T>*, const cpx<T>*, const cpx<T>*,
                          hipStream_t, Live);
 template <typename T>
-using irows_t = void (*)(const cpx<T>*, T*, long, int, int, const cpx<T>*, const cpx<T>*, hipStream_t, Live);
+using irows_t = void (*)(const cpx<T>*, T*, const RowP&, const cpx<T>*, const cpx<T>*, const cpx<T>*, hipStream_t,
+                         Live);
 template <typename T>
 using mid_t = void (*)(const Mid<T>&, hipStream_t);
 
+constexpr int kFolds = 4;  // R = 1, 2, 4, 8
 template <typename T>
 struct Rows {
-    frows_t<T> fwd = nullptr;
-    irows_t<T> inv = nullptr;
+    frows_t<T> fwd[kFolds] = {};
+    irows_t<T> inv[kFolds] = {};
 };
 template <typename T>
 struct Mids {
-    mid_t<T> one[9] = {};    // N0 = 1..8 planes
-    mid_t<T> multi[9] = {};  // more, in blocks of 6 or 8
+    mid_t<T> one[2][9] = {};    // [folded] N0 = 1..8 planes
+    mid_t<T> multi[2][9] = {};  // more, in blocks of 6 or 8
     int A = 0, B = 0;
-    mid_t<T> pick(int N0) const { return N0 <= 8 ? one[N0] : multi[mid_ib(N0)]; }
+    mid_t<T> pick(int N0, bool fold) const {
+        return N0 <= 8 ? one[fold][N0] : multi[fold][mid_ib(N0)];
+    }
 };
+inline int fold_index(int R) { return R == 1 ? 0 : (R == 2 ? 1 : (R == 4 ? 2 : 3)); }
+inline int table_rows_of(int Q, bool fold) { return table_rows(Q, fold); }
 template <typename T>
 Rows<T>& rows_of(int M);  // registries, defined in demag.hip
 template <typename T>
 Mids<T>& mids_of(int Q);
 
 // Rows per block: full 128-byte pieces of a column (16 rows of 8 bytes) while
-// the tile stays near 32 KB.
-template <typename T, int M>
+// the tile stays near 32 KB; folded, pieces of 32 bytes or more (neighbouring
+// blocks complete the lines in L2) at up to 72 KB.
+template <typename T, int M, int R>
 constexpr int frow_w() {
-    int w = 128 / (int)sizeof(cpx<T>);
-    while (w > 2 && ((long)w * M * (long)sizeof(cpx<T>) > 40000 || w * split2(M).B > 1024)) w /= 2;
+    constexpr int cs = (int)sizeof(cpx<T>), rh = R > 1 ? R / 2 : 1;
+    int w = 128 / cs;
+    if (R > 1) w = 16;
+    if (w < rh) w = rh;
+    while (w > 2 && w > rh && ((long)w * M * cs > (R > 1 ? 72000 : 40000) || w * split2(M).B > 1024)) w /= 2;
     while (w < 16 && w * split2(M).B < 64) w *= 2;
     return w;
 }
-template <typename T, int M>
-void launch_frows(const T* x, const T* msk, long mrows, cpx<T>* out, long nrows, int rows, int n2, T half,
-                  const cpx<T>* twM, const cpx<T>* twP, hipStream_t st, Live lv) {
-    constexpr int W = frow_w<T, M>();
-    hipLaunchKernelGGL((k_frows<T, M, W>), dim3((unsigned)((nrows + W - 1) / W)), dim3(W * split2(M).B), 0, st, x, msk,
-                       mrows, out, nrows, rows, n2, half, twM, twP, lv);
+template <typename T, int M, int R>
+unsigned frow_grid(const RowP& g) {
+    constexpr int W = frow_w<T, M, R>(), WA = R > 1 ? W / (R / 2) : W;
+    if (R == 1) return (unsigned)(((long)g.rows * g.nsolve + W - 1) / W);
+    return (unsigned)((long)g.nsolve * g.PC * ((g.Q + WA - 1) / WA));
 }
-template <typename T, int M>
-void launch_irows(const cpx<T>* in, T* x, long nrows, int rows, int n2, const cpx<T>* twM, const cpx<T>* twP,
+template <typename T, int M, int R>
+void launch_frows(const T* x, const T* msk, cpx<T>* out, const RowP& g, T half, const cpx<T>* twM, const cpx<T>* twP,
+                  const cpx<T>* tw1, hipStream_t st, Live lv) {
+    constexpr int W = frow_w<T, M, R>();
+    hipLaunchKernelGGL((k_frows<T, M, W, R>), dim3(frow_grid<T, M, R>(g)), dim3(W * split2(M).B), 0, st, x, msk, out,
+                       g, half, twM, twP, tw1, lv);
+}
+template <typename T, int M, int R>
+void launch_irows(const cpx<T>* in, T* x, const RowP& g, const cpx<T>* twM, const cpx<T>* twP, const cpx<T>* tw1,
                   hipStream_t st, Live lv) {
-    constexpr int W = frow_w<T, M>();
-    hipLaunchKernelGGL((k_irows<T, M, W>), dim3((unsigned)((nrows + W - 1) / W)), dim3(W * split2(M).B), 0, st, in, x,
-                       nrows, rows, n2, twM, twP, lv);
+    constexpr int W = frow_w<T, M, R>();
+    hipLaunchKernelGGL((k_irows<T, M, W, R>), dim3(frow_grid<T, M, R>(g)), dim3(W * split2(M).B), 0, st, in, x, g,
+                       twM, twP, tw1, lv);
 }
 
-template <typename T, int Q, int IB, bool MULTI>
+template <typename T, int Q, int IB, bool MULTI, bool FOLD>
 void launch_mid(const Mid<T>& m, hipStream_t st) {
     constexpr int A = split_even(Q).A, B = split_even(Q).B;
     const size_t lds = mid_lds(Q, A, B, m.N0, m.CB, sizeof(cpx<T>));
     const int nt = mid_nt(m.N0, Q, m.CB);
     if (lds > 65536)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fmid<T, Q, IB, MULTI>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fmid<T, Q, IB, MULTI, FOLD>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const unsigned g = (unsigned)((m.ncol + m.CB - 1) / m.CB) * (unsigned)m.nsolve;
-    hipLaunchKernelGGL((k_fmid<T, Q, IB, MULTI>), dim3(g), dim3(nt), lds, st, m);
+    hipLaunchKernelGGL((k_fmid<T, Q, IB, MULTI, FOLD>), dim3(g), dim3(nt), lds, st, m);
 }
 
+template <typename T, int M, int F>
+void add_rows_fold(Rows<T>& r) {
+    constexpr int R = 1 << F, W = frow_w<T, M, R>();
+    constexpr long lds = ((long)frow_lds<M, W>() + 2 * M) * (long)sizeof(cpx<T>);
+    if constexpr (lds <= kLds && W * split2(M).B <= 1024) {
+        r.fwd[F] = &launch_frows<T, M, R>;
+        r.inv[F] = &launch_irows<T, M, R>;
+    }
+}
 template <typename T, int M>
 void add_rows() {
-    if constexpr (two_level_ok(M) && M >= 8) rows_of<T>(M) = {&launch_frows<T, M>, &launch_irows<T, M>};
+    if constexpr (two_level_ok(M) && M >= 8) {
+        Rows<T>& r = rows_of<T>(M);
+        add_rows_fold<T, M, 0>(r), add_rows_fold<T, M, 1>(r), add_rows_fold<T, M, 2>(r);
+        if constexpr (sizeof(T) == 4) add_rows_fold<T, M, 3>(r);
+    }
 }
-template <typename T, int Q, int IB>
+template <typename T, int Q, int IB, bool FOLD>
 void add_mid_ib(Mids<T>& m) {
     // only what can fit a block (mid_fits): LDS, and items per thread
     constexpr int A = split_even(Q).A, B = split_even(Q).B;
     constexpr long lds = (3L * IB * A * (B + 1) + Q) * (long)sizeof(cpx<T>);
-    if constexpr (lds <= kLds && Q <= kMidMax * mid_itm(IB)) m.one[IB] = &launch_mid<T, Q, IB, false>;
-    if constexpr ((IB == 6 || IB == 8) && lds * 3 / 2 <= kLds) m.multi[IB] = &launch_mid<T, Q, IB, true>;
+    if constexpr (lds <= kLds && Q <= kMidMax * mid_itm(IB)) m.one[FOLD][IB] = &launch_mid<T, Q, IB, false, FOLD>;
+    if constexpr ((IB == 6 || IB == 8) && lds * 3 / 2 <= kLds)
+        m.multi[FOLD][IB] = &launch_mid<T, Q, IB, true, FOLD>;
+}
+template <typename T, int Q, bool FOLD>
+void add_mid_fold(Mids<T>& m) {
+    add_mid_ib<T, Q, 1, FOLD>(m), add_mid_ib<T, Q, 2, FOLD>(m), add_mid_ib<T, Q, 3, FOLD>(m);
+    add_mid_ib<T, Q, 4, FOLD>(m), add_mid_ib<T, Q, 5, FOLD>(m), add_mid_ib<T, Q, 6, FOLD>(m);
+    add_mid_ib<T, Q, 7, FOLD>(m), add_mid_ib<T, Q, 8, FOLD>(m);
 }
 template <typename T, int Q>
 void add_mid() {
@@ -618,13 +816,17 @@ void add_mid() {
         Mids<T>& m = mids_of<T>(Q);
         m.A = split_even(Q).A;
         m.B = split_even(Q).B;
-        add_mid_ib<T, Q, 1>(m), add_mid_ib<T, Q, 2>(m), add_mid_ib<T, Q, 3>(m), add_mid_ib<T, Q, 4>(m);
-        add_mid_ib<T, Q, 5>(m), add_mid_ib<T, Q, 6>(m), add_mid_ib<T, Q, 7>(m), add_mid_ib<T, Q, 8>(m);
+        add_mid_fold<T, Q, false>(m);
+        add_mid_fold<T, Q, true>(m);
     }
 }
-template <typename T, int L>
-void register_len() {
-    add_rows<T, L>();
-    add_mid<T, L>();
+// every length of a list
+template <typename T, int... L>
+void register_rows() {
+    (add_rows<T, L>(), ...);
+}
+template <typename T, int... Q>
+void register_mids() {
+    (add_mid<T, Q>(), ...);
 }
 }  // namespace fused

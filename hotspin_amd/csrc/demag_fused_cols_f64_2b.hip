@@ -1,0 +1,7 @@
+// Fused demag kernels: F64 columns of 2^k points (registered at library load).
+#include "demag_fused.hpp"
+namespace {
+struct Reg {
+    Reg() { fused::register_mids<double, 128, 256, 512, 1024>(); }
+} reg;
+}  // namespace

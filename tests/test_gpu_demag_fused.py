@@ -25,7 +25,9 @@ def _gpu():
     check("demag fused")
 
 
-SHAPES = ([(n0, 8, 16) for n0 in range(1, 10)] +           # planes per item, first of the blocked form
+# folded axis 1 (FP32 beyond 2048 points of N0 P1, FP64 beyond 1024): 2, 4, 8 and 16 ways
+SHAPES = ([(16, 128, 8), (64, 64, 16), (8, 256, 16), (20, 96, 12), (33, 80, 10), (3, 512, 8), (16, 512, 16)] +
+          [(n0, 8, 16) for n0 in range(1, 10)] +           # planes per item, first of the blocked form
           [(10, 8, 16), (12, 4, 8), (13, 8, 8), (16, 16, 8), (17, 4, 16), (33, 8, 8)] +
           [(2, 5, 10), (3, 6, 12), (2, 10, 20), (1, 12, 24), (3, 24, 48), (2, 20, 40), (4, 80, 10)] +
           [(1, 32, 128), (8, 256, 8), (2, 512, 8), (1, 384, 16), (5, 64, 512)])
