@@ -3,8 +3,10 @@
 // B = mu0 Ms0T0Mul * IFFT( K^ . FFT(m .* msat0T0) ), the algorithm of
 // MaxwellPlan.UpdateB (src/hotspin-core/modules/maxwell_convolution.go:103-131)
 // with the reference's cuFFT 3-D D2Z/Z2D replaced by five pruned passes of
-// the library's own LDS-staged FFT (fft.hpp).  Mesh N=(N0,N1,N2) internal,
-// logic size P (x2 on open axes, zeropad.go:12-22), M = P2/2, H2 = M+1:
+// the library's own LDS-staged FFT (fft.hpp), or by three kernels where the
+// columns fit in LDS (demag_fused.hpp: open meshes of up to 32 planes).  Mesh
+// N=(N0,N1,N2) internal, transform lengths P >= the logic size (x2 on open
+// axes, zeropad.go:12-22; set_lengths), M = P2/2, H2 = M+1.  The five passes:
 //   F1  rows, R2C along axis 2 (M-point complex FFT + split), only the N0*N1
 //       non-zero rows are read: m (3N)         -> X1 (3, N0, N1, H2)
 //   F2  columns along axis 1, input rows j < N1:  X1 -> X2 (3, N0, P1, H2)
@@ -371,9 +373,10 @@ __global__ void __launch_bounds__(64) k_kernel_newell(double* __restrict__ oct, 
 }
 
 // Fill the full real (P0,P1,P2) kernel of component c from its octant with
-// the mirror signs of kernel_magnetostatic.go:190-234.
-__global__ void k_kernel_fill(double* __restrict__ full, const double* __restrict__ oct, int s0, int s1, int s2) {
-    const int h0 = s0 / 2 + 1, h1 = s1 / 2 + 1, h2 = s2 / 2 + 1;
+// the mirror signs of kernel_magnetostatic.go:190-234 (octant h0 x h1 x h2;
+// distances beyond it, which no pair of cells has, are zero).
+__global__ void k_kernel_fill(double* __restrict__ full, const double* __restrict__ oct, int s0, int s1, int s2,
+                              int h0, int h1, int h2) {
     const long noct = (long)h0 * h1 * h2;
     const long n = (long)s0 * s1 * s2;
     long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -388,7 +391,7 @@ __global__ void k_kernel_fill(double* __restrict__ full, const double* __restric
     if (c == 5) sg = (fx != fy) ? -1.0 : 1.0;        // XY odd in x and y
     else if (c == 4) sg = (fx != fz) ? -1.0 : 1.0;   // XZ odd in x and z
     else if (c == 3) sg = (fy != fz) ? -1.0 : 1.0;   // YZ odd in y and z
-    full[c * n + g] = sg * oct[c * noct + ((long)xm * h1 + ym) * h2 + zm];
+    full[c * n + g] = xm < h0 && ym < h1 && zm < h2 ? sg * oct[c * noct + ((long)xm * h1 + ym) * h2 + zm] : 0.0;
 }
 
 // Keep the real part of the first octant of the transformed kernel, scaled by
@@ -411,7 +414,7 @@ __global__ void __launch_bounds__(256) k_kernel_extract(const cpx<double>* __res
         cpx<double> v = X[(((long)c * P0 + i) * P1 + j) * H2p + k];
         double r = v.x * norm;
         kern64[c * nk + g] = r;
-        kern32[(long)c * K0 * K1 * KP + ((long)i * K1 + j) * KP + k] = (float)r;
+        if (kern32) kern32[(long)c * K0 * K1 * KP + ((long)i * K1 + j) * KP + k] = (float)r;
         mi = fabs(v.y);
         mr = fabs(v.x);
     }
@@ -583,7 +586,14 @@ cpx<T>* make_twiddles(int L) {
 
 // ------------------------------------------------------------------ plan
 struct hs_demag {
+    // P: the lengths of the transforms, K: octant of the transformed kernel
     int N[3], P[3], K[3], pbc[3];
+    // the reference's logic size (2 N on open axes) and its octant, which
+    // hs_demag_sizes and hs_demag_kernel_f64 report; an open axis whose 2 N has
+    // no compiled family is transformed at a longer P (set_lengths)
+    int logic[3], logicK[3];
+    bool noalloc = false;     // hs_demag_field_f64_noalloc takes the mesh: its spectra at the logic size fit
+    double* kernL = nullptr;  // kernel octants at the logic size where P differs, else kern64
     double cell[3];
     int M, H2, H2p;  // H2p: spectrum row pitch (complex), a multiple of 16 = 128 bytes in FP32
     int KP;          // FP32 kernel row pitch (floats), a multiple of 32 = 128 bytes
@@ -625,32 +635,71 @@ struct Pipe {
     zconv_t<T, T> zc;
 };
 
-// Which passes have a compiled length family (FP32 with registered tile
-// variants; FP64 with a Stockham instantiation) and which take the
-// run-time-length kernels.  False when a generic length exceeds their LDS
+// Lengths with a compiled family: FP32 with registered tile variants, FP64
+// with a Stockham instantiation.
+bool rows32(int P2) {
+    return P2 % 2 == 0 && fft_supported(P2 / 2) && pick_r2c<float, float>(P2 / 2) &&
+           !hsdm::variants(P2 / 2).rows.empty();
+}
+bool rows64(int P2) {
+    return P2 % 2 == 0 && fft_supported(P2 / 2) && pick_r2c<double, double>(P2 / 2) &&
+           pick_c2r<double, double>(P2 / 2);
+}
+bool cols32(int P1) { return pick_cols<float, -1>(P1) && !hsdm::variants(P1).cols.empty(); }
+bool cols64(int P1) { return pick_cols<double, -1>(P1) != nullptr; }
+bool z32_ok(int P0) { return pick_zconv<float, float>(P0) && !hsdm::variants(P0).z.empty(); }
+bool z64_ok(int P0) { return pick_zconv<double, double>(P0) != nullptr; }
+
+// The lengths of the transforms and what follows from them: which passes take
+// the run-time-length kernels.  False when a generic length exceeds their LDS
 // limit (the FP64 kernel set-up transforms every axis).
-bool sizes_ok(hs_demag* d) {
-    const int M = d->M, P1 = d->P[1], P0 = d->P[0];
-    const bool even = d->P[2] % 2 == 0;
-    d->genR = !(even && fft_supported(M) && pick_r2c<float, float>(M) && !hsdm::variants(M).rows.empty());
-    d->gen1 = !(pick_cols<float, -1>(P1) && !hsdm::variants(P1).cols.empty());
-    d->gen0 = !(pick_zconv<float, float>(P0) && !hsdm::variants(P0).z.empty());
-    d->genRd = !(even && fft_supported(M) && pick_r2c<double, double>(M) && pick_c2r<double, double>(M));
-    d->gen1d = !pick_cols<double, -1>(P1);
-    d->gen0d = !pick_zconv<double, double>(P0);
-    d->gR = gen_fft_plan(even ? M : d->P[2]);
+bool set_lengths(hs_demag* d, const int P[3]) {
+    for (int c = 0; c < 3; c++) d->P[c] = P[c];
+    const int P0 = P[0], P1 = P[1], P2 = P[2];
+    d->M = P2 / 2;
+    d->H2 = d->M + 1;
+    d->H2p = (d->H2 + 15) / 16 * 16;
+    d->KP = (d->H2 + 31) / 32 * 32;
+    d->K[0] = P0 / 2 + 1;
+    d->K[1] = P1 / 2 + 1;
+    d->K[2] = d->H2;
+    d->genR = !rows32(P2);
+    d->gen1 = !cols32(P1);
+    d->gen0 = !z32_ok(P0);
+    d->genRd = !rows64(P2);
+    d->gen1d = !cols64(P1);
+    d->gen0d = !z64_ok(P0);
+    d->gR = gen_fft_plan(P2 % 2 == 0 ? d->M : P2);
     d->g1 = gen_fft_plan(P1);
     d->g0 = gen_fft_plan(P0);
     const int lim = gen_max_len<double>();
     return d->gR.L <= lim && P1 <= lim && P0 <= lim;
 }
+// The shortest compiled length >= P, P itself if there is none.
+// An open axis is zero-padded, so any length from 2 N - 1 on gives the same
+// convolution.  2 N itself where it is compiled; otherwise the next of 2^k,
+// 3 2^k and 5 2^k costs at most 1.33 times the points and runs the compiled
+// kernels instead of the run-time-length ones (FP32 field, run-time lengths
+// against padded: 100x75x7 78 -> 20 us, 33^3 171 -> 30, 100^3 383 -> 226,
+// 300x300x33 2086 -> 490, 300x300x17 2502 -> 141; no mesh was slower).
+template <typename F>
+int compiled_length(int P, F ok) {
+    int best = 0;
+#define X(n) \
+    for (int L : {n, 2 * n}) \
+        if (L >= P && ok(L) && (!best || L < best)) best = L;
+    HS_FFT_SIZES(X)
+#undef X
+    return best ? best : P;
+}
+
 // Fold R of axis 1 with which the fused kernels take the mesh (mid_fold), 0 if
 // they do not: open axes 0 and 1 (or one plane), an even padded x length,
 // registered lengths.
 template <typename T>
 int fused_fold(const hs_demag* d) {
     const int P1 = d->P[1], N0 = d->N[0];
-    if (d->P[2] % 2 || P1 != 2 * d->N[1] || !(N0 == 1 || d->P[0] == 2 * N0)) return 0;
+    if (d->P[2] % 2 || P1 < 2 * d->N[1] || !(N0 == 1 || d->P[0] >= 2 * N0)) return 0;
     return fused::mid_fold(N0, P1, sizeof(cpx<T>), [&](int R) {
         const auto& m = fused::mids_of<T>(P1 / R);
         return fused::rows_of<T>(d->M).fwd[fused::fold_index(R)] && m.A && m.pick(N0, R > 1) &&
@@ -687,7 +736,7 @@ int run_fused(hs_demag* d, const T* m, const T* msk, double srcMul, T* B, hipStr
     hs::prof_end(HS_PROF_F1, st);
     hs::prof_begin(HS_PROF_F3K, st);
     const int ncol = d->H2 * R;
-    const fused::Mid<T> a{X,    kt,     N0, ncol, fused::mid_cb(N0, Q, fm.A, fm.B, ncol, nsolve, sizeof(cpx<T>)),
+    const fused::Mid<T> a{X,    kt,     N0, N1, ncol, fused::mid_cb(N0, Q, fm.A, fm.B, ncol, nsolve, sizeof(cpx<T>)),
                           nsolve, R, tw1, live};
     fm.pick(N0, R > 1)(a, st);
     hs::prof_end(HS_PROF_F3K, st);
@@ -837,9 +886,15 @@ void tune32(hs_demag* d, hipStream_t st) {
     d->col32 = (d->gen1 || vc.cols.empty()) ? hsdm::ColV{} : vc.cols[0];
     d->z32 = (d->gen0 || vz.z.empty()) ? hsdm::ZV{} : vz.z[0];
     if (d->fold32) return;  // none of these passes runs
-    // a plan with a run-time-length pass keeps the first variant of its
-    // compiled passes (no timing)
+    // a plan with a run-time-length pass keeps the first variant of its compiled
+    // passes, and so does one at longer lengths than its logic size (unless
+    // forced): the timing takes 0.3 s, which meshes of any size would pay each
+    // for themselves
     if (!d->row32.r2c || !d->col32.fwd || !d->z32.fn) return;
+    if (d->kernL) {
+        apply_force(d, vr, vc, vz);
+        return;
+    }
     const TuneKey key{{d->N[0], d->N[1], d->N[2]}, {d->P[0], d->P[1], d->P[2]}};
     const std::array<int, 3> counts{(int)vr.rows.size(), (int)vc.cols.size(), (int)vz.z.size()};
     {
@@ -1049,18 +1104,57 @@ namespace {
 // static scratch of hs_demag_field_f64_noalloc (below)
 constexpr size_t kScratchBytes = size_t(64) << 20;
 // FP64 spectra of one solve of the plan's mesh: X1, then X2 and (run-time
-// axis-0 length only) Xz, each from a 256-byte boundary
+// axis-0 length only) Xz, each from a 256-byte boundary; fused: X alone
 size_t x_bytes(const hs_demag* d, int rows) { return sizeof(cpx<double>) * 3ull * rows * d->P[1] * d->H2p; }
 size_t up256(size_t b) { return (b + 255) / 256 * 256; }
-size_t noalloc_bytes(const hs_demag* d) {
+size_t noalloc_bytes(const hs_demag* d, int fold) {
+    if (fold) return sizeof(cpx<double>) * (size_t)fused_spectrum(d, fold);
     const size_t x1 = sizeof(cpx<double>) * 3ull * d->N[0] * d->N[1] * d->H2p;
     return up256(x1) + up256(x_bytes(d, d->N[0])) + (d->gen0d ? x_bytes(d, d->P[0]) : 0);
 }
 }  // namespace
 
-// kernel: 0 = Kernel_Arne at `accuracy`, 1 = Newell
+namespace {
+struct KernelBufs {
+    const double* oct;            // real-space octant at the logic size
+    double* full;                 // 6 P0 P1 P2
+    cpx<double>* X;               // 6 P0 P1 H2p
+    unsigned long long* maxbits;
+};
+// FP64 transform of the 6 real components at the plan's lengths, R2C rows, then
+// axes 1 and 0 in place (lengths without a compiled family take the
+// run-time-length passes), and its octant into k64 and k32 (or null).
+void kernel_transform(const hs_demag* d, const KernelBufs& b, double* k64, float* k32, hipStream_t st) {
+    const int P0 = d->P[0], P1 = d->P[1], P2 = d->P[2], H2 = d->H2, H2p = d->H2p;
+    const long P = (long)P0 * P1 * P2, nk = (long)d->K[0] * d->K[1] * d->K[2];
+    const Live all{nullptr, 1};
+    hipMemsetAsync(b.maxbits, 0, 2 * kExtractLanes * sizeof(unsigned long long), st);
+    hipLaunchKernelGGL(k_kernel_fill, dim3(hs::grid1d(P), 6), dim3(hs::kBlock), 0, st, b.full, b.oct, P0, P1, P2,
+                       d->logicK[0], d->logicK[1], d->logicK[2]);
+    if (d->genRd)
+        gen::r2c<double>(b.full, nullptr, 1, b.X, 6L * P0 * P1, P2, P2, H2p, d->gR,
+                         row_table<double>(d, d->twMd, d->twP2d), d->twP2d, st, all);
+    else
+        pick_r2c<double, double>(d->M)(b.full, nullptr, 1, b.X, 6L * P0 * P1, P2, H2p, d->twMd, d->twP2d, st);
+    Geo ga1 = {(long)P1 * H2p, 0, H2p, 1};
+    if (d->gen1d)
+        gen::cols<double, -1>(b.X, b.X, ga1, ga1, 6 * P0, P1, P1, H2, d->g1, d->tw1d, st, all);
+    else
+        pick_cols<double, -1>(P1)(b.X, b.X, ga1, ga1, 6 * P0, P1, P1, H2, d->tw1d, st);
+    Geo ga0 = {(long)P0 * P1 * H2p, (long)H2p, (long)P1 * H2p, P1};
+    if (auto f0 = pick_cols<double, -1>(P0))
+        f0(b.X, b.X, ga0, ga0, 6 * P1, P0, P0, H2, d->tw0d, st);
+    else
+        gen::cols<double, -1>(b.X, b.X, ga0, ga0, 6 * P1, P0, P0, H2, d->g0, d->tw0d, st, all);
+    hipLaunchKernelGGL(k_kernel_extract, dim3(hs::grid1d(nk), 6), dim3(hs::kBlock), 0, st, b.X, k64, k32, P0, P1, H2,
+                       H2p, d->K[0], d->K[1], d->KP, 1.0 / (double)P, b.maxbits);
+}
+}  // namespace
+
+// kernel: 0 = Kernel_Arne at `accuracy`, 1 = Newell; pad: transform open axes
+// without a compiled family at the next compiled length
 static hs_demag* demag_create(const int N[3], const double cell[3], const int pbc[3], int accuracy, int kernel,
-                              CUstream stream) {
+                              CUstream stream, bool pad = true) {
     if (!N || !cell || N[0] < 1 || N[1] < 1 || N[2] < 1) {
         hs::set_error(HS_EINVAL, "hs_demag_create: bad mesh");
         return nullptr;
@@ -1072,22 +1166,27 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
         d->N[c] = N[c];
         d->pbc[c] = pbc ? pbc[c] : 0;
         d->cell[c] = cell[c];
-        d->P[c] = (N[c] > 1 && d->pbc[c] == 0) ? 2 * N[c] : N[c];
+        d->logic[c] = (N[c] > 1 && d->pbc[c] == 0) ? 2 * N[c] : N[c];
+        d->logicK[c] = d->logic[c] / 2 + 1;
     }
-    d->M = d->P[2] / 2;
-    d->H2 = d->M + 1;
-    d->H2p = (d->H2 + 15) / 16 * 16;
-    d->KP = (d->H2 + 31) / 32 * 32;
-    d->K[0] = d->P[0] / 2 + 1;
-    d->K[1] = d->P[1] / 2 + 1;
-    d->K[2] = d->H2;
     d->ncell = (long)N[0] * N[1] * N[2];
-    if (!sizes_ok(d)) {
+    if (!set_lengths(d, d->logic)) {
         hs::set_error(HS_ESIZE, "hs_demag_create: a padded length (or half the padded x length) exceeds 4095");
         delete d;
         return nullptr;
     }
+    d->noalloc = noalloc_bytes(d, 0) <= kScratchBytes;
+    if (pad) {
+        auto open = [&](int c) { return d->logic[c] > N[c]; };
+        const int P[3] = {
+            open(0) ? compiled_length(d->P[0], [](int L) { return z32_ok(L) && z64_ok(L); }) : d->P[0],
+            open(1) ? compiled_length(d->P[1], [](int L) { return cols32(L) && cols64(L); }) : d->P[1],
+            open(2) ? compiled_length(d->P[2], [](int L) { return rows32(L) && rows64(L); }) : d->P[2]};
+        set_lengths(d, P);
+        if (d->noalloc && noalloc_bytes(d, fused_fold<double>(d)) > kScratchBytes) set_lengths(d, d->logic);
+    }
     const int P0 = d->P[0], P1 = d->P[1], P2 = d->P[2], H2 = d->H2, H2p = d->H2p, M = d->M;
+    const bool padded = P0 != d->logic[0] || P1 != d->logic[1] || P2 != d->logic[2];
     const long nk = (long)d->K[0] * d->K[1] * d->K[2];
     // twiddles
     d->twMf = make_twiddles<float>(M);
@@ -1110,39 +1209,42 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     if (!d->fold32 && d->gen0) hipMalloc(&d->Xzf, sizeof(cpx<float>) * 3L * P0 * P1 * H2p);
     if (d->fold32) hipMalloc(&d->kt32, sizeof(float) * fused_table(d, d->fold32));
     // the FP64 table now where hs_demag_field_f64_noalloc takes the mesh (it cannot allocate), else on first use
-    const bool tab64 = d->fold64 && noalloc_bytes(d) <= kScratchBytes;
+    const bool tab64 = d->fold64 && d->noalloc;
     if (tab64) hipMalloc(&d->kt64, sizeof(double) * fused_table(d, d->fold64));
-    // ---- Kernel_Arne on the device (FP64)
+    // ---- Kernel_Arne on the device (FP64), at the logic size
+    const int *Lg = d->logic, *LK = d->logicK;
     int r1[3], r2[3];
     for (int c = 0; c < 3; c++) {
         if (d->pbc[c] == 0) {
-            r1[c] = -(d->P[c] - 1) / 2;
-            r2[c] = (d->P[c] - 1) / 2;
+            r1[c] = -(Lg[c] - 1) / 2;
+            r2[c] = (Lg[c] - 1) / 2;
         } else {
-            r1[c] = -(d->P[c] * d->pbc[c] - 1);
-            r2[c] = (d->P[c] * d->pbc[c] - 1);
+            r1[c] = -(Lg[c] * d->pbc[c] - 1);
+            r2[c] = (Lg[c] * d->pbc[c] - 1);
         }
     }
-    if (d->P[2] == 1 && d->pbc[2] == 0) r2[2] = 0;
-    const long noct = (long)(P0 / 2 + 1) * (P1 / 2 + 1) * (P2 / 2 + 1);
+    if (Lg[2] == 1 && d->pbc[2] == 0) r2[2] = 0;
+    const long noct = (long)LK[0] * LK[1] * LK[2];
     double* oct = nullptr;
     double* full = nullptr;
     cpx<double>* X = nullptr;
     unsigned long long* maxbits = nullptr;
-    const long P = (long)P0 * P1 * P2;
+    const long P = (long)P0 * P1 * P2;  // no length of `logic` is longer
     hipMalloc(&oct, sizeof(double) * 6 * noct);
     hipMalloc(&full, sizeof(double) * 6 * P);
     hipMalloc(&X, sizeof(cpx<double>) * 6L * P0 * P1 * H2p);
     hipMalloc(&maxbits, 2 * kExtractLanes * sizeof(unsigned long long));
-    if (!oct || !full || !X || !maxbits || !d->kern64 || !d->kern32 || !d->X1f ||
+    if (padded) hipMalloc(&d->kernL, sizeof(double) * 6 * noct);
+    if (!oct || !full || !X || !maxbits || !d->kern64 || !d->kern32 || !d->X1f || (padded && !d->kernL) ||
         (!d->fold32 && (!d->X2f || (d->gen0 && !d->Xzf))) || (d->fold32 && !d->kt32) || (tab64 && !d->kt64)) {
-        hs::set_error(HS_ENOMEM, "hs_demag_create: out of device memory");
         hipFree(oct); hipFree(full); hipFree(X); hipFree(maxbits);
         hs_demag_destroy(d);
+        (void)hipGetLastError();
+        if (padded) return demag_create(N, cell, pbc, accuracy, kernel, stream, false);
+        hs::set_error(HS_ENOMEM, "hs_demag_create: out of device memory");
         return nullptr;
     }
     hipMemsetAsync(oct, 0, sizeof(double) * 6 * noct, st);
-    hipMemsetAsync(maxbits, 0, 2 * kExtractLanes * sizeof(unsigned long long), st);
     if (kernel == 1) {
         // far-field switch of the Newell tensor: the FP64 second differences
         // and the cell-averaged dipole have equal error (a few 1e-6 relative)
@@ -1150,10 +1252,10 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
         const double hmax = std::max(cell[0], std::max(cell[1], cell[2]));
         const double hmin = std::min(cell[0], std::min(cell[1], cell[2]));
         const double rfar = 35.0 * pow(hmax, 0.6) * pow(hmin, 0.4);
-        hipLaunchKernelGGL(k_kernel_newell, dim3(hs::div_up(noct, 64)), dim3(64), 0, st, oct, P0, P1, P2, cell[0],
-                           cell[1], cell[2], r1[0], r1[1], r1[2], r2[0], r2[1], r2[2], rfar);
+        hipLaunchKernelGGL(k_kernel_newell, dim3(hs::div_up(noct, 64)), dim3(64), 0, st, oct, Lg[0], Lg[1], Lg[2],
+                           cell[0], cell[1], cell[2], r1[0], r1[1], r1[2], r2[0], r2[1], r2[2], rfar);
     } else {
-        const ArneP ap{P0,    P1,    P2,      r1[0],   r1[1],   r1[2], r2[0],
+        const ArneP ap{Lg[0], Lg[1], Lg[2],   r1[0],   r1[1],   r1[2], r2[0],
                        r2[1], r2[2], cell[0], cell[1], cell[2], (double)(accuracy > 0 ? accuracy : 6)};
         // the list of near cells (at most 3 noct entries) in the memory of `full`, which is filled after it is read
         unsigned* near = reinterpret_cast<unsigned*>(full) + 2;
@@ -1161,7 +1263,6 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
         hipLaunchKernelGGL(k_kernel_arne, dim3(hs::div_up(3 * noct, 64)), dim3(64), 0, st, oct, ap, near, near - 2);
         hipLaunchKernelGGL(k_kernel_arne_near, dim3(1024), dim3(kNearThreads), 0, st, oct, ap, near, near - 2);
     }
-    hipLaunchKernelGGL(k_kernel_fill, dim3(hs::grid1d(P), 6), dim3(hs::kBlock), 0, st, full, oct, P0, P1, P2);
     // IsZero (maxwell_convolution.go:227-232): components below 1e-12 of the
     // global max are dropped.  Done on the host from the octant.
     std::vector<double> hoct(6 * noct);
@@ -1171,30 +1272,26 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     for (int c = 0; c < 6; c++)
         for (long i = 0; i < noct; i++) cmax[c] = fmax(cmax[c], fabs(hoct[c * noct + i]));
     for (int c = 0; c < 6; c++) gmax = fmax(gmax, cmax[c]);
-    // ---- FP64 transform of the 6 real components: R2C rows, then axes 1 and 0 in place
-    // (lengths without a compiled family take the run-time-length passes)
-    const Live all{nullptr, 1};
-    if (d->genRd)
-        gen::r2c<double>(full, nullptr, 1, X, 6L * P0 * P1, P2, P2, H2p, d->gR, row_table<double>(d, d->twMd, d->twP2d),
-                         d->twP2d, st, all);
-    else
-        pick_r2c<double, double>(M)(full, nullptr, 1, X, 6L * P0 * P1, P2, H2p, d->twMd, d->twP2d, st);
-    Geo ga1 = {(long)P1 * H2p, 0, H2p, 1};
-    if (d->gen1d)
-        gen::cols<double, -1>(X, X, ga1, ga1, 6 * P0, P1, P1, H2, d->g1, d->tw1d, st, all);
-    else
-        pick_cols<double, -1>(P1)(X, X, ga1, ga1, 6 * P0, P1, P1, H2, d->tw1d, st);
-    Geo ga0 = {(long)P0 * P1 * H2p, (long)H2p, (long)P1 * H2p, P1};
-    if (auto f0 = pick_cols<double, -1>(P0))
-        f0(X, X, ga0, ga0, 6 * P1, P0, P0, H2, d->tw0d, st);
-    else
-        gen::cols<double, -1>(X, X, ga0, ga0, 6 * P1, P0, P0, H2, d->g0, d->tw0d, st, all);
-    hipLaunchKernelGGL(k_kernel_extract, dim3(hs::grid1d(nk), 6), dim3(hs::kBlock), 0, st, X, d->kern64, d->kern32,
-                       P0, P1, H2, H2p, d->K[0], d->K[1], d->KP, 1.0 / (double)P, maxbits);
+    const KernelBufs kb{oct, full, X, maxbits};
+    kernel_transform(d, kb, d->kern64, d->kern32, st);
+    if (padded) {
+        hs_demag l;  // the transform at the logic size, for hs_demag_kernel_f64 alone
+        std::copy(d->logic, d->logic + 3, l.logic);
+        std::copy(d->logicK, d->logicK + 3, l.logicK);
+        set_lengths(&l, d->logic);
+        l.twMd = make_twiddles<double>(l.M);
+        l.twP2d = make_twiddles<double>(l.P[2]);
+        l.tw1d = make_twiddles<double>(l.P[1]);
+        l.tw0d = make_twiddles<double>(l.P[0]);
+        kernel_transform(&l, kb, d->kernL, nullptr, st);
+        hipStreamSynchronize(st);
+        for (void* p : {l.twMd, l.twP2d, l.tw1d, l.tw0d}) hipFree(p);
+    }
     for (int c = 0; c < 6; c++) {
         if (gmax > 0 && cmax[c] / gmax < 1e-12) {
             hipMemsetAsync(d->kern64 + c * nk, 0, sizeof(double) * nk, st);
             hipMemsetAsync(d->kern32 + c * nk32, 0, sizeof(float) * nk32, st);
+            if (padded) hipMemsetAsync(d->kernL + c * noct, 0, sizeof(double) * noct, st);
         }
     }
     if (d->fold32) fill_table<float>(d, d->kt32, d->fold32, st);
@@ -1235,7 +1332,7 @@ extern "C" hs_demag* hs_demag_create_newell(const int N[3], const double cell[3]
 
 extern "C" void hs_demag_destroy(hs_demag* d) {
     if (!d) return;
-    void* ps[] = {d->kt32,   d->kt64,   d->kern64, d->kern32, d->X1f, d->X2f, d->X1d, d->X2d, d->twMf, d->twP2f,
+    void* ps[] = {d->kernL,  d->kt32,   d->kt64,   d->kern64, d->kern32, d->X1f, d->X2f, d->X1d, d->X2d, d->twMf, d->twP2f,
                   d->tw1f,   d->tw0f,   d->twMd, d->twP2d, d->tw1d, d->tw0d, d->Xzf, d->Xzd};
     for (void* p : ps)
         if (p) hipFree(p);
@@ -1245,16 +1342,16 @@ extern "C" void hs_demag_destroy(hs_demag* d) {
 extern "C" int hs_demag_sizes(const hs_demag* d, int P[3], int K[3]) {
     if (!d) return HS_EINVAL;
     for (int c = 0; c < 3; c++) {
-        if (P) P[c] = d->P[c];
-        if (K) K[c] = d->K[c];
+        if (P) P[c] = d->logic[c];
+        if (K) K[c] = d->logicK[c];
     }
     return 0;
 }
 
 extern "C" int hs_demag_kernel_f64(const hs_demag* d, double* host_out) {
     if (!d || !host_out) return HS_EINVAL;
-    long nk = (long)d->K[0] * d->K[1] * d->K[2];
-    hipError_t e = hipMemcpy(host_out, d->kern64, sizeof(double) * 6 * nk, hipMemcpyDeviceToHost);
+    long nk = (long)d->logicK[0] * d->logicK[1] * d->logicK[2];
+    hipError_t e = hipMemcpy(host_out, d->kernL ? d->kernL : d->kern64, sizeof(double) * 6 * nk, hipMemcpyDeviceToHost);
     return e == hipSuccess ? 0 : (int)e;
 }
 
@@ -1359,8 +1456,7 @@ extern "C" int hs_demag_field_f64_noalloc(hs_demag* d, const double* m, const do
         hs::set_error(HS_EINVAL, "hs_demag_field_f64_noalloc");
         return HS_EINVAL;
     }
-    const size_t need = noalloc_bytes(d);
-    if (need > kScratchBytes) {
+    if (!d->noalloc) {
         hs::set_error(HS_ESIZE, "hs_demag_field_f64_noalloc: the mesh's FP64 spectra exceed the 64 MiB static "
                                 "scratch; use hs_demag_field_f64");
         return HS_ESIZE;
@@ -1417,6 +1513,7 @@ long hs_demag_footprint(const hs_demag* d) {
     long b = 6 * nk * (sizeof(double) + sizeof(float));
     b += (long)sizeof(cpx<float>) * (fused_spectrum(d, d->fold32) + (d->X2f ? 3L * d->N[0] * d->P[1] * d->H2p : 0)) *
          d->cap;
+    if (d->kernL) b += 6L * d->logicK[0] * d->logicK[1] * d->logicK[2] * (long)sizeof(double);
     if (d->kt32) b += fused_table(d, d->fold32) * (long)sizeof(float);
     if (d->kt64) b += fused_table(d, d->fold64) * (long)sizeof(double);
     b += 6L * d->K[0] * d->K[1] * (d->KP - d->H2) * (long)sizeof(float);

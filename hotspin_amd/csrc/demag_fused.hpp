@@ -59,7 +59,7 @@ template <typename T>
 struct Mid {
     cpx<T>* X;
     const T* kt;  // [column][d][KR][6]: -XX, YY, ZZ, YZ, kappa XZ, kappa XY
-    int N0, ncol, CB, nsolve, R;
+    int N0, N1, ncol, CB, nsolve, R;
     const cpx<T>* tw;  // w_P1^t, P1 = Q R
     const int* live;   // per-solve flags or null
 };
@@ -86,25 +86,126 @@ __device__ __forceinline__ double fmaT(double a, double b, double c) { return __
 // axis-0 items per thread: 3 IB values each, at most 24 in all
 constexpr int mid_itm(int IB) { return 8 / IB; }
 
+// Shape of a column's tile: compile-time here, at run time in k_fmid_any.
+template <int Q_, bool FOLD>
+struct Geom {
+    static constexpr int Q = Q_, A = split_even(Q_).A, B = split_even(Q_).B, BP = B + 1, PL = A * BP;
+    static constexpr int KR = table_rows(Q_, FOLD);
+};
+
 // The table entry (distance 0) of column tc's slot; sj = -1 for a mirrored row.
-template <typename T, int Q, bool FOLD>
-__device__ __forceinline__ const T* table_row(const Mid<T>& a, int tc, int slot, T& sj) {
-    constexpr int A = split_even(Q).A, B = split_even(Q).B;
+template <typename T, bool FOLD, typename G>
+__device__ __forceinline__ const T* table_row(const Mid<T>& a, const G& g, int tc, int slot, int k1, int k2, T& sj) {
     bool mir;
     int row;
     if constexpr (FOLD) {  // column k R + s: frequencies R q + s, mirrored at R (Q - 1 - q) + R - s
         const int k = tc / a.R, s = tc % a.R;
         mir = 2 * s > a.R;
-        row = mir ? Q - 1 - slot : slot;
+        row = mir ? g.Q - 1 - slot : slot;
         tc = k * (a.R / 2 + 1) + (mir ? a.R - s : s);
     } else {
-        const int k1 = slot / B, k2 = slot % B;
-        mir = k1 > A / 2;
-        row = mir ? (A - k1) * B + (B - 1 - k2) : slot;
+        mir = k1 > g.A / 2;
+        row = mir ? (g.A - k1) * g.B + (g.B - 1 - k2) : slot;
     }
     sj = mir ? T(-1) : T(1);
-    constexpr int KR = table_rows(Q, FOLD);
-    return a.kt + ((long)tc * a.N0 * KR + row) * 6;
+    return a.kt + ((long)tc * a.N0 * g.KR + row) * 6;
+}
+
+// Axis 0: y(i) = sum_i' K~(i - i') x(i') in place; one item = IB planes of the
+// three components at one slot (MULTI: N0 > IB).
+template <typename T, int IB, bool MULTI, bool FOLD, typename G>
+__device__ __forceinline__ void axis0(const Mid<T>& a, const G& g, cpx<T>* lds, int col0, int ncb) {
+    constexpr int ITM = mid_itm(IB);
+    const int tid = threadIdx.x, NT = blockDim.x, N0 = a.N0, PC = 3 * N0, PL = g.PL;
+    const int NIB = MULTI ? (N0 + IB - 1) / IB : 1, items = ncb * NIB * g.Q;
+    cpx<T> y[ITM][3][IB];
+#pragma unroll
+    for (int it = 0; it < ITM; it++) {
+        const int e = tid + it * NT;
+#pragma unroll
+        for (int q = 0; q < IB; q++) y[it][0][q] = y[it][1][q] = y[it][2][q] = {T(0), T(0)};
+        if (e < items) {
+            const int r = e / g.Q, slot = e - r * g.Q, ib = MULTI ? r % NIB : 0, col = MULTI ? r / NIB : r;
+            const int k1 = slot / g.B, k2 = slot - k1 * g.B;
+            T sj;
+            const T* kb = table_row<T, FOLD>(a, g, col0 + col, slot, k1, k2, sj);
+            const cpx<T>* xs = lds + col * PC * PL + k1 * g.BP + k2;
+            // K~ at plane distance ad >= 0 for this row
+            auto coef = [&](int ad, Coef<T>& w) {
+                w.load(kb + (long)ad * (6 * g.KR));
+                w.xy *= sj;
+                w.yz *= sj;
+            };
+            auto acc = [&](const Coef<T>& w, bool neg, const cpx<T>& x0, const cpx<T>& x1, const cpx<T>& x2,
+                           int q) {
+                const T xy = neg ? -w.xy : w.xy, xz = neg ? -w.xz : w.xz;
+                cpx<T>&a0 = y[it][0][q], &a1 = y[it][1][q], &a2 = y[it][2][q];
+                // chained into the accumulators: three fma each (a sum of products
+                // added afterwards takes a fourth instruction)
+                a0.x = fmaT(xz, x2.x, fmaT(xy, x1.x, fmaT(w.xx, x0.x, a0.x)));
+                a0.y = fmaT(xz, x2.y, fmaT(xy, x1.y, fmaT(w.xx, x0.y, a0.y)));
+                a1.x = fmaT(w.yz, x2.x, fmaT(w.yy, x1.x, fmaT(xy, x0.x, a1.x)));
+                a1.y = fmaT(w.yz, x2.y, fmaT(w.yy, x1.y, fmaT(xy, x0.y, a1.y)));
+                a2.x = fmaT(w.zz, x2.x, fmaT(w.yz, x1.x, fmaT(xz, x0.x, a2.x)));
+                a2.y = fmaT(w.zz, x2.y, fmaT(w.yz, x1.y, fmaT(xz, x0.y, a2.y)));
+            };
+            if constexpr (!MULTI) {  // N0 == IB: every distance in registers, signs known at compile time
+                Coef<T> w[IB];
+#pragma unroll
+                for (int d = 0; d < IB; d++) coef(d, w[d]);
+#pragma unroll
+                for (int i = 0; i < IB; i++) {
+                    const cpx<T> x0 = xs[i * PL], x1 = xs[(IB + i) * PL], x2 = xs[(2 * IB + i) * PL];
+#pragma unroll
+                    for (int q = 0; q < IB; q++) acc(w[q < i ? i - q : q - i], q < i, x0, x1, x2, q);
+                }
+            } else {
+                // window w[n] = K~(i0 - ip - 3 + n), n < IB + 3, over the input planes ip .. ip + 3
+                // (the sign of the odd components taken when a distance enters)
+                const int i0 = ib * IB;
+                Coef<T> w[IB + 3];
+                auto enter = [&](int d, Coef<T>& o) {
+                    coef(min(d < 0 ? -d : d, N0 - 1), o);
+                    if (d < 0) {
+                        o.xy = -o.xy;
+                        o.xz = -o.xz;
+                    }
+                };
+#pragma unroll
+                for (int n = 4; n < IB + 3; n++) enter(i0 - 3 + n, w[n - 4]);
+                for (int ip = 0; ip < N0; ip += 4) {
+#pragma unroll
+                    for (int n = IB + 2; n >= 4; n--) w[n] = w[n - 4];
+#pragma unroll
+                    for (int n = 0; n < 4; n++) enter(i0 - ip - 3 + n, w[n]);
+#pragma unroll
+                    for (int r2 = 0; r2 < 4; r2++) {
+                        const int i = min(ip + r2, N0 - 1);
+                        cpx<T> x0 = xs[i * PL], x1 = xs[(N0 + i) * PL], x2 = xs[(2 * N0 + i) * PL];
+                        if (ip + r2 >= N0) x0 = x1 = x2 = {T(0), T(0)};
+#pragma unroll
+                        for (int q = 0; q < IB; q++) acc(w[q - r2 + 3], false, x0, x1, x2, q);
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < ITM; it++) {
+        const int e = tid + it * NT;
+        if (e < items) {
+            const int r = e / g.Q, slot = e - r * g.Q, ib = MULTI ? r % NIB : 0, col = MULTI ? r / NIB : r;
+            const int k1 = slot / g.B, k2 = slot - k1 * g.B;
+            cpx<T>* o = lds + (col * PC + ib * IB) * PL + k1 * g.BP + k2;
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+#pragma unroll
+                for (int q = 0; q < IB; q++)
+                    if (!MULTI || ib * IB + q < N0) o[(c * N0 + q) * PL] = y[it][c][q];
+        }
+    }
+    __syncthreads();
 }
 
 // One block: CB columns of one solve, 3 N0 pencils of Q points each, held in
@@ -114,9 +215,9 @@ __device__ __forceinline__ const T* table_row(const Mid<T>& a, int tc, int slot,
 // Axis 0 in items of IB planes (MULTI: N0 > IB).
 template <typename T, int Q, int IB, bool MULTI, bool FOLD>
 __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
-    constexpr int A = split_even(Q).A, B = split_even(Q).B, BP = B + 1, PL = A * BP, AIN = FOLD ? A : A / 2;
-    constexpr int UA = (kEpt + A - 1) / A, UB = (kEpt + B - 1) / B, ITM = mid_itm(IB);
-    constexpr int KR = table_rows(Q, FOLD), N1 = FOLD ? Q : Q / 2;
+    using G = Geom<Q, FOLD>;
+    constexpr int A = G::A, B = G::B, BP = G::BP, PL = G::PL, AIN = FOLD ? A : A / 2;
+    constexpr int UA = (kEpt + A - 1) / A, UB = (kEpt + B - 1) / B;
     static_assert(A * B == Q && A % 2 == 0, "two-level split");
     extern __shared__ __align__(16) unsigned char mid_smem[];
     cpx<T>* tws = reinterpret_cast<cpx<T>*>(mid_smem);
@@ -127,6 +228,8 @@ __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
     if (a.live && !a.live[sol]) return;
     const int N0 = a.N0, col0 = tile * a.CB, ncb = min(a.CB, a.ncol - col0);
     const int PC = 3 * N0, NP = PC * ncb;
+    const int N1 = FOLD ? Q : a.N1;           // rows a column has in X
+    const bool half = FOLD || 2 * N1 == Q;    // uniform: they are those of the A-point inputs n1 < AIN
     cpx<T>* X = a.X + ((long)sol * a.ncol + col0) * (long)(PC * N1);
     {  // phase 1: A-point DFTs over n1 of the rows j = B n1 + n2 < N1 (the upper half is padding unless folded)
         cpx<T> v[UA][A];
@@ -134,9 +237,17 @@ __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
         for (int u = 0; u < UA; u++) {
             const int e = tid + u * NT;
             const int p = e / B, n2 = e % B;
-            const cpx<T>* xp = X + (e < NP * B ? p * N1 + n2 : 0);
+            const cpx<T>* xp = X + (e < NP * B ? p * N1 : 0) + n2;
+            if (half) {
 #pragma unroll
-            for (int n1 = 0; n1 < AIN; n1++) v[u][n1] = xp[B * n1];
+                for (int n1 = 0; n1 < AIN; n1++) v[u][n1] = xp[B * n1];
+            } else {
+#pragma unroll
+                for (int n1 = 0; n1 < AIN; n1++) v[u][n1] = xp[B * n1 + n2 < N1 ? B * n1 : -n2];
+#pragma unroll
+                for (int n1 = 0; n1 < AIN; n1++)
+                    if (B * n1 + n2 >= N1) v[u][n1] = {T(0), T(0)};
+            }
         }
         for (int t = tid; t < Q; t += NT) tws[t] = a.tw[FOLD ? t * a.R : t];
         __syncthreads();
@@ -175,95 +286,7 @@ __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
         }
     }
     __syncthreads();
-    {  // axis 0: y(i) = sum_i' K~(i - i') x(i'); one item = IB planes of the three components at one slot
-        const int NIB = MULTI ? (N0 + IB - 1) / IB : 1, items = ncb * NIB * Q;
-        cpx<T> y[ITM][3][IB];
-#pragma unroll
-        for (int it = 0; it < ITM; it++) {
-            const int e = tid + it * NT;
-#pragma unroll
-            for (int q = 0; q < IB; q++) y[it][0][q] = y[it][1][q] = y[it][2][q] = {T(0), T(0)};
-            if (e < items) {
-                const int slot = e % Q, r = e / Q, ib = MULTI ? r % NIB : 0, col = MULTI ? r / NIB : r;
-                T sj;
-                const T* kb = table_row<T, Q, FOLD>(a, col0 + col, slot, sj);
-                const cpx<T>* xs = lds + col * PC * PL + slot / B * BP + slot % B;
-                // K~ at plane distance ad >= 0 for this row
-                auto coef = [&](int ad, Coef<T>& w) {
-                    w.load(kb + (long)ad * (6 * KR));
-                    w.xy *= sj;
-                    w.yz *= sj;
-                };
-                auto acc = [&](const Coef<T>& w, bool neg, const cpx<T>& x0, const cpx<T>& x1, const cpx<T>& x2,
-                               int q) {
-                    const T xy = neg ? -w.xy : w.xy, xz = neg ? -w.xz : w.xz;
-                    cpx<T>&a0 = y[it][0][q], &a1 = y[it][1][q], &a2 = y[it][2][q];
-                    // chained into the accumulators: three fma each (a sum of products
-                    // added afterwards takes a fourth instruction)
-                    a0.x = fmaT(xz, x2.x, fmaT(xy, x1.x, fmaT(w.xx, x0.x, a0.x)));
-                    a0.y = fmaT(xz, x2.y, fmaT(xy, x1.y, fmaT(w.xx, x0.y, a0.y)));
-                    a1.x = fmaT(w.yz, x2.x, fmaT(w.yy, x1.x, fmaT(xy, x0.x, a1.x)));
-                    a1.y = fmaT(w.yz, x2.y, fmaT(w.yy, x1.y, fmaT(xy, x0.y, a1.y)));
-                    a2.x = fmaT(w.zz, x2.x, fmaT(w.yz, x1.x, fmaT(xz, x0.x, a2.x)));
-                    a2.y = fmaT(w.zz, x2.y, fmaT(w.yz, x1.y, fmaT(xz, x0.y, a2.y)));
-                };
-                if constexpr (!MULTI) {  // N0 == IB: every distance in registers, signs known at compile time
-                    Coef<T> w[IB];
-#pragma unroll
-                    for (int d = 0; d < IB; d++) coef(d, w[d]);
-#pragma unroll
-                    for (int i = 0; i < IB; i++) {
-                        const cpx<T> x0 = xs[i * PL], x1 = xs[(IB + i) * PL], x2 = xs[(2 * IB + i) * PL];
-#pragma unroll
-                        for (int q = 0; q < IB; q++) acc(w[q < i ? i - q : q - i], q < i, x0, x1, x2, q);
-                    }
-                } else {
-                    // window w[n] = K~(i0 - ip - 3 + n), n < IB + 3, over the input planes ip .. ip + 3
-                    // (the sign of the odd components taken when a distance enters)
-                    const int i0 = ib * IB;
-                    Coef<T> w[IB + 3];
-                    auto enter = [&](int d, Coef<T>& o) {
-                        coef(min(d < 0 ? -d : d, N0 - 1), o);
-                        if (d < 0) {
-                            o.xy = -o.xy;
-                            o.xz = -o.xz;
-                        }
-                    };
-#pragma unroll
-                    for (int n = 4; n < IB + 3; n++) enter(i0 - 3 + n, w[n - 4]);
-                    for (int ip = 0; ip < N0; ip += 4) {
-#pragma unroll
-                        for (int n = IB + 2; n >= 4; n--) w[n] = w[n - 4];
-#pragma unroll
-                        for (int n = 0; n < 4; n++) enter(i0 - ip - 3 + n, w[n]);
-#pragma unroll
-                        for (int r2 = 0; r2 < 4; r2++) {
-                            const int i = min(ip + r2, N0 - 1);
-                            cpx<T> x0 = xs[i * PL], x1 = xs[(N0 + i) * PL], x2 = xs[(2 * N0 + i) * PL];
-                            if (ip + r2 >= N0) x0 = x1 = x2 = {T(0), T(0)};
-#pragma unroll
-                            for (int q = 0; q < IB; q++) acc(w[q - r2 + 3], false, x0, x1, x2, q);
-                        }
-                    }
-                }
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < ITM; it++) {
-            const int e = tid + it * NT;
-            if (e < items) {
-                const int slot = e % Q, r = e / Q, ib = MULTI ? r % NIB : 0, col = MULTI ? r / NIB : r;
-                cpx<T>* o = lds + (col * PC + ib * IB) * PL + (slot / B) * BP + slot % B;
-#pragma unroll
-                for (int c = 0; c < 3; c++)
-#pragma unroll
-                    for (int q = 0; q < IB; q++)
-                        if (!MULTI || ib * IB + q < N0) o[(c * N0 + q) * PL] = y[it][c][q];
-            }
-        }
-    }
-    __syncthreads();
+    axis0<T, IB, MULTI, FOLD>(a, G{}, lds, col0, ncb);
     {  // inverse phase 2: B-point DFTs over k2 in place, then the twiddle
 #pragma unroll
         for (int u = 0; u < UB; u++) {
@@ -298,10 +321,15 @@ __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
                 cpx<T>* xp = X + p * N1 + n2;
                 if (p % PC < N0) {  // y_x = i v
 #pragma unroll
-                    for (int n1 = 0; n1 < AIN; n1++) xp[B * n1] = {-v[n1].y, v[n1].x};
-                } else {
+                    for (int n1 = 0; n1 < AIN; n1++) v[n1] = {-v[n1].y, v[n1].x};
+                }
+                if (half) {
 #pragma unroll
                     for (int n1 = 0; n1 < AIN; n1++) xp[B * n1] = v[n1];
+                } else {
+#pragma unroll
+                    for (int n1 = 0; n1 < AIN; n1++)
+                        if (B * n1 + n2 < N1) xp[B * n1] = v[n1];
                 }
             }
         }
@@ -352,15 +380,15 @@ struct RowMap {
             pen = b / ng - sol * g.PC;
         }
     }
-    // row of slot p (p = m WA + a), and whether it exists
+    // row of slot p (p = m WA + a), and whether it exists (a padded axis 1 has N1 < Q R / 2 rows)
     __device__ __forceinline__ long row(const RowP& g, int p, bool& in) const {
         if constexpr (R == 1) {
             in = row0 + p < (long)g.rows * g.nsolve;
             return in ? row0 + p : row0;
         } else {
-            const int j = j0 + p % WA;
-            in = j < g.Q;
-            return row0 + (in ? j : 0) + (long)g.Q * (p / WA);
+            const int a = j0 + p % WA, j = a + g.Q * (p / WA);
+            in = a < g.Q && j < g.N1;
+            return row0 + (in ? j : 0);
         }
     }
     __device__ __forceinline__ bool dead(const RowP& g, const Live& lv) const {

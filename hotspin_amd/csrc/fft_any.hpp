@@ -1,9 +1,10 @@
 // fft_any.hpp -- demag FFT passes for padded lengths chosen at run time.
 //
 // The compiled families (fft.hpp, fft2.hpp) cover lengths 2^k, 3*2^k and
-// 5*2^k with compile-time codelets.  Every other length -- 7 or 9 in a
-// factor, 100 = 2^2 5^2, an odd x length of a periodic axis, a one-cell
-// axis -- goes through these kernels, which take the length and its radix
+// 5*2^k with compile-time codelets, and an open axis is padded to one of them.
+// Every other length -- a periodic axis with 7 or 9 in a factor, 100 = 2^2 5^2,
+// an odd x length, a one-cell axis, an open axis beyond the longest compiled
+// length -- goes through these kernels, which take the length and its radix
 // sequence as arguments, like cuFFT's plans in the reference
 // (src/hotspin-core/gpu/fftplanX.go:55-60 plans D2Z/Z2D of any size).
 //

@@ -47,10 +47,12 @@ typedef struct hs_demag hs_demag;
  * 1/(P0 P1 P2) and stored in FP64 and FP32.  accuracy = 6 in the reference
  * (maxwell_convolution.go:96).  Blocks until the kernel is ready.
  * Any padded lengths up to 4095 (half the padded x length when it is even):
- * 2^k, 3*2^k and 5*2^k run compiled, tuned passes; other lengths (factors 7,
- * 9, 25, larger primes, odd periodic x lengths, one-cell axes) run passes
- * that take the length at run time, as cuFFT plans do in the reference
- * (gpu/fftplanX.go:55-60).  Returns NULL on error (hs_last_error). */
+ * 2^k, 3*2^k and 5*2^k run compiled passes, tuned by timing where the mesh is
+ * too large for the three-kernel convolution; an open axis of any other length
+ * is padded to the next of them.  Lengths that cannot be (periodic axes with
+ * factors 7, 9, 25 or larger primes, odd periodic x lengths, one-cell axes)
+ * run passes that take the length at run time, as cuFFT plans do in the
+ * reference (gpu/fftplanX.go:55-60).  Returns NULL on error (hs_last_error). */
 HS_API hs_demag* hs_demag_create(const int N[3], const double cell[3], const int pbc[3], int accuracy,
                                  CUstream stream);
 /* The same plan with the Newell demag tensor instead of Kernel_Arne: no
@@ -64,7 +66,8 @@ HS_API hs_demag* hs_demag_create(const int N[3], const double cell[3], const int
  * and passes as hs_demag_create. */
 HS_API hs_demag* hs_demag_create_newell(const int N[3], const double cell[3], const int pbc[3], CUstream stream);
 HS_API void hs_demag_destroy(hs_demag* d);
-/* P = logic (padded) size, K = kernel octant size (P0/2+1, P1/2+1, P2/2+1) */
+/* P = logic size (2 N on open axes, whatever length they are transformed at),
+ * K = its kernel octant (P0/2+1, P1/2+1, P2/2+1) */
 HS_API int hs_demag_sizes(const hs_demag* d, int P[3], int K[3]);
 /* Copy the FP64 kernel octants (6 planes XX,YY,ZZ,YZ,XZ,XY of K0*K1*K2) to host. */
 HS_API int hs_demag_kernel_f64(const hs_demag* d, double* host_out);
@@ -72,7 +75,8 @@ HS_API int hs_demag_kernel_f64(const hs_demag* d, double* host_out);
  * above 1e-12, maxwell_convolution.go:383-385) */
 HS_API double hs_demag_max_imag_ratio(const hs_demag* d);
 /* FP32 tile shapes the plan's autotuner picked: (W, NT) of the row passes
- * (F1/I1), the column passes (F2/I2) and the axis-0 product pass (F3K) */
+ * (F1/I1), the column passes (F2/I2) and the axis-0 product pass (F3K) of the
+ * five-pass form; the first variant's, untimed, in a three-kernel plan */
 HS_API int hs_demag_tiles(const hs_demag* d, int* out6);
 /* Number of registered FP32 variants of the row, column and axis-0 passes
  * for this plan's lengths (the environment variable HS_DEMAG_FORCE="r,c,z"
@@ -80,7 +84,9 @@ HS_API int hs_demag_tiles(const hs_demag* d, int* out6);
  * variants of a pass round differently (FP32, operation order); the timed
  * choice is kept per mesh shape for the process, and HS_TUNE_FILE=<path>
  * persists it across processes (read before timing, appended after), so
- * runs that share the file give the same bits. */
+ * runs that share the file give the same bits.  Three-kernel plans time
+ * nothing and always give the same bits; HS_DEMAG_FORCE keeps a plan's FP32
+ * field in the five passes. */
 HS_API int hs_demag_variant_count(const hs_demag* d, int* out3);
 /* B = mu0 * msat0T0Mul * (K conv (m .* msat0T0)), maxwell_convolution.go:103-131.
  * m, B: 3 device planes of N cells (m and B may not alias); msat0T0: device

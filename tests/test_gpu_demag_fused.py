@@ -71,3 +71,35 @@ def test_periodic_x_and_the_other_axes(N):
         d.field_f32(P(dm), None, 8e5, P(B))
         assert relerr(host(B), want) <= 2e-6
         d.close()
+
+
+# open axes whose 2 N has no compiled transform run at the next compiled length: one
+# ragged axis at a time, all three, odd x lengths, a folded axis 1 with rows missing
+# in its upper half (300 -> 640 points, FP32 folded 8 ways), more than 32 planes
+# (the five passes), one plane, and ragged axes next to periodic ones
+RAGGED = [((2, 8, 9), 0), ((2, 7, 16), 0), ((7, 8, 16), 0), ((7, 75, 100), 0), ((6, 45, 150), 0), ((1, 11, 13), 0),
+          ((16, 300, 18), 0), ((3, 23, 31), 0), ((8, 113, 37), 0), ((35, 9, 14), 0), ((49, 27, 22), 0),
+          ((3, 9, 26), (0, 0, 1)), ((3, 14, 18), (0, 1, 0)), ((7, 16, 18), (1, 0, 0)), ((5, 1, 22), 0), ((5, 22, 1), 0)]
+
+
+@pytest.mark.parametrize("N,pbc", RAGGED)
+def test_ragged_lengths(N, pbc):
+    cell, pbc = (2e-9, 3e-9, 2.5e-9), pbc or (0, 0, 0)
+    rng = np.random.default_rng(sum(N))
+    n = N[0] * N[1] * N[2]
+    m, msk = rng.standard_normal((3, n)), rng.random(n)
+    d, o = Demag(N, cell, pbc), po.Demag(N, cell, pbc)
+    assert d.P == tuple(2 * a if a > 1 and not p else a for a, p in zip(N, pbc))  # the logic size is reported
+    assert relerr(d.kernel(), o.kernel()) <= 1e-12
+    for w in (None, msk):
+        want = o.B(m, w, 8e5).reshape(3, n)
+        dm, dw = dev(m), None if w is None else dev(w)
+        for field in (d.field_f64, d.field_f64_noalloc):
+            B = empty((3, n))
+            field(P(dm), P(dw), 8e5, P(B))
+            assert relerr(host(B), want) <= 1e-12
+        dm, dw = dev(m, np.float32), None if w is None else dev(w, np.float32)
+        B = empty((3, n), torch.float32)
+        d.field_f32(P(dm), P(dw), 8e5, P(B))
+        assert relerr(host(B), want) <= 2e-6
+    d.close()
