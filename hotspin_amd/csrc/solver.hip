@@ -18,10 +18,12 @@
 #include <algorithm>
 #include <array>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <limits>
 #include <vector>
 
+#include "hostcopy.hpp"
 #include "hs_common.hpp"
 #include "philox.hpp"
 #include "xcd.hpp"
@@ -1566,6 +1568,7 @@ __global__ void k_gather_tm(const Clock* clk, const double* te1, const double* t
 
 struct hs_solver {
     hs_llb_params p;
+    std::shared_ptr<HostStage> host = HostStage::get();  // for states handed to the caller
     hipStream_t st;
     bool own_stream = false;
     long N;       // cells per solve
@@ -2415,6 +2418,18 @@ extern "C" int hs_solver_stage_variant(hs_solver* s) { return s ? s->stage_kind 
 extern "C" int hs_solver_stage_lean(hs_solver* s) { return s ? (int)(!s->tm && stage_lean(s, StageIO{})) : -1; }
 extern "C" int hs_solver_nsolve(hs_solver* s) { return s ? s->nsolve : -1; }
 
+// bytes of a device array of the solver to the caller's memory
+static void copy_out(hs_solver* s, void* host, const void* dev, size_t bytes, const char* who) {
+    hipError_t e;
+    if (s->host) {
+        e = s->host->out(host, dev, bytes, s->st);
+    } else {
+        e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s->st);
+        if (e == hipSuccess) e = hipStreamSynchronize(s->st);
+    }
+    if (e != hipSuccess) hs::set_error((int)e, who);
+}
+
 static bool whole_batch_ok(hs_solver* s, const char* who) {
     if (s->slot_mode) hs::set_error(HS_EINVAL, who);
     return !s->slot_mode;
@@ -2435,8 +2450,7 @@ extern "C" int hs_solver_set_m(hs_solver* s, const double* m) {
 extern "C" int hs_solver_get_m(hs_solver* s, double* m) {
     if (!s || !m) return HS_EINVAL;
     if (!whole_batch_ok(s, "hs_solver_get_m: handle is in slot mode")) return HS_EINVAL;
-    hipMemcpyAsync(m, s->y0, sizeof(double) * 3 * s->N * s->nsolve, hipMemcpyDeviceToHost, s->st);
-    hipStreamSynchronize(s->st);
+    copy_out(s, m, s->y0, sizeof(double) * 3 * s->N * s->nsolve, "hs_solver_get_m");
     HS_LAUNCH_CHECK("hs_solver_get_m");
     return hs_last_error();
 }
@@ -3266,9 +3280,7 @@ extern "C" int hs_slot_get_m(hs_solver* s, int slot, double* m) {
     hipStreamSynchronize(s->st);  // slot_host is then the device's current record
     const Clock c = s->slot_host[slot];
     const int set = c.state == HS_SLOT_RUNNING ? (int)(s->slot_iter & 1) : (int)c.home;
-    hipMemcpyAsync(m, slot_set(s, set).y + (long)slot * 3 * s->N, sizeof(double) * 3 * s->N, hipMemcpyDeviceToHost,
-                   s->st);
-    hipStreamSynchronize(s->st);
+    copy_out(s, m, slot_set(s, set).y + (long)slot * 3 * s->N, sizeof(double) * 3 * s->N, "hs_slot_get_m");
     HS_LAUNCH_CHECK("hs_slot_get_m");
     return hs_last_error();
 }
@@ -3455,9 +3467,8 @@ extern "C" int hs_solver_get_T(hs_solver* s, double* Te, double* Tp) {
         hs::set_error(HS_EINVAL, "hs_solver_get_T: not a two-temperature solver");
         return HS_EINVAL;
     }
-    if (Te) hipMemcpyAsync(Te, s->Te[0], sizeof(double) * s->N, hipMemcpyDeviceToHost, s->st);
-    if (Tp) hipMemcpyAsync(Tp, s->Tp[0], sizeof(double) * s->N, hipMemcpyDeviceToHost, s->st);
-    hipStreamSynchronize(s->st);
+    if (Te) copy_out(s, Te, s->Te[0], sizeof(double) * s->N, "hs_solver_get_T");
+    if (Tp) copy_out(s, Tp, s->Tp[0], sizeof(double) * s->N, "hs_solver_get_T");
     HS_LAUNCH_CHECK("hs_solver_get_T");
     return hs_last_error();
 }

@@ -1,0 +1,54 @@
+"""get_m returns the device state byte for byte around the size from which it
+is staged through pinned chunks (8 MB; chunks of 2 MB): below, at and just
+above it, with a partial last chunk, with more chunks than workers, and from
+two solvers in two threads at once (the second finds the buffers taken)."""
+import threading
+
+import numpy as np
+import pytest
+
+from hotspin_amd.api import Solver
+from tests.gpu_util import require_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _gpu():
+    require_gpu()
+
+
+def _solver(rows):
+    """A mesh of `rows` rows of 1024 cells: 24 KB of state each."""
+    n = 1024 * rows
+    s = Solver((1, rows, 1024), (2e-9,) * 3, demag=0, exchange=0, longfield=0)
+    m = np.random.default_rng(n).standard_normal((3, n))
+    s.set_m(m)
+    return s, m
+
+
+@pytest.mark.parametrize("rows", [1, 341, 342, 427, 1580])  # 341 rows: 8 MB less 8 KB
+def test_state_comes_back_unchanged(rows):
+    s, m = _solver(rows)
+    for _ in range(2):
+        assert np.array_equal(s.get_m(), m)
+    s.close()
+
+
+def test_two_solvers_in_two_threads():
+    pair = [_solver(850), _solver(1100)]
+    bad = []
+
+    def work(s, m):
+        for _ in range(4):
+            if not np.array_equal(s.get_m(), m):
+                bad.append(m.size)
+
+    th = [threading.Thread(target=work, args=p) for p in pair]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad
+    for s, _ in pair:
+        s.close()
