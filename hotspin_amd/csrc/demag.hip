@@ -485,37 +485,87 @@ using r2c_fn = void (*)(const void*, const void*, long, cpx<T>*, long, int, int,
 
 namespace {
 
+// FP64 kernel of a compiled length: the two-level register transforms of
+// fft2.hpp where they are the faster, the Stockham kernels of
+// demag_kernels.hpp elsewhere.  Times of one pass, Stockham / two-level:
+// - rows (33 MB): R2C 14.8 / 9.9 us at M = 64, 19.1 / 11.4 at 256, 16.2 / 13.3
+//   at 512; C2R 12.7 / 8.0, 17.0 / 8.8, 15.7 / 9.4; M = 1024 15.0 / 25.5.
+//   Eight rows a block (16 where eight give less than a wave, four from 384
+//   points on: R2C at 512 with eight 13.1, C2R 13.7).
+// - columns (107 MB out and in): 55 / 54 us at 32 points, 65 / 57 at 128,
+//   102 / 66 at 320, but 86 / 96 at 512 and within 5 % at 768 and 1024.
+// - axis 0 with the product (1.8 MB a plane): one lane a pencil up to 8
+//   points (12.0 / 5.7 us at 8), two up to 40 (39 / 16 at 32), four up to 128
+//   (86 / 32 at 64, 163 / 100 at 128): 565 / 190 us at 512x512x16, where the
+//   Stockham kernel took half the time of the field.
+template <int M>
+constexpr int rows2_w64() { return M >= 384 ? 4 : (8 * split2(M).B >= 64 ? 8 : 16); }
+template <typename T, int M>
+constexpr bool rows_two_level() { return sizeof(T) == 8 && M >= 16 && M <= 640 && two_level_ok(M); }
+template <typename T, int L>
+constexpr bool cols_two_level() { return sizeof(T) == 8 && L >= 32 && L <= 384 && two_level_ok(L); }
+
 template <typename T, typename TI, int M>
 void launch_r2c(const void* x, const void* msk, long mrows, cpx<T>* out, long nrows, int n2, int H2p,
                 const cpx<T>* twM, const cpx<T>* twP, hipStream_t st) {
-    constexpr int W = row_w<M>();
-    unsigned g = (unsigned)((nrows + W - 1) / W);
-    hipLaunchKernelGGL((k_r2c_rows<T, TI, M>), dim3(g), dim3(row_nt<M>()), 0, st, (const TI*)x, (const TI*)msk,
-                       mrows, out, nrows, n2, H2p, twM, twP, Live{nullptr, 1});
+    if constexpr (rows_two_level<T, M>()) {
+        constexpr int W = rows2_w64<M>();
+        hipLaunchKernelGGL((k_r2c_rows2<T, M, W>), dim3((unsigned)((nrows + W - 1) / W)), dim3(W * split2(M).B), 0, st,
+                           (const T*)x, (const T*)msk, mrows, out, nrows, n2, H2p, twM, twP, Live{nullptr, 1});
+    } else {
+        constexpr int W = row_w<M>();
+        unsigned g = (unsigned)((nrows + W - 1) / W);
+        hipLaunchKernelGGL((k_r2c_rows<T, TI, M>), dim3(g), dim3(row_nt<M>()), 0, st, (const TI*)x, (const TI*)msk,
+                           mrows, out, nrows, n2, H2p, twM, twP, Live{nullptr, 1});
+    }
 }
 template <typename T, typename TO, int M>
 void launch_c2r(const cpx<T>* in, void* x, long nrows, int n2, int H2p, const cpx<T>* twM, const cpx<T>* twP,
                 hipStream_t st) {
-    constexpr int W = row_w<M>();
-    unsigned g = (unsigned)((nrows + W - 1) / W);
-    hipLaunchKernelGGL((k_c2r_rows<T, TO, M>), dim3(g), dim3(row_nt<M>()), 0, st, in, (TO*)x, nrows, n2, H2p, twM,
-                       twP, Live{nullptr, 1});
+    if constexpr (rows_two_level<T, M>()) {
+        constexpr int W = rows2_w64<M>();
+        hipLaunchKernelGGL((k_c2r_rows2<T, M, W>), dim3((unsigned)((nrows + W - 1) / W)), dim3(W * split2(M).B), 0, st,
+                           in, (T*)x, nrows, n2, H2p, twM, twP, Live{nullptr, 1});
+    } else {
+        constexpr int W = row_w<M>();
+        unsigned g = (unsigned)((nrows + W - 1) / W);
+        hipLaunchKernelGGL((k_c2r_rows<T, TO, M>), dim3(g), dim3(row_nt<M>()), 0, st, in, (TO*)x, nrows, n2, H2p, twM,
+                           twP, Live{nullptr, 1});
+    }
 }
 template <typename T, int L, int S>
 void launch_cols(const cpx<T>* in, cpx<T>* out, Geo gi, Geo go, int npencil, int nin, int nkeep, int ncol,
                  const cpx<T>* tw, hipStream_t st) {
-    constexpr int W = col_w<T, L>();
-    dim3 g((unsigned)((ncol + W - 1) / W), (unsigned)npencil);
-    hipLaunchKernelGGL((k_cols<T, L, S>), g, dim3(col_nt<T, L>()), 0, st, in, out, gi, go, nin, nkeep, ncol, tw,
-                       Live{nullptr, 1});
+    if constexpr (cols_two_level<T, L>()) {
+        constexpr int W = 8;  // 128 bytes
+        dim3 g((unsigned)((ncol + W - 1) / W), (unsigned)npencil);
+        hipLaunchKernelGGL((k_cols2<T, L, S, W>), g, dim3(W * split2(L).B), 0, st, in, out, gi, go, nin, nkeep, ncol,
+                           tw, Live{nullptr, 1});
+    } else {
+        constexpr int W = col_w<T, L>();
+        dim3 g((unsigned)((ncol + W - 1) / W), (unsigned)npencil);
+        hipLaunchKernelGGL((k_cols<T, L, S>), g, dim3(col_nt<T, L>()), 0, st, in, out, gi, go, nin, nkeep, ncol, tw,
+                           Live{nullptr, 1});
+    }
 }
 template <typename T, typename TK, int L>
 void launch_zconv(cpx<T>* X, const TK* kern, int N0, int P1, int H2, int H2p, int K1, T srcMul, const cpx<T>* tw,
                   hipStream_t st) {
-    constexpr int W = z_w<T, L>();
-    dim3 g((unsigned)((H2 + W - 1) / W), (unsigned)(P1 / 2 + 1));
-    hipLaunchKernelGGL((k_zconv<T, TK, L>), g, dim3(z_nt<T, L>()), 0, st, X, kern, N0, P1, H2, H2p, K1, H2, srcMul,
-                       tw, Live{nullptr, 1});
+    auto grid = [&](int W) { return dim3((unsigned)((H2 + W - 1) / W), (unsigned)(P1 / 2 + 1)); };
+    const Live all{nullptr, 1};
+    if constexpr (sizeof(T) == 8 && L > 1 && L <= 8) {
+        hipLaunchKernelGGL((k_zconv2<T, TK, L, 16>), grid(16), dim3(96), 0, st, X, kern, N0, P1, H2, H2p, K1, H2,
+                           srcMul, tw, all);
+    } else if constexpr (sizeof(T) == 8 && L > 8 && L <= 40 && L % 2 == 0) {
+        hipLaunchKernelGGL((k_zconv2m<T, TK, L, 16, 2>), grid(16), dim3(192), 0, st, X, kern, N0, P1, H2, H2p, K1, H2,
+                           srcMul, tw, all);
+    } else if constexpr (sizeof(T) == 8 && L > 40 && L <= 128 && L % 4 == 0) {
+        hipLaunchKernelGGL((k_zconv2m<T, TK, L, 8, 4>), grid(8), dim3(192), 0, st, X, kern, N0, P1, H2, H2p, K1, H2,
+                           srcMul, tw, all);
+    } else {
+        hipLaunchKernelGGL((k_zconv<T, TK, L>), grid(z_w<T, L>()), dim3(z_nt<T, L>()), 0, st, X, kern, N0, P1, H2,
+                           H2p, K1, H2, srcMul, tw, all);
+    }
 }
 
 template <typename T, typename TI>

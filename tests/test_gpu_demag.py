@@ -238,3 +238,26 @@ def test_length_beyond_the_generic_passes_is_an_error():
     from hotspin_amd._lib import HotspinError
     with pytest.raises(HotspinError, match="hs error 10002"):  # HS_ESIZE
         Demag((1, 1, 4097), (2e-9, 2e-9, 2e-9))
+
+
+# FP64 five passes (a periodic axis 1 or more than 32 planes) at the lengths where their
+# kernels change: axis 0 with one, two and four lanes a pencil and beyond; columns
+# and rows in two levels and in Stockham stages
+FP64_PASSES = ([((n0, 8, 16), (0, 1, 0)) for n0 in (2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32)] +
+               [((n0, 4, 8), (0, 0, 0)) for n0 in (40, 48, 64, 80)] +
+               [((34, n1, 8), (0, 0, 0)) for n1 in (16, 24, 160, 192, 256)] +
+               [((34, 4, n2), (0, 0, 0)) for n2 in (16, 20, 24, 48, 96, 256, 320, 512, 640, 768)])
+
+
+@pytest.mark.parametrize("N,pbc", FP64_PASSES)
+def test_f64_passes_match_oracle(N, pbc):
+    cell = (2e-9, 3e-9, 2.5e-9)
+    rng = np.random.default_rng(sum(N))
+    n = N[0] * N[1] * N[2]
+    m, msk = rng.standard_normal((3, n)), rng.random(n)
+    d, o = Demag(N, cell, pbc), po.Demag(N, cell, pbc)
+    assert relerr(d.kernel(), o.kernel()) <= 1e-12
+    dm, dw, B = dev(m), dev(msk), empty((3, n))
+    d.field_f64(P(dm), P(dw), 8e5, P(B))
+    assert relerr(host(B), o.B(m, msk, 8e5).reshape(3, n)) <= 1e-12
+    d.close()
