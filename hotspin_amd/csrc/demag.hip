@@ -32,6 +32,7 @@
 #include <map>
 #include <vector>
 
+#include "hostcopy.hpp"
 #include "hs_common.hpp"
 
 #define HS_PI_D 3.141592653589793
@@ -394,6 +395,24 @@ __global__ void k_kernel_fill(double* __restrict__ full, const double* __restric
     full[c * n + g] = xm < h0 && ym < h1 && zm < h2 ? sg * oct[c * noct + ((long)xm * h1 + ym) * h2 + zm] : 0.0;
 }
 
+// max |oct| of each component into bits[6] (zeroed beforehand).  Copying the octant
+// to the host for its maxima took 1.6 of the 10.4 ms of a plan at 256x256x8.
+__global__ void __launch_bounds__(256) k_octant_max(const double* __restrict__ oct, long noct,
+                                                    unsigned long long* __restrict__ bits) {
+    __shared__ double wm[4];
+    const int c = blockIdx.y;
+    double m = 0;
+    for (long g = (long)blockIdx.x * blockDim.x + threadIdx.x; g < noct; g += (long)gridDim.x * blockDim.x)
+        m = fmax(m, fabs(oct[c * noct + g]));
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < (int)(blockDim.x >> 6); w++) m = fmax(m, wm[w]);
+        atomicMax(&bits[c], (unsigned long long)__double_as_longlong(m));
+    }
+}
+
 // Keep the real part of the first octant of the transformed kernel, scaled by
 // 1/(P0 P1 P2); record max|imag| and max|real| (extract(), maxwell_convolution.go:350-388).
 // kern64 rows at pitch H2, kern32 rows at pitch KP; the maxima go through a
@@ -490,8 +509,9 @@ namespace {
 // demag_kernels.hpp elsewhere.  Times of one pass, Stockham / two-level:
 // - rows (33 MB): R2C 14.8 / 9.9 us at M = 64, 19.1 / 11.4 at 256, 16.2 / 13.3
 //   at 512; C2R 12.7 / 8.0, 17.0 / 8.8, 15.7 / 9.4; M = 1024 15.0 / 25.5.
-//   Eight rows a block (16 where eight give less than a wave, four from 384
-//   points on: R2C at 512 with eight 13.1, C2R 13.7).
+//   Eight rows a block (16 where eight give less than a wave), four from 384
+//   points on (R2C at 384 with eight 24.7 against 13.5) except for R2C at 512,
+//   which keeps its occupancy with eight (77 against 93 us at 512x512x16).
 // - columns (107 MB out and in): 55 / 54 us at 32 points, 65 / 57 at 128,
 //   102 / 66 at 320, but 86 / 96 at 512 and within 5 % at 768 and 1024.
 // - axis 0 with the product (1.8 MB a plane): one lane a pencil up to 8
@@ -499,7 +519,10 @@ namespace {
 //   (86 / 32 at 64, 163 / 100 at 128): 565 / 190 us at 512x512x16, where the
 //   Stockham kernel took half the time of the field.
 template <int M>
-constexpr int rows2_w64() { return M >= 384 ? 4 : (8 * split2(M).B >= 64 ? 8 : 16); }
+constexpr int rows2_w64(bool c2r) {
+    if (M >= 384) return c2r || M != 512 ? 4 : 8;
+    return 8 * split2(M).B >= 64 ? 8 : 16;
+}
 template <typename T, int M>
 constexpr bool rows_two_level() { return sizeof(T) == 8 && M >= 16 && M <= 640 && two_level_ok(M); }
 template <typename T, int L>
@@ -509,7 +532,7 @@ template <typename T, typename TI, int M>
 void launch_r2c(const void* x, const void* msk, long mrows, cpx<T>* out, long nrows, int n2, int H2p,
                 const cpx<T>* twM, const cpx<T>* twP, hipStream_t st) {
     if constexpr (rows_two_level<T, M>()) {
-        constexpr int W = rows2_w64<M>();
+        constexpr int W = rows2_w64<M>(false);
         hipLaunchKernelGGL((k_r2c_rows2<T, M, W>), dim3((unsigned)((nrows + W - 1) / W)), dim3(W * split2(M).B), 0, st,
                            (const T*)x, (const T*)msk, mrows, out, nrows, n2, H2p, twM, twP, Live{nullptr, 1});
     } else {
@@ -523,7 +546,7 @@ template <typename T, typename TO, int M>
 void launch_c2r(const cpx<T>* in, void* x, long nrows, int n2, int H2p, const cpx<T>* twM, const cpx<T>* twP,
                 hipStream_t st) {
     if constexpr (rows_two_level<T, M>()) {
-        constexpr int W = rows2_w64<M>();
+        constexpr int W = rows2_w64<M>(true);
         hipLaunchKernelGGL((k_c2r_rows2<T, M, W>), dim3((unsigned)((nrows + W - 1) / W)), dim3(W * split2(M).B), 0, st,
                            in, (T*)x, nrows, n2, H2p, twM, twP, Live{nullptr, 1});
     } else {
@@ -1314,13 +1337,13 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
         hipLaunchKernelGGL(k_kernel_arne_near, dim3(1024), dim3(kNearThreads), 0, st, oct, ap, near, near - 2);
     }
     // IsZero (maxwell_convolution.go:227-232): components below 1e-12 of the
-    // global max are dropped.  Done on the host from the octant.
-    std::vector<double> hoct(6 * noct);
-    hipMemcpyAsync(hoct.data(), oct, sizeof(double) * 6 * noct, hipMemcpyDeviceToHost, st);
+    // global max are dropped.
+    hipMemsetAsync(maxbits, 0, 6 * sizeof(unsigned long long), st);
+    hipLaunchKernelGGL(k_octant_max, dim3(std::min(256, hs::div_up(noct, 256)), 6), dim3(256), 0, st, oct, noct,
+                       maxbits);
+    double gmax = 0, cmax[6];
+    hipMemcpyAsync(cmax, maxbits, sizeof(cmax), hipMemcpyDeviceToHost, st);
     hipStreamSynchronize(st);
-    double gmax = 0, cmax[6] = {0, 0, 0, 0, 0, 0};
-    for (int c = 0; c < 6; c++)
-        for (long i = 0; i < noct; i++) cmax[c] = fmax(cmax[c], fabs(hoct[c * noct + i]));
     for (int c = 0; c < 6; c++) gmax = fmax(gmax, cmax[c]);
     const KernelBufs kb{oct, full, X, maxbits};
     kernel_transform(d, kb, d->kern64, d->kern32, st);
@@ -1401,7 +1424,10 @@ extern "C" int hs_demag_sizes(const hs_demag* d, int P[3], int K[3]) {
 extern "C" int hs_demag_kernel_f64(const hs_demag* d, double* host_out) {
     if (!d || !host_out) return HS_EINVAL;
     long nk = (long)d->logicK[0] * d->logicK[1] * d->logicK[2];
-    hipError_t e = hipMemcpy(host_out, d->kernL ? d->kernL : d->kern64, sizeof(double) * 6 * nk, hipMemcpyDeviceToHost);
+    const double* k = d->kernL ? d->kernL : d->kern64;
+    const std::shared_ptr<HostStage> stage = HostStage::get();
+    const hipError_t e = stage ? stage->out(host_out, k, sizeof(double) * 6 * nk, nullptr)
+                               : hipMemcpy(host_out, k, sizeof(double) * 6 * nk, hipMemcpyDeviceToHost);
     return e == hipSuccess ? 0 : (int)e;
 }
 
