@@ -86,7 +86,7 @@ __device__ __forceinline__ double fmaT(double a, double b, double c) { return __
 // axis-0 items per thread: 3 IB values each, at most 24 in all
 constexpr int mid_itm(int IB) { return 8 / IB; }
 
-// Shape of a column's tile: compile-time here, at run time in k_fmid_any.
+// Shape of a column's tile.
 template <int Q_, bool FOLD>
 struct Geom {
     static constexpr int Q = Q_, A = split_even(Q_).A, B = split_even(Q_).B, BP = B + 1, PL = A * BP;
@@ -345,9 +345,33 @@ constexpr int row_pitch() {
     return M + 1 + ((64 / W - (M + 1)) % 32 + 32) % 32;
 }
 template <int M, int W>
-constexpr int frow_lds() {
+constexpr int frow_full() {
     constexpr int A = split2(M).A, B = split2(M).B;
     return (W * A * (B + 1) > W * row_pitch<M, W>()) ? W * A * (B + 1) : W * row_pitch<M, W>();
+}
+// Folded FP32 rows whose tile is larger than 48 KB go through LDS in halves,
+// even frequencies (in the exchange: even k1) first, then odd: the pairs k,
+// M - k that R2C and C2R need have one parity.  The room goes into more rows a
+// block, for longer pieces of a column: at 512x512x16, folded 8 ways, 32 rows
+// in halves (64-byte pieces) take 57 us forward and 77 inverse, 16 rows (32-byte
+// pieces) whole 73 and 81, in halves 76 and 82; the copy rate gives 32.
+template <typename T, int M, int W, int R>
+constexpr bool row_halves() {
+    return sizeof(T) == 4 && R > 1 && split2(M).A % 2 == 0 && split2(M).B % 2 == 0 &&
+           (long)frow_full<M, W>() * (long)sizeof(cpx<T>) > 49152;
+}
+// pitch of a row's half spectrum: 32 / WA lanes of each of WA rows on distinct banks
+template <int M, int WA>
+constexpr int half_pitch() {
+    constexpr int n = M / 2 + 1, want = WA >= 32 ? 1 : 32 / WA;
+    return n + ((want - n) % 32 + 32) % 32;
+}
+template <typename T, int M, int W, int R>
+constexpr int frow_lds() {
+    constexpr int A = split2(M).A, B = split2(M).B;
+    if (!row_halves<T, M, W, R>()) return frow_full<M, W>();
+    constexpr int x = W * (A / 2) * (B + 1), y = W * half_pitch<M, (R > 1 ? W / (R / 2) : W)>();
+    return x > y ? x : y;
 }
 
 // Rows of a block.  R = 1: W consecutive rows.  R > 1 (axis 1 folded by R):
@@ -410,11 +434,20 @@ __global__ void __launch_bounds__(NT) k_frows(const T* __restrict__ x, const T* 
                                               const cpx<T>* __restrict__ tw1, Live lv) {
     constexpr int A = split2(M).A, B = split2(M).B, BP = B + 1, PM = row_pitch<M, W>();
     static_assert(A * B == M && A <= B, "two-level split");
-    __shared__ cpx<T> lds[frow_lds<M, W>()];
+    __shared__ cpx<T> lds[frow_lds<T, M, W, R>()];
     __shared__ cpx<T> tws[M + 1];
+    constexpr bool HALVES = row_halves<T, M, W, R>();
     const int tid = threadIdx.x, n2 = g.n2;
     const RowMap<W, R> rm(g);
     if (rm.dead(g, lv)) return;
+    cpx<T> u[B];
+    const int k1 = tid % A, p2 = tid / A;
+    // X[k] = E + w^k O from Z[k] and Z[M - k]
+    auto split = [&](const cpx<T>& zk, const cpx<T>& zm, int k) {
+        const cpx<T> E = {half * (zk.x + zm.x), half * (zk.y - zm.y)};
+        const cpx<T> O = {half * (zk.y + zm.y), half * (zm.x - zk.x)};
+        return cadd(E, cmul(tws[k], O));
+    };
     constexpr int TA = (M + NT - 1) / NT, TB = (M + 1 + NT - 1) / NT;
     cpx<T> ta[TA], tb[TB];
 #pragma unroll
@@ -475,15 +508,65 @@ __global__ void __launch_bounds__(NT) k_frows(const T* __restrict__ x, const T* 
             if (tid + q * NT < M) tws[tid + q * NT] = ta[q];
         __syncthreads();
         dft_reg<T, A, -1>(v);
+        if constexpr (HALVES) {
 #pragma unroll
-        for (int k1 = 0; k1 < A; k1++) lds[(p * A + k1) * BP + nb] = k1 ? cmul(v[k1], tws[nb * k1]) : v[k1];
+            for (int k1 = 1; k1 < A; k1++) v[k1] = cmul(v[k1], tws[nb * k1]);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+#pragma unroll
+                for (int q = 0; q < A / 2; q++) lds[(p * (A / 2) + q) * BP + nb] = v[2 * q + h];
+                __syncthreads();
+                if (tid < W * A && k1 % 2 == h) {
+#pragma unroll
+                    for (int m = 0; m < B; m++) u[m] = lds[(p2 * (A / 2) + k1 / 2) * BP + m];
+                }
+                __syncthreads();
+            }
+        } else {
+#pragma unroll
+            for (int k1 = 0; k1 < A; k1++) lds[(p * A + k1) * BP + nb] = k1 ? cmul(v[k1], tws[nb * k1]) : v[k1];
+        }
     }
-    __syncthreads();
+    if constexpr (!HALVES) __syncthreads();
 #pragma unroll
     for (int q = 0; q < TB; q++)
         if (tid + q * NT <= M) tws[tid + q * NT] = tb[q];
-    cpx<T> u[B];
-    const int k1 = tid % A, p2 = tid / A;
+    if constexpr (HALVES) {
+        constexpr int RH = R / 2, WA = W / RH, KS = NT / WA, PH = half_pitch<M, WA>();
+        if (tid < W * A) dft_reg<T, B, -1>(u);
+        const int a = tid % WA, kk = tid / WA, j = rm.j0 + a;
+        const bool jin = j < g.Q;
+        cpx<T> wj[R];
+#pragma unroll
+        for (int s = 1; s < R; s++) wj[s] = tw1[s * (jin ? j : 0)];
+        const long cs = (long)g.PC * g.Q;
+        cpx<T>* o = out + rm.sol * (long)(M + 1) * R * cs + (long)rm.pen * g.Q + j;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (h) __syncthreads();
+            if (tid < W * A && k1 % 2 == h) {
+#pragma unroll
+                for (int k2 = 0; k2 < B; k2++) lds[p2 * PH + (k1 + A * k2) / 2] = u[k2];
+            }
+            __syncthreads();
+            if (jin)
+                for (int k = h + 2 * kk; k <= M; k += 2 * KS) {
+                    cpx<T> f[R];
+#pragma unroll
+                    for (int m = 0; m < R; m++) {
+                        f[m] = {T(0), T(0)};
+                        if (m < RH) {
+                            const cpx<T>* z = lds + (m * WA + a) * PH;
+                            f[m] = split(z[(k == M ? 0 : k) / 2], z[(k == 0 ? 0 : M - k) / 2], k);
+                        }
+                    }
+                    dft_reg<T, R, -1>(f);
+#pragma unroll
+                    for (int s = 0; s < R; s++) o[((long)k * R + s) * cs] = s ? cmul(f[s], wj[s]) : f[s];
+                }
+        }
+        return;
+    }
     if (tid < W * A) {
 #pragma unroll
         for (int m = 0; m < B; m++) u[m] = lds[(p2 * A + k1) * BP + m];
@@ -495,13 +578,8 @@ __global__ void __launch_bounds__(NT) k_frows(const T* __restrict__ x, const T* 
         for (int k2 = 0; k2 < B; k2++) lds[p2 * PM + k1 + A * k2] = u[k2];
     }
     __syncthreads();
-    // split X[k] = E + w^k O
-    auto split = [&](int p, int k) {
-        const cpx<T> zk = lds[p * PM + (k == M ? 0 : k)];
-        const cpx<T> zm = lds[p * PM + (k == 0 ? 0 : M - k)];
-        const cpx<T> E = {half * (zk.x + zm.x), half * (zk.y - zm.y)};
-        const cpx<T> O = {half * (zk.y + zm.y), half * (zm.x - zk.x)};
-        return cadd(E, cmul(tws[k], O));
+    auto split_row = [&](int p, int k) {
+        return split(lds[p * PM + (k == M ? 0 : k)], lds[p * PM + (k == 0 ? 0 : M - k)], k);
     };
     if constexpr (R == 1) {  // lanes walk the W rows first, so that a column's W values leave together
         const int p = tid % W, kk = tid / W;
@@ -511,8 +589,8 @@ __global__ void __launch_bounds__(NT) k_frows(const T* __restrict__ x, const T* 
             const long sol = r / g.rows;
             cpx<T>* o = out + sol * (M + 1) * (long)g.rows + (r - sol * g.rows);
 #pragma unroll
-            for (int q = 0; q < A; q++) o[(long)(kk + B * q) * g.rows] = split(p, kk + B * q);
-            if (kk == 0) o[(long)M * g.rows] = split(p, M);
+            for (int q = 0; q < A; q++) o[(long)(kk + B * q) * g.rows] = split_row(p, kk + B * q);
+            if (kk == 0) o[(long)M * g.rows] = split_row(p, M);
         }
     } else {  // ... the WA values of j' first
         constexpr int RH = R / 2, WA = W / RH, KS = NT / WA;
@@ -526,7 +604,7 @@ __global__ void __launch_bounds__(NT) k_frows(const T* __restrict__ x, const T* 
             for (int k = kk; k <= M; k += KS) {
                 cpx<T> f[R];
 #pragma unroll
-                for (int m = 0; m < R; m++) f[m] = m < RH ? split(m * WA + a, k) : cpx<T>{T(0), T(0)};
+                for (int m = 0; m < R; m++) f[m] = m < RH ? split_row(m * WA + a, k) : cpx<T>{T(0), T(0)};
                 dft_reg<T, R, -1>(f);
 #pragma unroll
                 for (int s = 0; s < R; s++) o[((long)k * R + s) * cs] = s ? cmul(f[s], wj[s]) : f[s];
@@ -543,12 +621,24 @@ __global__ void __launch_bounds__(NT) k_irows(const cpx<T>* __restrict__ in, T* 
                                               const cpx<T>* __restrict__ tw1, Live lv) {
     constexpr int A = split2(M).A, B = split2(M).B, BP = B + 1, PM = row_pitch<M, W>();
     static_assert(A * B == M && A <= B, "two-level split");
-    __shared__ cpx<T> lds[frow_lds<M, W>()];
+    __shared__ cpx<T> lds[frow_lds<T, M, W, R>()];
     __shared__ cpx<T> tws[M];
     __shared__ cpx<T> twp[M];
+    constexpr bool HALVES = row_halves<T, M, W, R>();
     const int tid = threadIdx.x, n2 = g.n2;
     const RowMap<W, R> rm(g);
     if (rm.dead(g, lv)) return;
+    const int nb = tid % B, p = tid / B;
+    cpx<T> v[A];
+    // Z[k] of C2R from X[k] and X[M - k]
+    auto join = [&](const cpx<T>& a, const cpx<T>& b, int k) -> cpx<T> {
+        const cpx<T> s = {a.x + b.x, a.y - b.y};
+        const cpx<T> d = {a.x - b.x, a.y + b.y};
+        cpx<T> w = twp[k];
+        w.y = -w.y;
+        const cpx<T> wd = cmul(w, d);
+        return {s.x - wd.y, s.y + wd.x};
+    };
     {
         constexpr int TA = (M + NT - 1) / NT;
         cpx<T> ta[TA], tb[TA];
@@ -571,6 +661,63 @@ __global__ void __launch_bounds__(NT) k_irows(const cpx<T>* __restrict__ in, T* 
 #pragma unroll
             for (int q = 0; q < A; q++) lds[p * PM + kk + B * q] = v[q];
             if (kk == 0) lds[p * PM + M] = vm;
+        } else if constexpr (HALVES) {
+            constexpr int RH = R / 2, WA = W / RH, KS = NT / WA, PH = half_pitch<M, WA>(), U = (M / 2 + KS - 1) / KS;
+            const int a = tid % WA, kk = tid / WA, j = rm.j0 + a < g.Q ? rm.j0 + a : 0;
+            cpx<T> wj[R];
+#pragma unroll
+            for (int s = 1; s < R; s++) {
+                wj[s] = tw1[s * j];
+                wj[s].y = -wj[s].y;
+            }
+            const long cs = (long)g.PC * g.Q;
+            const cpx<T>* q0 = in + rm.sol * (long)(M + 1) * R * cs + (long)rm.pen * g.Q + j;
+            // the R columns of frequency k, and their last radix into LDS
+            auto fetch = [&](int k, cpx<T>* f) {
+#pragma unroll
+                for (int s = 0; s < R; s++) f[s] = q0[((long)k * R + s) * cs];
+            };
+            auto place = [&](int k, cpx<T>* f) {
+#pragma unroll
+                for (int s = 1; s < R; s++) f[s] = cmul(f[s], wj[s]);
+                dft_reg<T, R, +1>(f);
+#pragma unroll
+                for (int m = 0; m < RH; m++) lds[(m * WA + a) * PH + k / 2] = f[m];
+            };
+            auto freq = [&](int h, int u) { return h + 2 * (kk + u * KS); };  // < M: one of half h
+            cpx<T> f[U][R], fm[R];
+#pragma unroll
+            for (int u = 0; u < U; u++) fetch(freq(0, u) < M ? freq(0, u) : 0, f[u]);
+            if (kk == 0) fetch(M, fm);
+#pragma unroll
+            for (int q = 0; q < TA; q++) {
+                const int e = tid + q * NT;
+                if (e < M) {
+                    tws[e] = ta[q];
+                    twp[e] = tb[q];
+                }
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (freq(h, u) < M) place(freq(h, u), f[u]);
+                if (h == 0 && kk == 0) place(M, fm);
+                __syncthreads();
+                if (nb % 2 == h) {
+                    const cpx<T>* z = lds + p * PH;
+#pragma unroll
+                    for (int n1 = 0; n1 < A; n1++) {
+                        const int k = B * n1 + nb;
+                        v[n1] = join(z[k / 2], z[(M - k) / 2], k);
+                    }
+                }
+                if (h == 0) {
+#pragma unroll
+                    for (int u = 0; u < U; u++) fetch(freq(1, u) < M ? freq(1, u) : 1, f[u]);
+                }
+                __syncthreads();
+            }
         } else {
             constexpr int RH = R / 2, WA = W / RH, KS = NT / WA, U = 16 / R > 1 ? 16 / R : 1;
             const int a = tid % WA, kk = tid / WA, j = rm.j0 + a < g.Q ? rm.j0 + a : 0;
@@ -603,46 +750,59 @@ __global__ void __launch_bounds__(NT) k_irows(const cpx<T>* __restrict__ in, T* 
                 }
             }
         }
+        if constexpr (!HALVES) {
 #pragma unroll
-        for (int q = 0; q < TA; q++) {
-            const int e = tid + q * NT;
-            if (e < M) {
-                tws[e] = ta[q];
-                twp[e] = tb[q];
+            for (int q = 0; q < TA; q++) {
+                const int e = tid + q * NT;
+                if (e < M) {
+                    tws[e] = ta[q];
+                    twp[e] = tb[q];
+                }
             }
         }
     }
-    __syncthreads();
-    const int nb = tid % B, p = tid / B;
-    cpx<T> v[A];
+    if constexpr (!HALVES) {
+        __syncthreads();
 #pragma unroll
-    for (int n1 = 0; n1 < A; n1++) {
-        const int k = B * n1 + nb;
-        cpx<T> a = lds[p * PM + k];
-        cpx<T> b = lds[p * PM + (M - k)];
-        cpx<T> s = {a.x + b.x, a.y - b.y};
-        cpx<T> d = {a.x - b.x, a.y + b.y};
-        cpx<T> w = twp[k];
-        w.y = -w.y;
-        cpx<T> wd = cmul(w, d);
-        v[n1] = {s.x - wd.y, s.y + wd.x};
+        for (int n1 = 0; n1 < A; n1++) {
+            const int k = B * n1 + nb;
+            v[n1] = join(lds[p * PM + k], lds[p * PM + (M - k)], k);
+        }
+        __syncthreads();
     }
-    __syncthreads();
     dft_reg<T, A, +1>(v);
 #pragma unroll
-    for (int k1 = 0; k1 < A; k1++) {
+    for (int k1 = 1; k1 < A; k1++) {
         cpx<T> w = tws[nb * k1];
         w.y = -w.y;
-        lds[(p * A + k1) * BP + nb] = k1 ? cmul(v[k1], w) : v[k1];
+        v[k1] = cmul(v[k1], w);
     }
-    __syncthreads();
+    cpx<T> u[B];
+    const int k1 = tid % A, p2 = tid / A;
+    if constexpr (HALVES) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (h) __syncthreads();
+#pragma unroll
+            for (int q = 0; q < A / 2; q++) lds[(p * (A / 2) + q) * BP + nb] = v[2 * q + h];
+            __syncthreads();
+            if (tid < W * A && k1 % 2 == h) {
+#pragma unroll
+                for (int m = 0; m < B; m++) u[m] = lds[(p2 * (A / 2) + k1 / 2) * BP + m];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int k1 = 0; k1 < A; k1++) lds[(p * A + k1) * BP + nb] = v[k1];
+        __syncthreads();
+    }
     if (tid < W * A) {
-        const int k1 = tid % A, p2 = tid / A;
         bool rin;
         const long r = rm.row(g, p2, rin);
-        cpx<T> u[B];
+        if constexpr (!HALVES) {
 #pragma unroll
-        for (int m = 0; m < B; m++) u[m] = lds[(p2 * A + k1) * BP + m];
+            for (int m = 0; m < B; m++) u[m] = lds[(p2 * A + k1) * BP + m];
+        }
         dft_reg<T, B, +1>(u);
         if (rin) {
             using V2 = typename std::conditional<sizeof(T) == 4, float2, double2>::type;
@@ -761,21 +921,23 @@ template <typename T>
 Mids<T>& mids_of(int Q);
 
 // Rows per block: full 128-byte pieces of a column (16 rows of 8 bytes) while
-// the tile stays near 32 KB; folded, pieces of 32 bytes or more (neighbouring
-// blocks complete the lines in L2) at up to 72 KB.
+// the tile stays near 32 KB; folded, 16 rows or as many as 72 KB hold, and in
+// halves (row_halves) 32 or as many as 70 KB and a block's threads hold
+// (neighbouring blocks complete the lines in L2).
 template <typename T, int M, int R>
 constexpr int frow_w() {
     constexpr int cs = (int)sizeof(cpx<T>), rh = R > 1 ? R / 2 : 1;
-    int w = 128 / cs;
-    if (R > 1) w = 16;
+    const bool halves = row_halves<T, M, 16, R>();
+    int w = R == 1 ? 128 / cs : (halves ? 32 : 16);
     if (w < rh) w = rh;
-    while (w > 2 && w > rh && ((long)w * M * cs > (R > 1 ? 72000 : 40000) || w * split2(M).B > 1024)) w /= 2;
+    while (w > 2 && w > rh && ((long)w * M * cs > (R == 1 ? 40000 : (halves ? 140000 : 72000)) || w * split2(M).B > 1024))
+        w /= 2;
     while (w < 16 && w * split2(M).B < 64) w *= 2;
     return w;
 }
-template <typename T, int M, int R>
+template <int W, int R>
 unsigned frow_grid(const RowP& g) {
-    constexpr int W = frow_w<T, M, R>(), WA = R > 1 ? W / (R / 2) : W;
+    constexpr int WA = R > 1 ? W / (R / 2) : W;
     if (R == 1) return (unsigned)(((long)g.rows * g.nsolve + W - 1) / W);
     return (unsigned)((long)g.nsolve * g.PC * ((g.Q + WA - 1) / WA));
 }
@@ -783,14 +945,14 @@ template <typename T, int M, int R>
 void launch_frows(const T* x, const T* msk, cpx<T>* out, const RowP& g, T half, const cpx<T>* twM, const cpx<T>* twP,
                   const cpx<T>* tw1, hipStream_t st, Live lv) {
     constexpr int W = frow_w<T, M, R>();
-    hipLaunchKernelGGL((k_frows<T, M, W, R>), dim3(frow_grid<T, M, R>(g)), dim3(W * split2(M).B), 0, st, x, msk, out,
+    hipLaunchKernelGGL((k_frows<T, M, W, R>), dim3(frow_grid<W, R>(g)), dim3(W * split2(M).B), 0, st, x, msk, out,
                        g, half, twM, twP, tw1, lv);
 }
 template <typename T, int M, int R>
 void launch_irows(const cpx<T>* in, T* x, const RowP& g, const cpx<T>* twM, const cpx<T>* twP, const cpx<T>* tw1,
                   hipStream_t st, Live lv) {
     constexpr int W = frow_w<T, M, R>();
-    hipLaunchKernelGGL((k_irows<T, M, W, R>), dim3(frow_grid<T, M, R>(g)), dim3(W * split2(M).B), 0, st, in, x, g,
+    hipLaunchKernelGGL((k_irows<T, M, W, R>), dim3(frow_grid<W, R>(g)), dim3(W * split2(M).B), 0, st, in, x, g,
                        twM, twP, tw1, lv);
 }
 
@@ -809,7 +971,7 @@ void launch_mid(const Mid<T>& m, hipStream_t st) {
 template <typename T, int M, int F>
 void add_rows_fold(Rows<T>& r) {
     constexpr int R = 1 << F, W = frow_w<T, M, R>();
-    constexpr long lds = ((long)frow_lds<M, W>() + 2 * M) * (long)sizeof(cpx<T>);
+    constexpr long lds = ((long)frow_lds<T, M, W, R>() + 2 * M) * (long)sizeof(cpx<T>);
     if constexpr (lds <= kLds && W * split2(M).B <= 1024) {
         r.fwd[F] = &launch_frows<T, M, R>;
         r.inv[F] = &launch_irows<T, M, R>;

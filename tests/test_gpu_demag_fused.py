@@ -103,3 +103,17 @@ def test_ragged_lengths(N, pbc):
         d.field_f32(P(dm), P(dw), 8e5, P(B))
         assert relerr(host(B), want) <= 2e-6
     d.close()
+
+
+# folded FP32 rows that go through LDS in halves, 32 or 16 to a block, against the FP64 field
+@pytest.mark.parametrize("N", [(3, 384, 1024), (8, 320, 384), (16, 512, 512), (9, 200, 768), (4, 512, 640), (16, 500, 333)])
+def test_folded_long_rows(N):
+    n = N[0] * N[1] * N[2]
+    m = np.random.default_rng(n).standard_normal((3, n))
+    d = Demag(N, (2e-9, 3e-9, 2.5e-9))
+    dm, df = dev(m), dev(m, np.float32)
+    B, Bf = empty((3, n)), empty((3, n), torch.float32)
+    d.field_f64(P(dm), None, 8e5, P(B))
+    d.field_f32(P(df), None, 8e5, P(Bf))
+    assert relerr(host(Bf), host(B)) <= 2e-6
+    d.close()
