@@ -1268,6 +1268,15 @@ __global__ void k_axpy1(const double* __restrict__ y0, const double* __restrict_
     if (fout) fout[I] = (float)v;
 }
 
+// A slot's parameters (admission only) and record from the launch arguments:
+// one launch in place of three copies from pageable memory, each of which the
+// host waits for.
+__global__ void k_slot_put(SolveP* sp, Clock* clk, int* live, SolveP q, Clock c, int lv) {
+    if (sp) *sp = q;
+    *clk = c;
+    *live = lv;
+}
+
 __global__ void k_set_state(const double* y, float* mf, int normalize, long N) {
     long I = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (I >= N) return;
@@ -3212,7 +3221,6 @@ extern "C" int hs_slot_admit(hs_solver* s, int slot, const double* m, double TMu
     q.seed = seed;
     q.stream = stream;
     s->sp_host[slot] = q;
-    hipMemcpyAsync(s->sp + slot, &s->sp_host[slot], sizeof(SolveP), hipMemcpyHostToDevice, s->st);
     // state into the set that the next iteration reads, its FP32 copy and field
     const Set cur = slot_set(s, (int)(s->slot_iter & 1));
     const long off = (long)slot * 3 * s->N;
@@ -3231,9 +3239,8 @@ extern "C" int hs_slot_admit(hs_solver* s, int slot, const double* m, double TMu
     c.end = (uint32_t)(step0 + nsteps);
     c.state = nsteps > 0 ? HS_SLOT_RUNNING : HS_SLOT_DONE;
     c.home = (uint32_t)(s->slot_iter & 1);
-    hipMemcpyAsync(s->clk + slot, &c, sizeof(Clock), hipMemcpyHostToDevice, s->st);
-    const int lv = c.state == HS_SLOT_RUNNING ? 1 : 0;
-    hipMemcpyAsync(s->live + slot, &lv, sizeof(int), hipMemcpyHostToDevice, s->st);
+    hipLaunchKernelGGL(k_slot_put, dim3(1), dim3(1), 0, s->st, s->sp + slot, s->clk + slot, s->live + slot, q, c,
+                       c.state == HS_SLOT_RUNNING ? 1 : 0);
     hipStreamSynchronize(s->st);
     s->slot_host[slot] = c;
     HS_LAUNCH_CHECK("hs_slot_admit");
@@ -3291,8 +3298,10 @@ extern "C" int hs_slot_release(hs_solver* s, int slot) {
         return HS_EINVAL;
     }
     // ordered after the iterations already enqueued on the solver's stream
-    hipMemsetAsync(s->clk + slot, 0, sizeof(Clock), s->st);
-    hipMemsetAsync(s->live + slot, 0, sizeof(int), s->st);
+    Clock c;
+    memset(&c, 0, sizeof(c));
+    hipLaunchKernelGGL(k_slot_put, dim3(1), dim3(1), 0, s->st, (SolveP*)nullptr, s->clk + slot, s->live + slot,
+                       SolveP{}, c, 0);
     hipStreamSynchronize(s->st);
     memset(&s->slot_host[slot], 0, sizeof(Clock));
     HS_LAUNCH_CHECK("hs_slot_release");
