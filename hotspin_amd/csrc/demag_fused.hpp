@@ -8,8 +8,9 @@
 //            kernel, inverse FFT along axis 1            X  -> X (in place)
 //   k_irows  C2R along axis 2                            X  -> B
 // so the spectrum is written twice and read twice and the padded axis 1
-// exists in LDS only: 24 N + 48 N0 N1 H2 + 24 N0 (KR/..) bytes instead of
-// 24 N + 48 N0 N1 H2 + 96 N0 P1 H2.
+// exists in LDS only.  Bytes a field in FP32: 24 N + 96 N0 N1 H2 and the
+// kernel table, instead of 24 N + 96 N0 N1 H2 + 96 N0 P1 H2 and the octant; with
+// axis 1 folded (k_frows) 24 N + 96 N0 P1 H2 and the table.
 //
 // X is column-major: [solve][k][c][i][j], k the x frequency, so that a column
 // is one contiguous piece and W rows of the row passes (consecutive j) make
@@ -354,7 +355,7 @@ constexpr int frow_full() {
 // M - k that R2C and C2R need have one parity.  The room goes into more rows a
 // block, for longer pieces of a column: at 512x512x16, folded 8 ways, 32 rows
 // in halves (64-byte pieces) take 57 us forward and 77 inverse, 16 rows (32-byte
-// pieces) whole 73 and 81, in halves 76 and 82; the copy rate gives 32.
+// pieces) whole 73 and 81, in halves 76 and 82; 252 MB at the copy rate take 53.
 template <typename T, int M, int W, int R>
 constexpr bool row_halves() {
     return sizeof(T) == 4 && R > 1 && split2(M).A % 2 == 0 && split2(M).B % 2 == 0 &&
