@@ -753,8 +753,8 @@ bool set_lengths(hs_demag* d, const int P[3]) {
 // convolution.  2 N itself where it is compiled; otherwise the next of 2^k,
 // 3 2^k and 5 2^k costs at most 1.33 times the points and runs the compiled
 // kernels instead of the run-time-length ones (FP32 field, run-time lengths
-// against padded: 100x75x7 78 -> 20 us, 33^3 171 -> 30, 100^3 383 -> 226,
-// 300x300x33 2086 -> 490, 300x300x17 2502 -> 141; no mesh was slower).
+// against padded: 100x75x7 78 -> 20 us, 33^3 171 -> 25, 100^3 383 -> 222,
+// 300x300x33 2086 -> 334, 300x300x17 2502 -> 138; no mesh was slower).
 template <typename F>
 int compiled_length(int P, F ok) {
     int best = 0;
@@ -960,11 +960,21 @@ void tune32(hs_demag* d, hipStream_t st) {
     d->z32 = (d->gen0 || vz.z.empty()) ? hsdm::ZV{} : vz.z[0];
     if (d->fold32) return;  // none of these passes runs
     // a plan with a run-time-length pass keeps the first variant of its compiled
-    // passes, and so does one at longer lengths than its logic size (unless
-    // forced): the timing takes 0.3 s, which meshes of any size would pay each
-    // for themselves
+    // passes
     if (!d->row32.r2c || !d->col32.fwd || !d->z32.fn) return;
+    // a plan at longer lengths than its logic size is not timed (0.3 s, which
+    // meshes of any size would pay each for themselves).  It takes what the
+    // timing picks at twelve shapes of 40 to 128 planes, or what came within a few
+    // per cent of it: the last rows (two-level, eight a block), two-level
+    // columns of 16 and, up to 128 points of axis 0, four lanes a pencil (the last
+    // but one); the last beyond.  50x50x49 40 us a field against 55 with the
+    // first variants, 100x100x36 66 / 90, 300x300x33 334 / 490.
     if (d->kernL) {
+        d->row32 = d->rowi32 = vr.rows.back();
+        const int nt = 16 * split2(d->P[1]).B;
+        auto c = std::find_if(vc.cols.begin(), vc.cols.end(), [&](const hsdm::ColV& v) { return v.W == 16 && v.NT == nt; });
+        if (c != vc.cols.end()) d->col32 = *c;
+        d->z32 = vz.z[d->P[0] <= 128 && vz.z.size() > 1 ? vz.z.size() - 2 : vz.z.size() - 1];
         apply_force(d, vr, vc, vz);
         return;
     }
