@@ -42,27 +42,46 @@
 #include "demag_fused.hpp"
 #include "fft_any.hpp"
 
-hsdm::Variants& hsdm::variants(int L) {
-    static std::map<int, hsdm::Variants> reg;
-    return reg[L];
+// Kernels by length.  Written by the static constructors of the files that
+// compile them and only read afterwards: a look-up of another length finds an
+// empty entry and adds none, so threads may look up side by side.
+namespace {
+template <typename V>
+std::map<int, V>& registry() {
+    static std::map<int, V> reg;
+    return reg;
 }
+template <typename V>
+const V& find_in_registry(int L) {
+    static const V none{};
+    const auto it = registry<V>().find(L);
+    return it == registry<V>().end() ? none : it->second;
+}
+}  // namespace
+
+hsdm::Variants& hsdm::add_variants(int L) { return registry<hsdm::Variants>()[L]; }
+const hsdm::Variants& hsdm::variants(int L) { return find_in_registry<hsdm::Variants>(L); }
 
 namespace fused {
 template <typename T>
-Rows<T>& rows_of(int M) {
-    static std::map<int, Rows<T>> reg;
-    return reg[M];
-}
+Rows<T>& add_rows_of(int M) { return registry<Rows<T>>()[M]; }
 template <typename T>
-Mids<T>& mids_of(int Q) {
-    static std::map<int, Mids<T>> reg;
-    return reg[Q];
-}
-template Rows<float>& rows_of<float>(int);
-template Rows<double>& rows_of<double>(int);
-template Mids<float>& mids_of<float>(int);
-template Mids<double>& mids_of<double>(int);
+Mids<T>& add_mids_of(int Q) { return registry<Mids<T>>()[Q]; }
+template <typename T>
+const Rows<T>& rows_of(int M) { return find_in_registry<Rows<T>>(M); }
+template <typename T>
+const Mids<T>& mids_of(int Q) { return find_in_registry<Mids<T>>(Q); }
+template Rows<float>& add_rows_of<float>(int);
+template Rows<double>& add_rows_of<double>(int);
+template Mids<float>& add_mids_of<float>(int);
+template Mids<double>& add_mids_of<double>(int);
 }  // namespace fused
+
+extern "C" int hs_demag_registered(void) {
+    return (int)(registry<hsdm::Variants>().size() + registry<fused::Rows<float>>().size() +
+                 registry<fused::Rows<double>>().size() + registry<fused::Mids<float>>().size() +
+                 registry<fused::Mids<double>>().size());
+}
 
 // ------------------------------------------------------------------ Kernel_Arne (FP64)
 // The field of the charged faces of the source cell (direction s), averaged
@@ -693,6 +712,8 @@ struct hs_demag {
     // three-kernel convolution (demag_fused.hpp): the fold of axis 1, 0 = not
     // taken, FP32 and FP64 decided separately; kt64 may be filled on first use
     int fold32 = 0, fold64 = 0;
+    fused::Form<float> form32;   // their kernels
+    fused::Form<double> form64;
     float* kt32 = nullptr;
     double* kt64 = nullptr;
     cpx<float>* Xzf = nullptr;   // (cap, 3, P0, P1, H2p): the axis-0 spectrum of a run-time-length F3K
@@ -774,10 +795,19 @@ int fused_fold(const hs_demag* d) {
     const int P1 = d->P[1], N0 = d->N[0];
     if (d->P[2] % 2 || P1 < 2 * d->N[1] || !(N0 == 1 || d->P[0] >= 2 * N0)) return 0;
     return fused::mid_fold(N0, P1, sizeof(cpx<T>), [&](int R) {
-        const auto& m = fused::mids_of<T>(P1 / R);
+        const fused::Mids<T>& m = fused::mids_of<T>(P1 / R);
         return fused::rows_of<T>(d->M).fwd[fused::fold_index(R)] && m.A && m.pick(N0, R > 1) &&
                fused::mid_fits(N0, P1 / R, m.A, m.B, sizeof(cpx<T>));
     });
+}
+// the kernels of fold R, resolved at creation: a field call looks nothing up
+template <typename T>
+fused::Form<T> fused_form(const hs_demag* d, int R) {
+    if (!R) return {};
+    const fused::Rows<T>& r = fused::rows_of<T>(d->M);
+    const fused::Mids<T>& m = fused::mids_of<T>(d->P[1] / R);
+    const int f = fused::fold_index(R);
+    return {r.fwd[f], r.inv[f], m.pick(d->N[0], R > 1), m.A, m.B};
 }
 // values of the fused spectrum (per solve) and of its kernel table
 long fused_spectrum(const hs_demag* d, int R) { return 3L * d->N[0] * (R > 1 ? d->P[1] : d->N[1]) * d->H2p; }
@@ -787,8 +817,7 @@ long fused_table(const hs_demag* d, int R) {
 }
 // Fills the table of fold R from the FP64 octant.
 template <typename T>
-void fill_table(const hs_demag* d, T* kt, int R, hipStream_t st) {
-    const auto& m = fused::mids_of<T>(d->P[1] / R);
+void fill_table(const hs_demag* d, T* kt, int R, const fused::Form<T>& m, hipStream_t st) {
     const int KR = fused_rows(d, R);
     hipLaunchKernelGGL(k_kernel_table<T>, dim3(hs::grid1d((long)d->H2 * fused::table_cols(R) * KR), 6),
                        dim3(hs::kBlock), 0, st, d->kern64, kt, d->N[0], d->P[0], d->P[1], d->H2, d->K[0], d->K[1], R,
@@ -798,23 +827,22 @@ void fill_table(const hs_demag* d, T* kt, int R, hipStream_t st) {
 // The fused convolution of nsolve solves (X: nsolve x fused_spectrum values).
 template <typename T>
 int run_fused(hs_demag* d, const T* m, const T* msk, double srcMul, T* B, hipStream_t st, cpx<T>* X, const T* kt,
-              int R, const cpx<T>* twM, const cpx<T>* twP2, const cpx<T>* tw1, int nsolve, const int* live) {
-    const int N0 = d->N[0], N1 = d->N[1], Q = d->P[1] / R, f = fused::fold_index(R);
-    const auto& fr = fused::rows_of<T>(d->M);
-    const auto& fm = fused::mids_of<T>(Q);
+              int R, const fused::Form<T>& fm, const cpx<T>* twM, const cpx<T>* twP2, const cpx<T>* tw1, int nsolve,
+              const int* live) {
+    const int N0 = d->N[0], N1 = d->N[1], Q = d->P[1] / R;
     const fused::RowP g{3 * N0 * N1, N1, Q, 3 * N0, nsolve, d->N[2], (long)N0 * N1};
     const Live lrows{live, g.rows};
     hs::prof_begin(HS_PROF_F1, st);
-    fr.fwd[f](m, msk, X, g, T(0.5 * srcMul), twM, twP2, tw1, st, lrows);
+    fm.fwd(m, msk, X, g, T(0.5 * srcMul), twM, twP2, tw1, st, lrows);
     hs::prof_end(HS_PROF_F1, st);
     hs::prof_begin(HS_PROF_F3K, st);
     const int ncol = d->H2 * R;
     const fused::Mid<T> a{X,    kt,     N0, N1, ncol, fused::mid_cb(N0, Q, fm.A, fm.B, ncol, nsolve, sizeof(cpx<T>)),
                           nsolve, R, tw1, live};
-    fm.pick(N0, R > 1)(a, st);
+    fm.mid(a, st);
     hs::prof_end(HS_PROF_F3K, st);
     hs::prof_begin(HS_PROF_I1, st);
-    fr.inv[f](X, B, g, twM, twP2, tw1, st, lrows);
+    fm.inv(X, B, g, twM, twP2, tw1, st, lrows);
     hs::prof_end(HS_PROF_I1, st);
     HS_LAUNCH_CHECK("hs_demag_field");
     return hs_last_error();
@@ -838,8 +866,8 @@ int run_field32(hs_demag* d, const float* m, const float* msk, double srcMul, fl
         return HS_EINVAL;
     }
     if (d->fold32)
-        return run_fused<float>(d, m, msk, srcMul, B, st, X1, d->kt32, d->fold32, d->twMf, d->twP2f, d->tw1f, nsolve,
-                                live);
+        return run_fused<float>(d, m, msk, srcMul, B, st, X1, d->kt32, d->fold32, d->form32, d->twMf, d->twP2f, d->tw1f,
+                                nsolve, live);
     const long nrows = 3L * N0 * N1 * nsolve;
     Geo g1 = {(long)N1 * H2p, 0, H2p, 1};
     Geo g2 = {(long)P1 * H2p, 0, H2p, 1};
@@ -938,7 +966,7 @@ void tune_file_append(const hs_demag* d, const std::array<int, 3>& counts, const
     }
 }
 
-void apply_force(hs_demag* d, hsdm::Variants& vr, hsdm::Variants& vc, hsdm::Variants& vz) {
+void apply_force(hs_demag* d, const hsdm::Variants& vr, const hsdm::Variants& vc, const hsdm::Variants& vz) {
     // HS_DEMAG_FORCE="r,c,z": variant indices to use instead of the timed
     // choice (-1 keeps it), for tests that cover every registered variant
     if (const char* f = getenv("HS_DEMAG_FORCE")) {
@@ -952,9 +980,9 @@ void apply_force(hs_demag* d, hsdm::Variants& vr, hsdm::Variants& vc, hsdm::Vari
 }
 
 void tune32(hs_demag* d, hipStream_t st) {
-    hsdm::Variants& vr = hsdm::variants(d->M);
-    hsdm::Variants& vc = hsdm::variants(d->P[1]);
-    hsdm::Variants& vz = hsdm::variants(d->P[0]);
+    const hsdm::Variants& vr = hsdm::variants(d->M);
+    const hsdm::Variants& vc = hsdm::variants(d->P[1]);
+    const hsdm::Variants& vz = hsdm::variants(d->P[0]);
     d->row32 = d->rowi32 = (d->genR || vr.rows.empty()) ? hsdm::RowV{} : vr.rows[0];
     d->col32 = (d->gen1 || vc.cols.empty()) ? hsdm::ColV{} : vc.cols[0];
     d->z32 = (d->gen0 || vz.z.empty()) ? hsdm::ZV{} : vz.z[0];
@@ -1128,7 +1156,7 @@ int run_field(hs_demag* d, const T* m, const T* msk, double srcMul, T* B, hipStr
     const int H2 = d->H2, H2p = d->H2p, M = d->M;
     if constexpr (sizeof(T) == 8)
         if (d->fold64)
-            return run_fused<T>(d, m, msk, srcMul, B, st, X1, d->kt64, d->fold64, twM, twP2, tw1, 1, nullptr);
+            return run_fused<T>(d, m, msk, srcMul, B, st, X1, d->kt64, d->fold64, d->form64, twM, twP2, tw1, 1, nullptr);
     auto r2c = d->genRd ? nullptr : pick_r2c<T, T>(M);
     auto c2r = d->genRd ? nullptr : pick_c2r<T, T>(M);
     auto f1 = d->gen1d ? nullptr : pick_cols<T, -1>(P1);
@@ -1287,6 +1315,8 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     // HS_DEMAG_FORCE asks for particular five-pass variants
     d->fold32 = getenv("HS_DEMAG_FORCE") ? 0 : fused_fold<float>(d);
     d->fold64 = fused_fold<double>(d);
+    d->form32 = fused_form<float>(d, d->fold32);
+    d->form64 = fused_form<double>(d, d->fold64);
     hipMalloc(&d->X1f, sizeof(cpx<float>) * fused_spectrum(d, d->fold32));
     if (!d->fold32) hipMalloc(&d->X2f, sizeof(cpx<float>) * 3L * N[0] * P1 * H2p);
     if (!d->fold32 && d->gen0) hipMalloc(&d->Xzf, sizeof(cpx<float>) * 3L * P0 * P1 * H2p);
@@ -1377,8 +1407,8 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
             if (padded) hipMemsetAsync(d->kernL + c * noct, 0, sizeof(double) * noct, st);
         }
     }
-    if (d->fold32) fill_table<float>(d, d->kt32, d->fold32, st);
-    if (tab64) fill_table<double>(d, d->kt64, d->fold64, st);
+    if (d->fold32) fill_table<float>(d, d->kt32, d->fold32, d->form32, st);
+    if (tab64) fill_table<double>(d, d->kt64, d->fold64, d->form64, st);
     unsigned long long mb[2 * kExtractLanes];
     hipMemcpyAsync(mb, maxbits, sizeof(mb), hipMemcpyDeviceToHost, st);
     hipStreamSynchronize(st);
@@ -1496,7 +1526,7 @@ extern "C" int hs_demag_field_f64(hs_demag* d, const double* m, const double* ms
             return HS_ENOMEM;
         }
         if (tab) {  // ready for calls on any stream
-            fill_table<double>(d, d->kt64, d->fold64, hs::S(stream));
+            fill_table<double>(d, d->kt64, d->fold64, d->form64, hs::S(stream));
             hipStreamSynchronize(hs::S(stream));
         }
     }

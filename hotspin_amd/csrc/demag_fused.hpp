@@ -916,10 +916,24 @@ struct Mids {
 };
 inline int fold_index(int R) { return R == 1 ? 0 : (R == 2 ? 1 : (R == 4 ? 2 : 3)); }
 inline int table_rows_of(int Q, bool fold) { return table_rows(Q, fold); }
+// The kernels of one plan.
 template <typename T>
-Rows<T>& rows_of(int M);  // registries, defined in demag.hip
+struct Form {
+    frows_t<T> fwd = nullptr;
+    irows_t<T> inv = nullptr;
+    mid_t<T> mid = nullptr;
+    int A = 0, B = 0;  // split of the mid kernel's columns
+};
+// registries (demag.hip): the entry to fill at library load, and the entry of a
+// length for reading (an empty one if there is none)
 template <typename T>
-Mids<T>& mids_of(int Q);
+Rows<T>& add_rows_of(int M);
+template <typename T>
+Mids<T>& add_mids_of(int Q);
+template <typename T>
+const Rows<T>& rows_of(int M);
+template <typename T>
+const Mids<T>& mids_of(int Q);
 
 // Rows per block: full 128-byte pieces of a column (16 rows of 8 bytes) while
 // the tile stays near 32 KB; folded, 16 rows or as many as 72 KB hold, and in
@@ -981,7 +995,7 @@ void add_rows_fold(Rows<T>& r) {
 template <typename T, int M>
 void add_rows() {
     if constexpr (two_level_ok(M) && M >= 8) {
-        Rows<T>& r = rows_of<T>(M);
+        Rows<T>& r = add_rows_of<T>(M);
         add_rows_fold<T, M, 0>(r), add_rows_fold<T, M, 1>(r), add_rows_fold<T, M, 2>(r);
         if constexpr (sizeof(T) == 4) add_rows_fold<T, M, 3>(r);
     }
@@ -1004,7 +1018,7 @@ void add_mid_fold(Mids<T>& m) {
 template <typename T, int Q>
 void add_mid() {
     if constexpr (split_even(Q).A > 0) {
-        Mids<T>& m = mids_of<T>(Q);
+        Mids<T>& m = add_mids_of<T>(Q);
         m.A = split_even(Q).A;
         m.B = split_even(Q).B;
         add_mid_fold<T, Q, false>(m);

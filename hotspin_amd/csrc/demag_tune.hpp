@@ -36,7 +36,10 @@ struct Variants {
     std::vector<ColV> cols;
     std::vector<ZV> z;
 };
-Variants& variants(int L);  // registry (defined in demag.hip)
+// registry (demag.hip): the entry to fill at library load, and the entry of a
+// length for reading (an empty one if there is none)
+Variants& add_variants(int L);
+const Variants& variants(int L);
 
 constexpr long kLdsMax = 163840;
 constexpr int round64(int v) { return (v + 63) / 64 * 64; }
@@ -255,7 +258,7 @@ void add_z(Variants& v) {  // a block holds a pencil pair: 6W pencils
 
 template <int L>
 void register_size() {
-    Variants& v = variants(L);
+    Variants& v = add_variants(L);
     add_row<L, 2, 8>(v);
     add_row<L, 4, 8>(v);
     add_row<L, 8, 8>(v);

@@ -88,6 +88,11 @@ HS_API int hs_demag_tiles(const hs_demag* d, int* out6);
  * nothing and always give the same bits; HS_DEMAG_FORCE keeps a plan's FP32
  * field in the five passes. */
 HS_API int hs_demag_variant_count(const hs_demag* d, int* out3);
+/* Entries in the tables of compiled transform kernels that plans look their
+ * lengths up in.  They are filled when the library is loaded and never change
+ * afterwards, whatever lengths are asked for: threads that make plans and
+ * threads that evaluate fields read them without a lock. */
+HS_API int hs_demag_registered(void);
 /* B = mu0 * msat0T0Mul * (K conv (m .* msat0T0)), maxwell_convolution.go:103-131.
  * m, B: 3 device planes of N cells (m and B may not alias); msat0T0: device
  * mask or NULL.  FP64 variant: FP64 FFT passes; FP32 variant: FP32 passes. */
