@@ -53,8 +53,19 @@ bool HostStage::ready() {
     return true;
 }
 
+// Memory the runtime does not know: pinned, managed and device memory it copies
+// to directly.
+static bool pageable(const void* host) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, host) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
 hipError_t HostStage::out(void* host, const void* dev, size_t bytes, hipStream_t st) {
-    if (bytes >= kLeast && std::thread::hardware_concurrency() >= 2 * kWorkers) {
+    if (bytes >= kLeast && std::thread::hardware_concurrency() >= 2 * kWorkers && pageable(host)) {
         int device = -1;
         std::unique_lock<std::mutex> lk(mu_, std::try_to_lock);
         if (lk.owns_lock() && hipGetDevice(&device) == hipSuccess && device == device_ && ready())

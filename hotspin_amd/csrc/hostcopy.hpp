@@ -9,7 +9,9 @@
 // 19 MB.  A chunk costs about 16 us beside its transfer (4 workers, 100 MB:
 // 13.2 ms with 128 KB chunks, 4.8 with 512 KB, 2.8 with 2 MB), and 8 workers are
 // no faster than 4.  Uploads gain nothing below 32 MB (19 MB: 0.62 ms against
-// 0.54) and stay with the runtime.
+// 0.54) and stay with the runtime, and so do copies to pinned memory, which it
+// moves in one transfer (20 MB: 0.36 ms against 0.66 through the chunks, 106 MB:
+// 1.86 against 2.71).
 #pragma once
 
 #include <hip/hip_runtime.h>

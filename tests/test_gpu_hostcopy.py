@@ -52,3 +52,35 @@ def test_two_solvers_in_two_threads():
     assert not bad
     for s, _ in pair:
         s.close()
+
+
+def test_pinned_destination_is_one_transfer():
+    """A pinned destination takes the runtime's direct transfer: at 20 MB 0.36 ms
+    against 0.66 through the staging buffers, so 1.4 times torch's own copy of as
+    many bytes to the same buffer separates the two."""
+    import time
+
+    from hotspin_amd._lib import check, lib
+    from tests.gpu_util import torch
+
+    s, m = _solver(820)
+    pin = torch.empty(m.shape, dtype=torch.float64, pin_memory=True)
+    src = torch.zeros(m.shape, dtype=torch.float64, device="cuda")
+
+    def best(copy):
+        t = []
+        for _ in range(12):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            copy()
+            torch.cuda.synchronize()
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    plain = best(lambda: pin.copy_(src))
+    got = best(lambda: lib().hs_solver_get_m(s._h, pin.data_ptr()))
+    check("get_m to pinned memory")
+    assert np.array_equal(pin.numpy(), m)
+    print("20 MB to pinned memory: torch %.3f ms, get_m %.3f ms" % (plain * 1e3, got * 1e3))
+    assert got <= 1.4 * plain
+    s.close()
