@@ -65,7 +65,9 @@ static bool pageable(const void* host) {
 }
 
 hipError_t HostStage::out(void* host, const void* dev, size_t bytes, hipStream_t st) {
-    if (bytes >= kLeast && std::thread::hardware_concurrency() >= 2 * kWorkers && pageable(host)) {
+    // hipStreamPerThread would be another stream in each worker
+    if (bytes >= kLeast && st != hipStreamPerThread && std::thread::hardware_concurrency() >= 2 * kWorkers &&
+        pageable(host)) {
         int device = -1;
         std::unique_lock<std::mutex> lk(mu_, std::try_to_lock);
         if (lk.owns_lock() && hipGetDevice(&device) == hipSuccess && device == device_ && ready())

@@ -84,3 +84,22 @@ def test_pinned_destination_is_one_transfer():
     print("20 MB to pinned memory: torch %.3f ms, get_m %.3f ms" % (plain * 1e3, got * 1e3))
     assert got <= 1.4 * plain
     s.close()
+
+
+def test_state_of_a_solver_on_the_per_thread_stream():
+    """hipStreamPerThread (handle 2) names a different stream in every thread, so a
+    copy ordered on it cannot be shared out to workers; the state is whole after
+    a step enqueued on it."""
+    n = 1024 * 450
+    kw = dict(demag=0, exchange=1, lexMul=3e-9, longfield=0, msat0T0Mul=1e6, gammaLL=2.211e5, torque=1, zeeman=1,
+              Bext=(0.0, 0.1, 0.2))
+    m = np.random.default_rng(4).standard_normal((3, n))
+    m /= np.linalg.norm(m, axis=0)
+    out = []
+    for stream in (None, 2):
+        s = Solver((1, 450, 1024), (2e-9,) * 3, stream=stream, **kw)
+        s.set_m(m)
+        s.run("rk4", 5, 1e-15)
+        out.append(s.get_m())
+        s.close()
+    assert np.array_equal(out[0], out[1]) and not np.array_equal(out[0], m)
