@@ -794,7 +794,7 @@ template <typename T>
 int fused_fold(const hs_demag* d) {
     const int P1 = d->P[1], N0 = d->N[0];
     if (d->P[2] % 2 || P1 < 2 * d->N[1] || !(N0 == 1 || d->P[0] >= 2 * N0)) return 0;
-    return fused::mid_fold(N0, P1, sizeof(cpx<T>), [&](int R) {
+    return fused::mid_fold(N0, P1, sizeof(cpx<T>), std::equal(d->P, d->P + 3, d->logic), [&](int R) {
         const fused::Mids<T>& m = fused::mids_of<T>(P1 / R);
         return fused::rows_of<T>(d->M).fwd[fused::fold_index(R)] && m.A && m.pick(N0, R > 1) &&
                fused::mid_fits(N0, P1 / R, m.A, m.B, sizeof(cpx<T>));

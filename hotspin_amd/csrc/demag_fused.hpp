@@ -211,9 +211,9 @@ __device__ __forceinline__ void axis0(const Mid<T>& a, const G& g, cpx<T>* lds, 
 
 // One block: CB columns of one solve, 3 N0 pencils of Q points each, held in
 // LDS as lds[pencil * A (B+1) + k1 (B+1) + k2] (the odd row pitch keeps both
-// phases free of bank conflicts).  blockDim.x = elements / kEpt, rounded up
-// to whole waves.
-// Axis 0 in items of IB planes (MULTI: N0 > IB).
+// phases free of bank conflicts).  Axis 0 in items of IB planes (MULTI: N0 >
+// IB); blockDim.x gives a thread mid_itm(IB) items, 15 to 24 elements, rounded up
+// to whole waves (mid_nt).
 template <typename T, int Q, int IB, bool MULTI, bool FOLD>
 __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
     using G = Geom<Q, FOLD>;
@@ -859,24 +859,36 @@ constexpr long kTile = 3072;
 constexpr int kPlanes = 32;
 inline long mid_elems(size_t cs) { return kTile * 8 / (long)cs; }
 // Fold R of axis 1 for N0 planes and P1 points (fits(R): registered and a
-// column fits a block), 0 if none.  No folding up to 6144 elements a column
-// (FP64: 3072).  Beyond, a column leaves too few blocks a CU, and folding
-// until it has 3072 elements is best while the rows still leave in 64-byte
-// pieces (R <= 4: 42.4 us a field at 256x256x8 against 45.7 with R = 2 and
-// 48.3 without), else until it has 6144 (R = 8 at 512x512x16: 298 us, R = 16
-// with 16-byte pieces 334; five passes 317).  FP64 stops at R = 4: beyond, the
-// five passes are faster (512x512x16: 1050 us against 1127 with R = 16).
+// column fits a block; timed: the plan's five passes would be timed), 0 if
+// none.  No folding up to 6144 elements a column (FP64: 3072).  Beyond, a
+// column leaves too few blocks a CU, and folding until it has 3072 elements is
+// best while the rows still leave in 64-byte pieces (R <= 4: 42.4 us a field at
+// 256x256x8 against 45.7 with R = 2 and 48.3 without), else until it has 6144
+// (R = 8 at 512x512x16: 298 us, R = 16 with 16-byte pieces 334; five passes
+// 317) in blocks of at most 256 threads: five and six waves run badly (R = 4
+// with 320 threads against R = 8: 320x320x10 109 us a field against 87, five
+// passes 89; 128x128x26 70 against 54, five passes 55).
+// FP64 stops at R = 4, with which 256x256x8 leaves the five passes behind
+// (73 us against 96); beyond, it has no row kernels.
+// More than 16 planes on compiled lengths stay with the five passes rather
+// than fold.  One field, folded / five passes: 64x64x24 30.3 / 27.2 us,
+// 96x96x24 39.5 / 35.1, 256x64x20 46.0 / 39.2, 128x128x32 62.4 / 52.8; RK4 steps
+// of batches are between 0.9 (64x256x20) and 1.14 (512x64x24) times as long.
+// Without folding, batches decide: one field of 32^3 takes 25.1 us against
+// 20.3, but a step of 64 solves 729 us against 945.  A plan at padded lengths has
+// untimed passes, and folds (96x96x30: a step of 8 solves 789 us against 893).
 template <typename F>
-int mid_fold(int N0, int P1, size_t cs, F fits) {
+int mid_fold(int N0, int P1, size_t cs, bool timed, F fits) {
     const long el = kTile;
     if (N0 > kPlanes) return 0;
     auto ok = [&](int R, long most) { return P1 % R == 0 && 3L * N0 * (P1 / R) <= most && fits(R); };
     if (ok(1, cs == 8 ? 2 * el : el)) return 1;
+    if (cs == 8 && N0 > kPlanes / 2 && timed) return 0;
     for (int R = 2; R <= 4; R *= 2)
         if (ok(R, el)) return R;
     if (cs == 8)
         for (int R = 2; R <= 8; R *= 2)
-            if (ok(R, 2 * el)) return R;
+            if (mid_nt(N0, P1 / R, 1) <= 256 && ok(R, 2 * el)) return R;
     return ok(1, 1L << 40) ? 1 : 0;
 }
 // Columns per block: about kTile elements, fewer while the launch would leave
