@@ -769,22 +769,70 @@ bool set_lengths(hs_demag* d, const int P[3]) {
     const int lim = gen_max_len<double>();
     return d->gR.L <= lim && P1 <= lim && P0 <= lim;
 }
-// The shortest compiled length >= P, P itself if there is none.
+// Axis c of length L runs compiled kernels in FP32 and FP64.
+bool axis_compiled(int c, int L) {
+    if (c == 0) return z32_ok(L) && z64_ok(L);
+    return c == 1 ? cols32(L) && cols64(L) : rows32(L) && rows64(L);
+}
+// The shortest compiled length >= P of axis c, P itself if there is none.
 // An open axis is zero-padded, so any length from 2 N - 1 on gives the same
 // convolution.  2 N itself where it is compiled; otherwise the next of 2^k,
 // 3 2^k and 5 2^k costs at most 1.33 times the points and runs the compiled
 // kernels instead of the run-time-length ones (FP32 field, run-time lengths
 // against padded: 100x75x7 78 -> 20 us, 33^3 171 -> 25, 100^3 383 -> 222,
 // 300x300x33 2086 -> 334, 300x300x17 2502 -> 138; no mesh was slower).
-template <typename F>
-int compiled_length(int P, F ok) {
+int compiled_length(int c, int P) {
     int best = 0;
 #define X(n) \
     for (int L : {n, 2 * n}) \
-        if (L >= P && ok(L) && (!best || L < best)) best = L;
+        if (L >= P && axis_compiled(c, L) && (!best || L < best)) best = L;
     HS_FFT_SIZES(X)
 #undef X
     return best ? best : P;
+}
+// Relative time of the five passes of N at lengths P: points of each pass (rows
+// and axis 1 there and back, axis 0 with the product in one) times 2, and for a
+// run-time length 2 more for each stage of up to 8 points or R for a stage of a
+// prime R, which sums directly.
+double passes_cost(const int N[3], const int P[3]) {
+    auto len = [&](int c) {
+        if (axis_compiled(c, P[c])) return 2;
+        const GenFFT g = gen_fft_plan(c == 2 && P[2] % 2 == 0 ? P[2] / 2 : P[c]);
+        int t = 2;
+        for (int s = 0; s < g.nst; s++) t += g.r[s] <= 8 ? 2 : g.r[s];
+        return t;
+    };
+    const double H2 = P[2] / 2 + 1;
+    return 2.0 * N[0] * N[1] * (P[2] / 2) * len(2) + 2.0 * N[0] * P[1] * H2 * len(1) +
+           P[0] * P[1] * H2 * (2 * len(0) + 4);
+}
+// Lengths of the transforms: open axes at their next compiled length.  Where one
+// has none (more than 128 planes, more than 1024 rows, 2048 cells along x) its
+// run-time pass pays for the padding of the others, so only the axes are padded
+// with which passes_cost is least: 100x64x140 291 us a field at 2 N, 331 padded;
+// 49x49x130 301 / 383; but 16x37x140 511 / 63.  (Run-time lengths of
+// periodic axes do not count: at 60 such meshes padding the others was 9 %
+// slower at worst, in FP64, and up to 40 times faster.)
+void padded_lengths(const int N[3], const int logic[3], int P[3]) {
+    int full[3];
+    bool all = true;
+    for (int c = 0; c < 3; c++) {
+        const bool open = logic[c] > N[c];
+        full[c] = open ? compiled_length(c, logic[c]) : logic[c];
+        all = all && (!open || axis_compiled(c, full[c]));
+    }
+    std::copy(all ? full : logic, (all ? full : logic) + 3, P);
+    if (all) return;
+    double least = passes_cost(N, logic);
+    for (int s = 1; s < 8; s++) {
+        int Q[3];
+        for (int c = 0; c < 3; c++) Q[c] = s >> c & 1 ? full[c] : logic[c];
+        const double t = passes_cost(N, Q);
+        if (t < least) {
+            least = t;
+            std::copy(Q, Q + 3, P);
+        }
+    }
 }
 
 // Fold R of axis 1 with which the fused kernels take the mesh (mid_fold), 0 if
@@ -1288,11 +1336,8 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     }
     d->noalloc = noalloc_bytes(d, 0) <= kScratchBytes;
     if (pad) {
-        auto open = [&](int c) { return d->logic[c] > N[c]; };
-        const int P[3] = {
-            open(0) ? compiled_length(d->P[0], [](int L) { return z32_ok(L) && z64_ok(L); }) : d->P[0],
-            open(1) ? compiled_length(d->P[1], [](int L) { return cols32(L) && cols64(L); }) : d->P[1],
-            open(2) ? compiled_length(d->P[2], [](int L) { return rows32(L) && rows64(L); }) : d->P[2]};
+        int P[3];
+        padded_lengths(N, d->logic, P);
         set_lengths(d, P);
         if (d->noalloc && noalloc_bytes(d, fused_fold<double>(d)) > kScratchBytes) set_lengths(d, d->logic);
     }

@@ -54,3 +54,41 @@ def test_form_of_the_fp32_convolution(monkeypatch, N, five):
     d.close()
     # FP32 round-off of transforms of up to 2048 points and sums of up to 96 products
     assert relerr(own, want) <= 2e-6 and relerr(forced, want) <= 2e-6
+
+
+def _compiled(d):
+    """Which of the plan's row, column and axis-0 passes run compiled kernels."""
+    import ctypes as C
+    from hotspin_amd._lib import lib
+    cnt = (C.c_int * 3)()
+    assert lib().hs_demag_variant_count(d._h, cnt) == 0
+    return tuple(c > 0 for c in cnt)
+
+
+# an open axis without a compiled length (more than 128 planes, more than 1024 rows,
+# more than 2048 cells along x) beside others that have one at 2 N, could be padded to
+# one, or gain by it: (rows, columns, axis 0) compiled
+BESIDE_RUN_TIME = [((140, 64, 100), (False, True, False)), ((130, 49, 49), (False, False, False)),
+                   ((140, 16, 37), (True, True, False)), ((200, 20, 33), (True, True, False)),
+                   ((7, 1100, 49), (False, False, True)), ((3, 1300, 10), (True, False, True)),
+                   ((3, 37, 2100), (False, True, True)), ((129, 3, 4), (True, True, False))]
+
+
+@pytest.mark.parametrize("N,compiled", BESIDE_RUN_TIME)
+def test_padding_beside_a_run_time_length(N, compiled):
+    from oracle import pyoracle as po
+    n = N[0] * N[1] * N[2]
+    rng = np.random.default_rng(n)
+    m, msk = rng.standard_normal((3, n)), rng.random(n)
+    d, o = Demag(N, CELL), po.Demag(N, CELL)
+    assert d.P == o.P and d.K == o.K
+    assert _compiled(d) == compiled
+    assert relerr(d.kernel(), o.kernel()) <= 1e-12
+    want = o.B(m, msk, 8e5).reshape(3, n)
+    dm, dw, B = dev(m), dev(msk), empty((3, n))
+    d.field_f64(P(dm), P(dw), 8e5, P(B))
+    assert relerr(host(B), want) <= 1e-12
+    dm, dw, B = dev(m, np.float32), dev(msk, np.float32), empty((3, n), torch.float32)
+    d.field_f32(P(dm), P(dw), 8e5, P(B))
+    assert relerr(host(B), want) <= 2e-6
+    d.close()
