@@ -691,7 +691,7 @@ struct hs_demag {
     int KP;          // FP32 kernel row pitch (floats), a multiple of 32 = 128 bytes
     long ncell;
     double* kern64 = nullptr;
-    float* kern32 = nullptr;
+    float* kern32 = nullptr;  // the five FP32 passes' copy (fold32 = 0)
     cpx<float>*X1f = nullptr, *X2f = nullptr;
     cpx<double>*X1d = nullptr, *X2d = nullptr;
     cpx<float>*twMf = nullptr, *twP2f = nullptr, *tw1f = nullptr, *tw0f = nullptr;
@@ -1354,14 +1354,14 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     d->tw1d = make_twiddles<double>(P1);
     d->tw0d = make_twiddles<double>(P0);
     hipMalloc(&d->kern64, sizeof(double) * 6 * nk);
-    const long nk32 = (long)d->K[0] * d->K[1] * d->KP;
-    hipMalloc(&d->kern32, sizeof(float) * 6 * nk32);
-    if (d->kern32) hipMemsetAsync(d->kern32, 0, sizeof(float) * 6 * nk32, st);
     // HS_DEMAG_FORCE asks for particular five-pass variants
     d->fold32 = getenv("HS_DEMAG_FORCE") ? 0 : fused_fold<float>(d);
     d->fold64 = fused_fold<double>(d);
     d->form32 = fused_form<float>(d, d->fold32);
     d->form64 = fused_form<double>(d, d->fold64);
+    const long nk32 = (long)d->K[0] * d->K[1] * d->KP;
+    if (!d->fold32) hipMalloc(&d->kern32, sizeof(float) * 6 * nk32);
+    if (d->kern32) hipMemsetAsync(d->kern32, 0, sizeof(float) * 6 * nk32, st);
     hipMalloc(&d->X1f, sizeof(cpx<float>) * fused_spectrum(d, d->fold32));
     if (!d->fold32) hipMalloc(&d->X2f, sizeof(cpx<float>) * 3L * N[0] * P1 * H2p);
     if (!d->fold32 && d->gen0) hipMalloc(&d->Xzf, sizeof(cpx<float>) * 3L * P0 * P1 * H2p);
@@ -1393,8 +1393,8 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     hipMalloc(&X, sizeof(cpx<double>) * 6L * P0 * P1 * H2p);
     hipMalloc(&maxbits, 2 * kExtractLanes * sizeof(unsigned long long));
     if (padded) hipMalloc(&d->kernL, sizeof(double) * 6 * noct);
-    if (!oct || !full || !X || !maxbits || !d->kern64 || !d->kern32 || !d->X1f || (padded && !d->kernL) ||
-        (!d->fold32 && (!d->X2f || (d->gen0 && !d->Xzf))) || (d->fold32 && !d->kt32) || (tab64 && !d->kt64)) {
+    if (!oct || !full || !X || !maxbits || !d->kern64 || !d->X1f || (padded && !d->kernL) ||
+        (!d->fold32 && (!d->kern32 || !d->X2f || (d->gen0 && !d->Xzf))) || (d->fold32 && !d->kt32) || (tab64 && !d->kt64)) {
         hipFree(oct); hipFree(full); hipFree(X); hipFree(maxbits);
         hs_demag_destroy(d);
         (void)hipGetLastError();
@@ -1448,7 +1448,7 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     for (int c = 0; c < 6; c++) {
         if (gmax > 0 && cmax[c] / gmax < 1e-12) {
             hipMemsetAsync(d->kern64 + c * nk, 0, sizeof(double) * nk, st);
-            hipMemsetAsync(d->kern32 + c * nk32, 0, sizeof(float) * nk32, st);
+            if (d->kern32) hipMemsetAsync(d->kern32 + c * nk32, 0, sizeof(float) * nk32, st);
             if (padded) hipMemsetAsync(d->kernL + c * noct, 0, sizeof(double) * noct, st);
         }
     }
@@ -1667,17 +1667,17 @@ extern "C" int hs_demag_reserve(hs_demag* d, int nsolve) {
     return 0;
 }
 long hs_demag_ncell(const hs_demag* d) { return d->ncell; }
-// device bytes of the plan: kernel octant (FP64 + FP32), FP32 spectra of
-// `cap` solves, FP64 spectra when allocated, twiddle tables
+// device bytes of the plan: kernel octant (FP64; FP32 for the five passes) and
+// tables, FP32 spectra of `cap` solves, FP64 spectra when allocated, twiddle tables
 long hs_demag_footprint(const hs_demag* d) {
     const long nk = (long)d->K[0] * d->K[1] * d->K[2];
-    long b = 6 * nk * (sizeof(double) + sizeof(float));
+    long b = 6 * nk * (long)sizeof(double);
+    if (d->kern32) b += 6L * d->K[0] * d->K[1] * d->KP * (long)sizeof(float);
     b += (long)sizeof(cpx<float>) * (fused_spectrum(d, d->fold32) + (d->X2f ? 3L * d->N[0] * d->P[1] * d->H2p : 0)) *
          d->cap;
     if (d->kernL) b += 6L * d->logicK[0] * d->logicK[1] * d->logicK[2] * (long)sizeof(double);
     if (d->kt32) b += fused_table(d, d->fold32) * (long)sizeof(float);
     if (d->kt64) b += fused_table(d, d->fold64) * (long)sizeof(double);
-    b += 6L * d->K[0] * d->K[1] * (d->KP - d->H2) * (long)sizeof(float);
     if (d->X1d)
         b += (long)sizeof(cpx<double>) * (fused_spectrum(d, d->fold64) + (d->X2d ? 3L * d->N[0] * d->P[1] * d->H2p : 0));
     if (d->Xzf) b += (long)sizeof(cpx<float>) * 3L * d->P[0] * d->P[1] * d->H2p * d->cap;

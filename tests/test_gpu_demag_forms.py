@@ -92,3 +92,18 @@ def test_padding_beside_a_run_time_length(N, compiled):
     d.field_f32(P(dm), P(dw), 8e5, P(B))
     assert relerr(host(B), want) <= 2e-6
     d.close()
+
+
+# three-kernel meshes beyond the size whose FP64 table is kept for hs_demag_field_f64_noalloc
+@pytest.mark.parametrize("N", [(8, 256, 256), (1, 1024, 1024), (2, 640, 640), (16, 512, 512)])
+def test_three_kernel_plan_holds_no_five_pass_kernel(monkeypatch, N):
+    """The footprint by which requests are admitted is no larger than with the five
+    passes, whose FP32 kernel octant (16 to 114 MB here) nothing reads."""
+    from hotspin_amd.api import SlotBatch
+    kw = dict(msat0T0Mul=1e6, demag=1, gammaLL=2.211e5, torque=1)
+    own = SlotBatch(N, CELL, 1, **kw)
+    monkeypatch.setenv("HS_DEMAG_FORCE", "-1,-1,-1")
+    five = SlotBatch(N, CELL, 1, **kw)
+    assert own.footprint() <= five.footprint()
+    own.close()
+    five.close()
