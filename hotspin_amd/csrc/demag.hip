@@ -661,19 +661,6 @@ zconv_t<T, TK> pick_zconv(int L) {
     return nullptr;
 }
 
-template <typename T>
-cpx<T>* make_twiddles(int L) {
-    std::vector<cpx<T>> h(L > 0 ? L : 1);
-    for (int t = 0; t < L; t++) {
-        long double a = -2.0L * 3.14159265358979323846264338327950288L * (long double)t / (long double)L;
-        h[t] = {(T)cosl(a), (T)sinl(a)};
-    }
-    cpx<T>* d = nullptr;
-    if (hipMalloc(&d, sizeof(cpx<T>) * h.size()) != hipSuccess) return nullptr;
-    hipMemcpy(d, h.data(), sizeof(cpx<T>) * h.size(), hipMemcpyHostToDevice);
-    return d;
-}
-
 }  // namespace
 
 // ------------------------------------------------------------------ plan
@@ -696,6 +683,7 @@ struct hs_demag {
     cpx<double>*X1d = nullptr, *X2d = nullptr;
     cpx<float>*twMf = nullptr, *twP2f = nullptr, *tw1f = nullptr, *tw0f = nullptr;
     cpx<double>*twMd = nullptr, *twP2d = nullptr, *tw1d = nullptr, *tw0d = nullptr;
+    unsigned char* tw = nullptr;  // the tables above
     double max_imag_ratio = 0;
     // FP32 pass variants chosen by timing at plan creation
     hsdm::RowV row32{};   // forward (R2C) row pass
@@ -768,6 +756,36 @@ bool set_lengths(hs_demag* d, const int P[3]) {
     d->g0 = gen_fft_plan(P0);
     const int lim = gen_max_len<double>();
     return d->gR.L <= lim && P1 <= lim && P0 <= lim;
+}
+size_t up256(size_t b) { return (b + 255) / 256 * 256; }
+// The roots exp(-2 pi i t / L) of the plan's lengths, FP64 and (f32) FP32, in one
+// allocation and one copy; false without memory.
+bool make_twiddles(hs_demag* d, bool f32) {
+    const int L[4] = {d->M, d->P[2], d->P[1], d->P[0]};
+    cpx<double>** pd[4] = {&d->twMd, &d->twP2d, &d->tw1d, &d->tw0d};
+    cpx<float>** pf[4] = {&d->twMf, &d->twP2f, &d->tw1f, &d->tw0f};
+    size_t at[5] = {0};  // an FP64 table, then its FP32 copy
+    for (int k = 0; k < 4; k++)
+        at[k + 1] = at[k] + up256(sizeof(cpx<double>) * (L[k] + 1)) + (f32 ? up256(sizeof(cpx<float>) * (L[k] + 1)) : 0);
+    if (hipMalloc(&d->tw, at[4]) != hipSuccess) {
+        d->tw = nullptr;
+        return false;
+    }
+    std::vector<unsigned char> host(at[4]);
+    for (int k = 0; k < 4; k++) {
+        const size_t f = at[k] + up256(sizeof(cpx<double>) * (L[k] + 1));
+        cpx<double>* hd = reinterpret_cast<cpx<double>*>(&host[at[k]]);
+        cpx<float>* hf = f32 ? reinterpret_cast<cpx<float>*>(&host[f]) : nullptr;
+        for (int t = 0; t < L[k]; t++) {
+            const long double a = -2.0L * 3.14159265358979323846264338327950288L * (long double)t / (long double)L[k];
+            const long double c = cosl(a), s = sinl(a);
+            hd[t] = {(double)c, (double)s};
+            if (hf) hf[t] = {(float)c, (float)s};
+        }
+        *pd[k] = reinterpret_cast<cpx<double>*>(d->tw + at[k]);
+        if (f32) *pf[k] = reinterpret_cast<cpx<float>*>(d->tw + f);
+    }
+    return hipMemcpy(d->tw, host.data(), at[4], hipMemcpyHostToDevice) == hipSuccess;
 }
 // Axis c of length L runs compiled kernels in FP32 and FP64.
 bool axis_compiled(int c, int L) {
@@ -1265,7 +1283,6 @@ constexpr size_t kScratchBytes = size_t(64) << 20;
 // FP64 spectra of one solve of the plan's mesh: X1, then X2 and (run-time
 // axis-0 length only) Xz, each from a 256-byte boundary; fused: X alone
 size_t x_bytes(const hs_demag* d, int rows) { return sizeof(cpx<double>) * 3ull * rows * d->P[1] * d->H2p; }
-size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 size_t noalloc_bytes(const hs_demag* d, int fold) {
     if (fold) return sizeof(cpx<double>) * (size_t)fused_spectrum(d, fold);
     const size_t x1 = sizeof(cpx<double>) * 3ull * d->N[0] * d->N[1] * d->H2p;
@@ -1344,15 +1361,14 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     const int P0 = d->P[0], P1 = d->P[1], P2 = d->P[2], H2 = d->H2, H2p = d->H2p, M = d->M;
     const bool padded = P0 != d->logic[0] || P1 != d->logic[1] || P2 != d->logic[2];
     const long nk = (long)d->K[0] * d->K[1] * d->K[2];
-    // twiddles
-    d->twMf = make_twiddles<float>(M);
-    d->twP2f = make_twiddles<float>(P2);
-    d->tw1f = make_twiddles<float>(P1);
-    d->tw0f = make_twiddles<float>(P0);
-    d->twMd = make_twiddles<double>(M);
-    d->twP2d = make_twiddles<double>(P2);
-    d->tw1d = make_twiddles<double>(P1);
-    d->tw0d = make_twiddles<double>(P0);
+    bool tables = make_twiddles(d, true);
+    hs_demag l;  // the transform at the logic size, for hs_demag_kernel_f64 alone
+    if (padded) {
+        std::copy(d->logic, d->logic + 3, l.logic);
+        std::copy(d->logicK, d->logicK + 3, l.logicK);
+        set_lengths(&l, d->logic);
+        tables = make_twiddles(&l, false) && tables;
+    }
     hipMalloc(&d->kern64, sizeof(double) * 6 * nk);
     // HS_DEMAG_FORCE asks for particular five-pass variants
     d->fold32 = getenv("HS_DEMAG_FORCE") ? 0 : fused_fold<float>(d);
@@ -1393,9 +1409,9 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     hipMalloc(&X, sizeof(cpx<double>) * 6L * P0 * P1 * H2p);
     hipMalloc(&maxbits, 2 * kExtractLanes * sizeof(unsigned long long));
     if (padded) hipMalloc(&d->kernL, sizeof(double) * 6 * noct);
-    if (!oct || !full || !X || !maxbits || !d->kern64 || !d->X1f || (padded && !d->kernL) ||
+    if (!tables || !oct || !full || !X || !maxbits || !d->kern64 || !d->X1f || (padded && !d->kernL) ||
         (!d->fold32 && (!d->kern32 || !d->X2f || (d->gen0 && !d->Xzf))) || (d->fold32 && !d->kt32) || (tab64 && !d->kt64)) {
-        hipFree(oct); hipFree(full); hipFree(X); hipFree(maxbits);
+        hipFree(oct); hipFree(full); hipFree(X); hipFree(maxbits); hipFree(l.tw);
         hs_demag_destroy(d);
         (void)hipGetLastError();
         if (padded) return demag_create(N, cell, pbc, accuracy, kernel, stream, false);
@@ -1433,17 +1449,9 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     const KernelBufs kb{oct, full, X, maxbits};
     kernel_transform(d, kb, d->kern64, d->kern32, st);
     if (padded) {
-        hs_demag l;  // the transform at the logic size, for hs_demag_kernel_f64 alone
-        std::copy(d->logic, d->logic + 3, l.logic);
-        std::copy(d->logicK, d->logicK + 3, l.logicK);
-        set_lengths(&l, d->logic);
-        l.twMd = make_twiddles<double>(l.M);
-        l.twP2d = make_twiddles<double>(l.P[2]);
-        l.tw1d = make_twiddles<double>(l.P[1]);
-        l.tw0d = make_twiddles<double>(l.P[0]);
         kernel_transform(&l, kb, d->kernL, nullptr, st);
         hipStreamSynchronize(st);
-        for (void* p : {l.twMd, l.twP2d, l.tw1d, l.tw0d}) hipFree(p);
+        hipFree(l.tw);
     }
     for (int c = 0; c < 6; c++) {
         if (gmax > 0 && cmax[c] / gmax < 1e-12) {
@@ -1490,8 +1498,8 @@ extern "C" hs_demag* hs_demag_create_newell(const int N[3], const double cell[3]
 
 extern "C" void hs_demag_destroy(hs_demag* d) {
     if (!d) return;
-    void* ps[] = {d->kernL,  d->kt32,   d->kt64,   d->kern64, d->kern32, d->X1f, d->X2f, d->X1d, d->X2d, d->twMf, d->twP2f,
-                  d->tw1f,   d->tw0f,   d->twMd, d->twP2d, d->tw1d, d->tw0d, d->Xzf, d->Xzd};
+    void* ps[] = {d->kernL, d->kt32, d->kt64, d->kern64, d->kern32, d->X1f, d->X2f,
+                  d->X1d,   d->X2d,  d->Xzf,  d->Xzd,    d->tw};
     for (void* p : ps)
         if (p) hipFree(p);
     delete d;
