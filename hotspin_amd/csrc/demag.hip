@@ -1519,7 +1519,11 @@ extern "C" int hs_demag_kernel_f64(const hs_demag* d, double* host_out) {
     long nk = (long)d->logicK[0] * d->logicK[1] * d->logicK[2];
     const double* k = d->kernL ? d->kernL : d->kern64;
     const std::shared_ptr<HostStage> stage = HostStage::get();
-    const hipError_t e = stage ? stage->out(host_out, k, sizeof(double) * 6 * nk, nullptr)
+    // a plan is read once: with no solver alive, fresh buffers cost more than they give
+    // up to 29 MB (64^3, 13 MB, 2.5 ms against the runtime's 0.75; 256x256x8, 29 MB, 0.9
+    // or, where their pages are pinned anew, 2.8 against 1.6; 256x256x16, 53 MB, 1.9
+    // against 5.2)
+    const hipError_t e = stage ? stage->out(host_out, k, sizeof(double) * 6 * nk, nullptr, size_t(48) << 20)
                                : hipMemcpy(host_out, k, sizeof(double) * 6 * nk, hipMemcpyDeviceToHost);
     return e == hipSuccess ? 0 : (int)e;
 }

@@ -64,13 +64,14 @@ static bool pageable(const void* host) {
     return a.type == hipMemoryTypeUnregistered;
 }
 
-hipError_t HostStage::out(void* host, const void* dev, size_t bytes, hipStream_t st) {
+hipError_t HostStage::out(void* host, const void* dev, size_t bytes, hipStream_t st, size_t worth) {
     // hipStreamPerThread would be another stream in each worker
     if (bytes >= kLeast && st != hipStreamPerThread && std::thread::hardware_concurrency() >= 2 * kWorkers &&
         pageable(host)) {
         int device = -1;
         std::unique_lock<std::mutex> lk(mu_, std::try_to_lock);
-        if (lk.owns_lock() && hipGetDevice(&device) == hipSuccess && device == device_ && ready())
+        if (lk.owns_lock() && hipGetDevice(&device) == hipSuccess && device == device_ && (pin_ || bytes >= worth) &&
+            ready())
             return staged(static_cast<unsigned char*>(host), static_cast<const unsigned char*>(dev), bytes, st);
     }
     const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);

@@ -26,8 +26,10 @@ class HostStage {
     HostStage& operator=(const HostStage&) = delete;
     ~HostStage();
     // Copies in order on st (a stream of the current device) and returns when
-    // the host memory is written.
-    hipError_t out(void* host, const void* dev, size_t bytes, hipStream_t st);
+    // the host memory is written.  Makes the buffers if there are none yet and the
+    // copy has `worth` bytes: fresh ones cost up to 2 ms where the runtime has
+    // to pin their pages, which a solver's many reads pay once.
+    hipError_t out(void* host, const void* dev, size_t bytes, hipStream_t st, size_t worth = 0);
     // The current device's stage, one for all who hold it (the buffers, 16 MB,
     // go when the last lets go); null if there is none to be had.
     static std::shared_ptr<HostStage> get();
