@@ -1399,19 +1399,21 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     }
     if (Lg[2] == 1 && d->pbc[2] == 0) r2[2] = 0;
     const long noct = (long)LK[0] * LK[1] * LK[2];
-    double* oct = nullptr;
-    double* full = nullptr;
-    cpx<double>* X = nullptr;
-    unsigned long long* maxbits = nullptr;
     const long P = (long)P0 * P1 * P2;  // no length of `logic` is longer
-    hipMalloc(&oct, sizeof(double) * 6 * noct);
-    hipMalloc(&full, sizeof(double) * 6 * P);
-    hipMalloc(&X, sizeof(cpx<double>) * 6L * P0 * P1 * H2p);
-    hipMalloc(&maxbits, 2 * kExtractLanes * sizeof(unsigned long long));
+    // the temporaries in one allocation: each further one of some MB takes up to 0.2 ms to free
+    const size_t boct = up256(sizeof(double) * 6 * noct), bfull = up256(sizeof(double) * 6 * P),
+                 bX = up256(sizeof(cpx<double>) * 6L * P0 * P1 * H2p);
+    unsigned char* tmp = nullptr;
+    hipMalloc(&tmp, boct + bfull + bX + 2 * kExtractLanes * sizeof(unsigned long long));
+    double* const oct = reinterpret_cast<double*>(tmp);
+    double* const full = reinterpret_cast<double*>(tmp + boct);
+    cpx<double>* const X = reinterpret_cast<cpx<double>*>(tmp + boct + bfull);
+    unsigned long long* const maxbits = reinterpret_cast<unsigned long long*>(tmp + boct + bfull + bX);
     if (padded) hipMalloc(&d->kernL, sizeof(double) * 6 * noct);
-    if (!tables || !oct || !full || !X || !maxbits || !d->kern64 || !d->X1f || (padded && !d->kernL) ||
+    if (!tables || !tmp || !d->kern64 || !d->X1f || (padded && !d->kernL) ||
         (!d->fold32 && (!d->kern32 || !d->X2f || (d->gen0 && !d->Xzf))) || (d->fold32 && !d->kt32) || (tab64 && !d->kt64)) {
-        hipFree(oct); hipFree(full); hipFree(X); hipFree(maxbits); hipFree(l.tw);
+        hipFree(tmp);
+        hipFree(l.tw);
         hs_demag_destroy(d);
         (void)hipGetLastError();
         if (padded) return demag_create(N, cell, pbc, accuracy, kernel, stream, false);
@@ -1474,10 +1476,7 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
         mr = fmax(mr, b);
     }
     d->max_imag_ratio = mr > 0 ? mi / mr : 0;
-    hipFree(oct);
-    hipFree(full);
-    hipFree(X);
-    hipFree(maxbits);
+    hipFree(tmp);
     tune32(d, st);
     HS_LAUNCH_CHECK("hs_demag_create");
     if (hs_last_error()) {

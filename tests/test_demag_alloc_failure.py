@@ -71,7 +71,8 @@ def plan(N, lo, hi):
     return out
 for N in {meshes!r}:
     d, err, n, _ = plan(N, -1, -1)
-    assert d and not err and n >= 8, (N, err, n)
+    # each allocation of some MB costs up to 0.2 ms: tables, octants, spectra and one for all temporaries
+    assert d and not err and 5 <= n <= 8, (N, err, n)
     for k in range(n):  # from allocation k on: the retry of a padded plan at its logic size fails too
         d, err, _, launches = plan(N, k, 1 << 30)
         assert not d and err == 10004 and launches == 0, (N, k, err, launches)
