@@ -1056,19 +1056,24 @@ void tune32(hs_demag* d, hipStream_t st) {
     // a plan with a run-time-length pass keeps the first variant of its compiled
     // passes
     if (!d->row32.r2c || !d->col32.fwd || !d->z32.fn) return;
-    // a plan at longer lengths than its logic size is not timed (0.3 s, which
-    // meshes of any size would pay each for themselves).  It takes what the
-    // timing picks at twelve shapes of 40 to 128 planes, or what came within a few
-    // per cent of it: the last rows (two-level, eight a block), two-level
-    // columns of 16 and, up to 128 points of axis 0, four lanes a pencil (the last
-    // but one); the last beyond.  50x50x49 40 us a field against 55 with the
-    // first variants, 100x100x36 66 / 90, 300x300x33 334 / 490.
+    // A plan at longer lengths than its logic size is not timed (0.3 s, which
+    // meshes of any size would pay each for themselves).  It takes two-level rows
+    // and columns, eight to a block (sixteen where eight make less than a wave), and
+    // four lanes a pencil on axis 0 (one lane below 16 points); where a length has
+    // none, the last variant, radix stages.  One field in us with these columns,
+    // sixteen to a block, and the radix stages: 50x50x49 36.3, 36.9, 38.8;
+    // 100x100x36 60.5, 58.6, 64.2; 190x190x33 121, 124, 141; 300x300x33 299, 333,
+    // 327 (490 with the first variant of each pass).  Axis 0 with the others it has:
+    // 100x100x36 63 against 68 to 125, periodic 100x100x16 41 against 39 to 53.
     if (d->kernL) {
-        d->row32 = d->rowi32 = vr.rows.back();
-        const int nt = 16 * split2(d->P[1]).B;
-        auto c = std::find_if(vc.cols.begin(), vc.cols.end(), [&](const hsdm::ColV& v) { return v.W == 16 && v.NT == nt; });
-        if (c != vc.cols.end()) d->col32 = *c;
-        d->z32 = vz.z[d->P[0] <= 128 && vz.z.size() > 1 ? vz.z.size() - 2 : vz.z.size() - 1];
+        using hsdm::Kind;
+        auto pick = [](const auto& list, Kind kind, int W) {
+            const auto* v = hsdm::find_variant(list, kind, W);
+            return v ? *v : list.back();
+        };
+        d->row32 = d->rowi32 = pick(vr.rows, Kind::two_level, 8);
+        d->col32 = pick(vc.cols, Kind::two_level, 8);
+        d->z32 = d->P[0] < 16 ? pick(vz.z, Kind::lane_nt, 32) : pick(vz.z, Kind::lanes4, 8);
         apply_force(d, vr, vc, vz);
         return;
     }

@@ -18,16 +18,24 @@ using cols32_t = void (*)(const cpx<float>*, cpx<float>*, Geo, Geo, int, int, in
                           hipStream_t, Live);
 using z32_t = void (*)(cpx<float>*, const float*, int, int, int, int, int, int, float, const cpx<float>*,
                        hipStream_t, int, Live);
+// what a variant runs: the radix stages of demag_kernels.hpp, or of fft2.hpp the
+// two-level register transforms (whole, of half length, with a split or padded
+// exchange) and axis 0 with one, two or four lanes a pencil (one: plain, product in
+// halves, also in 128 registers, non-temporal)
+enum class Kind { stages, two_level, half, split, padded, lane, lane_halves, lane_halves128, lane_nt, lanes2, lanes4 };
 struct RowV {
+    Kind kind;
     int W, NT;
     r2c32_t r2c;
     c2r32_t c2r;
 };
 struct ColV {
+    Kind kind;
     int W, NT;
     cols32_t fwd, inv;
 };
 struct ZV {
+    Kind kind;
     int W, NT;
     z32_t fn;
 };
@@ -40,6 +48,14 @@ struct Variants {
 // length for reading (an empty one if there is none)
 Variants& add_variants(int L);
 const Variants& variants(int L);
+// The variant of a kind with W pencils a block, else the last of that kind, else null.
+template <typename V>
+const V* find_variant(const std::vector<V>& list, Kind kind, int W) {
+    const V* found = nullptr;
+    for (const V& v : list)
+        if (v.kind == kind && (!found || found->W != W)) found = &v;
+    return found;
+}
 
 constexpr long kLdsMax = 163840;
 constexpr int round64(int v) { return (v + 63) / 64 * 64; }
@@ -82,12 +98,12 @@ void launch_cols2_32(const cpx<float>* in, cpx<float>* out, Geo gi, Geo go, int 
 template <int M, int W, int E>
 void add_row(Variants& v) {
     constexpr int NT = clamp_nt((long)M * W / E);
-    if constexpr ((long)(M + 1) * W * 8 <= kLdsMax) v.rows.push_back({W, NT, &launch_r2c32<M, W, NT>, &launch_c2r32<M, W, NT>});
+    if constexpr ((long)(M + 1) * W * 8 <= kLdsMax) v.rows.push_back({Kind::stages, W, NT, &launch_r2c32<M, W, NT>, &launch_c2r32<M, W, NT>});
 }
 template <int L, int W, int E>
 void add_col(Variants& v) {
     constexpr int NT = clamp_nt((long)L * W / E);
-    if constexpr ((long)L * W * 8 <= kLdsMax) v.cols.push_back({W, NT, &launch_cols32<L, -1, W, NT>, &launch_cols32<L, 1, W, NT>});
+    if constexpr ((long)L * W * 8 <= kLdsMax) v.cols.push_back({Kind::stages, W, NT, &launch_cols32<L, -1, W, NT>, &launch_cols32<L, 1, W, NT>});
 }
 template <int L, int W>
 void launch_z2_32(cpx<float>* X, const float* kern, int N0, int P1, int H2, int H2p, int K1, int kp, float srcMul,
@@ -100,7 +116,7 @@ void launch_z2_32(cpx<float>* X, const float* kern, int N0, int P1, int H2, int 
 template <int L, int W>
 void add_z2(Variants& v) {
     if constexpr (reg_dft_ok(L) && L > 1 && L <= 64 && (long)L * 6 * W * 8 <= kLdsMax)
-        v.z.push_back({W, 6 * W, &launch_z2_32<L, W>});
+        v.z.push_back({Kind::lane, W, 6 * W, &launch_z2_32<L, W>});
 }
 
 // the same with the kernel product in two real halves (fft2.hpp k_zconv2s)
@@ -122,12 +138,12 @@ void launch_z2s4_32(cpx<float>* X, const float* kern, int N0, int P1, int H2, in
 template <int L, int W>
 void add_z2s4(Variants& v) {
     if constexpr (reg_dft_ok(L) && L > 1 && L <= 64 && (long)L * 6 * W * 4 <= kLdsMax)
-        v.z.push_back({W, 6 * W, &launch_z2s4_32<L, W>});
+        v.z.push_back({Kind::lane_halves128, W, 6 * W, &launch_z2s4_32<L, W>});
 }
 template <int L, int W>
 void add_z2s(Variants& v) {
     if constexpr (reg_dft_ok(L) && L > 1 && L <= 64 && (long)L * 6 * W * 4 <= kLdsMax)
-        v.z.push_back({W, 6 * W, &launch_z2s_32<L, W>});
+        v.z.push_back({Kind::lane_halves, W, 6 * W, &launch_z2s_32<L, W>});
 }
 
 // the same with non-temporal pencil loads and stores (fft2.hpp k_zconv2n)
@@ -141,7 +157,7 @@ void launch_z2n_32(cpx<float>* X, const float* kern, int N0, int P1, int H2, int
 template <int L, int W>
 void add_z2n(Variants& v) {
     if constexpr (reg_dft_ok(L) && L > 1 && L <= 64 && (long)L * 6 * W * 8 <= kLdsMax)
-        v.z.push_back({W, 6 * W, &launch_z2n_32<L, W>});
+        v.z.push_back({Kind::lane_nt, W, 6 * W, &launch_z2n_32<L, W>});
 }
 
 // the same with Q = 2 or 4 lanes per pencil, L = Q H with 4 <= H <= 32
@@ -157,7 +173,7 @@ template <int L, int W, int Q>
 void add_z2m(Variants& v) {
     if constexpr (L % Q == 0 && L / Q >= 4 && L / Q <= 32 && L >= 16 && reg_dft_ok(L / Q) &&
                   (long)L * 6 * W * 8 <= kLdsMax && 6 * Q * W <= 1024)
-        v.z.push_back({W, 6 * Q * W, &launch_z2m_32<L, W, Q>});
+        v.z.push_back({Q == 2 ? Kind::lanes2 : Kind::lanes4, W, 6 * Q * W, &launch_z2m_32<L, W, Q>});
 }
 
 // two-level register FFT columns (fft2.hpp): W columns, W * B threads
@@ -166,7 +182,7 @@ void add_col2(Variants& v) {
     if constexpr (two_level_ok(L) && L > 1) {
         constexpr int NT = W * split2(L).B;
         if constexpr ((long)(L * W + L) * 8 <= kLdsMax && NT >= 64 && NT <= 1024)
-            v.cols.push_back({W, NT, &launch_cols2_32<L, -1, W>, &launch_cols2_32<L, 1, W>});
+            v.cols.push_back({Kind::two_level, W, NT, &launch_cols2_32<L, -1, W>, &launch_cols2_32<L, 1, W>});
     }
 }
 
@@ -183,7 +199,7 @@ void add_col2s(Variants& v) {
     if constexpr (two_level_ok(L) && L > 1) {
         constexpr int NT = W * split2(L).B;
         if constexpr ((long)L * W * 4 + (long)L * 8 <= kLdsMax && NT >= 64 && NT <= 1024)
-            v.cols.push_back({W, NT, &launch_cols2s_32<L, -1, W>, &launch_cols2s_32<L, 1, W>});
+            v.cols.push_back({Kind::split, W, NT, &launch_cols2s_32<L, -1, W>, &launch_cols2s_32<L, 1, W>});
     }
 }
 
@@ -201,7 +217,7 @@ void add_col2p(Variants& v) {
         constexpr int NT = W * split2(L).B;
         if constexpr ((long)split2(L).A * (split2(L).B * W + W) * 4 + (long)L * 8 <= kLdsMax && NT >= 64 &&
                       NT <= 1024)
-            v.cols.push_back({W, NT, &launch_cols2p_32<L, -1, W>, &launch_cols2p_32<L, 1, W>});
+            v.cols.push_back({Kind::padded, W, NT, &launch_cols2p_32<L, -1, W>, &launch_cols2p_32<L, 1, W>});
     }
 }
 // half-length column pass (fft2.hpp k_cols2h) for a zero-padded axis: the
@@ -224,7 +240,7 @@ void add_col2h(Variants& v) {
     if constexpr (L % 2 == 0 && L >= 4 && two_level_ok(L) && two_level_ok(L / 2)) {
         constexpr int NTh = W * split2(L / 2).B, NT = W * split2(L).B;
         if constexpr ((long)(L * W + L) * 8 <= kLdsMax && NTh >= 64 && NTh <= 1024 && NT >= 64 && NT <= 1024)
-            v.cols.push_back({W, NTh, &launch_cols2h_32<L, -1, W>, &launch_cols2h_32<L, 1, W>});
+            v.cols.push_back({Kind::half, W, NTh, &launch_cols2h_32<L, -1, W>, &launch_cols2h_32<L, 1, W>});
     }
 }
 
@@ -246,14 +262,14 @@ void add_row2(Variants& v) {
     if constexpr (two_level_ok(M) && M > 1) {
         constexpr int NT = W * split2(M).B;
         if constexpr (((long)rows2_lds<M, W>() + 2L * M) * 8 <= kLdsMax && NT >= 64 && NT <= 1024)
-            v.rows.push_back({W, NT, &launch_r2c2_32<M, W>, &launch_c2r2_32<M, W>});
+            v.rows.push_back({Kind::two_level, W, NT, &launch_r2c2_32<M, W>, &launch_c2r2_32<M, W>});
     }
 }
 
 template <int L, int W, int E>
 void add_z(Variants& v) {  // a block holds a pencil pair: 6W pencils
     constexpr int NT = clamp_nt((long)L * 6 * W / E);
-    if constexpr (L <= 256 && (long)L * 6 * W * 8 <= kLdsMax) v.z.push_back({W, NT, &launch_z32<L, W, NT>});
+    if constexpr (L <= 256 && (long)L * 6 * W * 8 <= kLdsMax) v.z.push_back({Kind::stages, W, NT, &launch_z32<L, W, NT>});
 }
 
 template <int L>

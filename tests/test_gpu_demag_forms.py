@@ -107,3 +107,26 @@ def test_three_kernel_plan_holds_no_five_pass_kernel(monkeypatch, N):
     assert own.footprint() <= five.footprint()
     own.close()
     five.close()
+
+
+# padded plans in five passes: the tiles (pencils a block, threads) of two-level rows,
+# two-level columns and the axis-0 pass with four lanes a pencil, one lane below 16 points
+@pytest.mark.parametrize("N,pbc,tiles", [((36, 100, 100), (0, 0, 0), [8, 128, 8, 128, 8, 192]),
+                                         ((33, 33, 31), (0, 0, 0), [8, 64, 8, 80, 8, 192]),
+                                         ((40, 129, 129), (0, 0, 0), [8, 128, 8, 160, 8, 192]),
+                                         ((33, 300, 70), (0, 0, 0), [8, 80, 8, 256, 8, 192]),
+                                         ((8, 190, 100), (1, 0, 0), [8, 128, 8, 192, 32, 192])])
+def test_fixed_variants_of_padded_five_pass_plans(N, pbc, tiles):
+    import ctypes as C
+    from hotspin_amd._lib import lib
+    n = N[0] * N[1] * N[2]
+    d, t = Demag(N, CELL, pbc), (C.c_int * 6)()
+    assert lib().hs_demag_tiles(d._h, t) == 0
+    assert list(t) == tiles
+    m = np.random.default_rng(n).standard_normal((3, n))
+    dm, B = dev(m), empty((3, n))
+    d.field_f64(P(dm), None, 8e5, P(B))
+    m32, Bf = dev(m, np.float32), empty((3, n), torch.float32)
+    d.field_f32(P(m32), None, 8e5, P(Bf))
+    assert relerr(host(Bf), host(B)) <= 2e-6  # FP32 round-off of transforms of up to 1280 points
+    d.close()
