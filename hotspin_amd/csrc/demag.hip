@@ -529,8 +529,12 @@ namespace {
 // - rows (33 MB): R2C 14.8 / 9.9 us at M = 64, 19.1 / 11.4 at 256, 16.2 / 13.3
 //   at 512; C2R 12.7 / 8.0, 17.0 / 8.8, 15.7 / 9.4; M = 1024 15.0 / 25.5.
 //   Eight rows a block (16 where eight give less than a wave), four from 384
-//   points on (R2C at 384 with eight 24.7 against 13.5) except for R2C at 512,
-//   which keeps its occupancy with eight (77 against 93 us at 512x512x16).
+//   points on (C2R; R2C at 384 with eight 24.7 against 13.5).  R2C at 512 keeps
+//   eight: of the three lengths from 384 on it alone gains in small and large
+//   launches.  A field with eight / four: 512x512x16 734 / 753 us and 512x64x34
+//   187 / 194; 384x512x16 558 / 567 but 384x64x34 142 / 134, where the tile's 192
+//   threads are too few; 640x512x16 962 / 940 and 640x64x34 272 / 257, where its LDS
+//   leaves a CU one block.
 // - columns (107 MB out and in): 55 / 54 us at 32 points, 65 / 57 at 128,
 //   102 / 66 at 320, but 86 / 96 at 512 and within 5 % at 768 and 1024.
 // - axis 0 with the product (1.8 MB a plane): one lane a pencil up to 8
