@@ -25,11 +25,11 @@
 #include <stdio.h>
 
 #include <array>
-#include <map>
-#include <mutex>
 #include <string.h>
 
 #include <map>
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "hostcopy.hpp"
@@ -677,6 +677,9 @@ struct hs_demag {
     int logic[3], logicK[3];
     bool noalloc = false;     // hs_demag_field_f64_noalloc takes the mesh: its spectra at the logic size fit
     double* kernL = nullptr;  // kernel octants at the logic size where P differs, else kern64
+    // the FP64 fields at the logic size (its kern64 is kernL), where the spectra at P
+    // do not fit the static array of hs_demag_field_f64_noalloc
+    hs_demag* f64 = nullptr;
     double cell[3];
     int M, H2, H2p;  // H2p: spectrum row pitch (complex), a multiple of 16 = 128 bytes in FP32
     int KP;          // FP32 kernel row pitch (floats), a multiple of 32 = 128 bytes
@@ -1365,23 +1368,26 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
         int P[3];
         padded_lengths(N, d->logic, P);
         set_lengths(d, P);
-        if (d->noalloc && noalloc_bytes(d, fused_fold<double>(d)) > kScratchBytes) set_lengths(d, d->logic);
     }
     const int P0 = d->P[0], P1 = d->P[1], P2 = d->P[2], H2 = d->H2, H2p = d->H2p, M = d->M;
     const bool padded = P0 != d->logic[0] || P1 != d->logic[1] || P2 != d->logic[2];
     const long nk = (long)d->K[0] * d->K[1] * d->K[2];
     bool tables = make_twiddles(d, true);
-    hs_demag l;  // the transform at the logic size, for hs_demag_kernel_f64 alone
+    // the plan at the logic size: for hs_demag_kernel_f64, and for the FP64 fields where
+    // the padded ones would take them from hs_demag_field_f64_noalloc
+    std::unique_ptr<hs_demag, decltype(&hs_demag_destroy)> low(padded ? new hs_demag() : nullptr, hs_demag_destroy);
     if (padded) {
-        std::copy(d->logic, d->logic + 3, l.logic);
-        std::copy(d->logicK, d->logicK + 3, l.logicK);
-        set_lengths(&l, d->logic);
-        tables = make_twiddles(&l, false) && tables;
+        std::copy(d->N, d->N + 3, low->N);
+        std::copy(d->logic, d->logic + 3, low->logic);
+        std::copy(d->logicK, d->logicK + 3, low->logicK);
+        set_lengths(low.get(), d->logic);
+        tables = make_twiddles(low.get(), false) && tables;
     }
+    const bool low64 = padded && d->noalloc && noalloc_bytes(d, fused_fold<double>(d)) > kScratchBytes;
     hipMalloc(&d->kern64, sizeof(double) * 6 * nk);
     // HS_DEMAG_FORCE asks for particular five-pass variants
     d->fold32 = getenv("HS_DEMAG_FORCE") ? 0 : fused_fold<float>(d);
-    d->fold64 = fused_fold<double>(d);
+    d->fold64 = low64 ? 0 : fused_fold<double>(d);
     d->form32 = fused_form<float>(d, d->fold32);
     d->form64 = fused_form<double>(d, d->fold64);
     const long nk32 = (long)d->K[0] * d->K[1] * d->KP;
@@ -1422,7 +1428,6 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     if (!tables || !tmp || !d->kern64 || !d->X1f || (padded && !d->kernL) ||
         (!d->fold32 && (!d->kern32 || !d->X2f || (d->gen0 && !d->Xzf))) || (d->fold32 && !d->kt32) || (tab64 && !d->kt64)) {
         hipFree(tmp);
-        hipFree(l.tw);
         hs_demag_destroy(d);
         (void)hipGetLastError();
         if (padded) return demag_create(N, cell, pbc, accuracy, kernel, stream, false);
@@ -1460,9 +1465,12 @@ static hs_demag* demag_create(const int N[3], const double cell[3], const int pb
     const KernelBufs kb{oct, full, X, maxbits};
     kernel_transform(d, kb, d->kern64, d->kern32, st);
     if (padded) {
-        kernel_transform(&l, kb, d->kernL, nullptr, st);
+        kernel_transform(low.get(), kb, d->kernL, nullptr, st);
         hipStreamSynchronize(st);
-        hipFree(l.tw);
+        if (low64) {
+            low->kern64 = d->kernL;
+            d->f64 = low.release();
+        }
     }
     for (int c = 0; c < 6; c++) {
         if (gmax > 0 && cmax[c] / gmax < 1e-12) {
@@ -1506,6 +1514,10 @@ extern "C" hs_demag* hs_demag_create_newell(const int N[3], const double cell[3]
 
 extern "C" void hs_demag_destroy(hs_demag* d) {
     if (!d) return;
+    if (d->f64) {
+        d->f64->kern64 = nullptr;  // d's kernL
+        hs_demag_destroy(d->f64);
+    }
     void* ps[] = {d->kernL, d->kt32, d->kt64, d->kern64, d->kern32, d->X1f, d->X2f,
                   d->X1d,   d->X2d,  d->Xzf,  d->Xzd,    d->tw};
     for (void* p : ps)
@@ -1572,6 +1584,7 @@ extern "C" int hs_demag_field_f64(hs_demag* d, const double* m, const double* ms
         hs::set_error(HS_EINVAL, "hs_demag_field_f64");
         return HS_EINVAL;
     }
+    if (d->f64) d = d->f64;
     if (!d->X1d) {
         hipMalloc(&d->X1d, sizeof(cpx<double>) * fused_spectrum(d, d->fold64));
         if (!d->fold64) hipMalloc(&d->X2d, sizeof(cpx<double>) * 3L * d->N[0] * d->P[1] * d->H2p);
@@ -1642,6 +1655,7 @@ extern "C" int hs_demag_field_f64_noalloc(hs_demag* d, const double* m, const do
                                 "scratch; use hs_demag_field_f64");
         return HS_ESIZE;
     }
+    if (d->f64) d = d->f64;
     unsigned char* base = static_cast<unsigned char*>(scratch_address());
     if (!base) {
         hs::set_error(HS_EINVAL, "hs_demag_field_f64_noalloc: no device address for the static scratch");
@@ -1693,9 +1707,13 @@ long hs_demag_footprint(const hs_demag* d) {
     const long nk = (long)d->K[0] * d->K[1] * d->K[2];
     long b = 6 * nk * (long)sizeof(double);
     if (d->kern32) b += 6L * d->K[0] * d->K[1] * d->KP * (long)sizeof(float);
-    b += (long)sizeof(cpx<float>) * (fused_spectrum(d, d->fold32) + (d->X2f ? 3L * d->N[0] * d->P[1] * d->H2p : 0)) *
-         d->cap;
-    if (d->kernL) b += 6L * d->logicK[0] * d->logicK[1] * d->logicK[2] * (long)sizeof(double);
+    if (d->X1f)
+        b += (long)sizeof(cpx<float>) *
+             (fused_spectrum(d, d->fold32) + (d->X2f ? 3L * d->N[0] * d->P[1] * d->H2p : 0)) * d->cap;
+    if (d->f64)
+        b += hs_demag_footprint(d->f64);  // with its kern64, d's kernL
+    else if (d->kernL)
+        b += 6L * d->logicK[0] * d->logicK[1] * d->logicK[2] * (long)sizeof(double);
     if (d->kt32) b += fused_table(d, d->fold32) * (long)sizeof(float);
     if (d->kt64) b += fused_table(d, d->fold64) * (long)sizeof(double);
     if (d->X1d)

@@ -47,12 +47,16 @@ typedef struct hs_demag hs_demag;
  * 1/(P0 P1 P2) and stored in FP64 and FP32.  accuracy = 6 in the reference
  * (maxwell_convolution.go:96).  Blocks until the kernel is ready.
  * Any padded lengths up to 4095 (half the padded x length when it is even):
- * 2^k, 3*2^k and 5*2^k run compiled passes, tuned by timing where the mesh is
- * too large for the three-kernel convolution; an open axis of any other length
- * is padded to the next of them.  Lengths that cannot be (periodic axes with
- * factors 7, 9, 25 or larger primes, odd periodic x lengths, one-cell axes)
- * run passes that take the length at run time, as cuFFT plans do in the
- * reference (gpu/fftplanX.go:55-60).  Returns NULL on error (hs_last_error). */
+ * 2^k, 3*2^k and 5*2^k run compiled passes, tuned by timing where the mesh does
+ * not take the three-kernel convolution; an open axis of any other length is
+ * padded to the next of them.  Lengths that cannot be (periodic axes with
+ * factors 7, 9, 25 or larger primes, odd periodic x lengths, one-cell axes, open
+ * axes beyond 128 planes, 1024 rows or 2048 cells along x) run passes that take
+ * the length at run time, as cuFFT plans do in the reference
+ * (gpu/fftplanX.go:55-60); beside such an open axis the others are padded only
+ * where it pays, and FP64 fields stay at 2 N where only then
+ * hs_demag_field_f64_noalloc takes the mesh.  Returns NULL on error
+ * (hs_last_error). */
 HS_API hs_demag* hs_demag_create(const int N[3], const double cell[3], const int pbc[3], int accuracy,
                                  CUstream stream);
 /* The same plan with the Newell demag tensor instead of Kernel_Arne: no

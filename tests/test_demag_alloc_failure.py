@@ -119,7 +119,7 @@ def _run(tmp_path, child, **values):
 
 # three kernels; padded lengths in three kernels and in five passes; run-time lengths
 # (a one-cell axis).  None of these plans times its passes, which takes real events.
-@pytest.mark.parametrize("meshes,single", [([(2, 8, 16), (4, 64, 64)], True), ([(7, 75, 100), (3, 9, 7), (40, 9, 11)], False),
+@pytest.mark.parametrize("meshes,single", [([(2, 8, 16), (4, 64, 64)], True), ([(7, 75, 100), (3, 9, 7), (40, 9, 11), (24, 140, 110)], False),
                                            ([(4, 8, 1)], True)])
 def test_failed_allocations_are_reported_before_any_launch(tmp_path, meshes, single):
     _run(tmp_path, FAILURES, meshes=meshes, single=single)

@@ -130,3 +130,32 @@ def test_fixed_variants_of_padded_five_pass_plans(N, pbc, tiles):
     d.field_f32(P(m32), None, 8e5, P(Bf))
     assert relerr(host(Bf), host(B)) <= 2e-6  # FP32 round-off of transforms of up to 1280 points
     d.close()
+
+
+# meshes whose FP64 spectra fit the static array of hs_demag_field_f64_noalloc at 2 N but
+# not padded: three kernels, folded; five passes
+@pytest.mark.parametrize("N", [(24, 140, 110), (40, 129, 65)])
+def test_fp32_is_padded_where_fp64_stays_at_the_logic_size(N):
+    """The FP32 field runs compiled passes; both FP64 entries take the mesh and agree
+    bit for bit; the octant is that of 2 N."""
+    from oracle import pyoracle as po
+    n = N[0] * N[1] * N[2]
+    rng = np.random.default_rng(n)
+    m, msk = rng.standard_normal((3, n)), rng.random(n)
+    d, o = Demag(N, CELL), po.Demag(N, CELL)
+    assert d.P == o.P and d.K == o.K
+    assert _compiled(d) == (True, True, True)
+    assert relerr(d.kernel(), o.kernel()) <= 1e-12
+    want = o.B(m, msk, 8e5).reshape(3, n)
+    dm, dw = dev(m), dev(msk)
+    out = []
+    for field in (d.field_f64_noalloc, d.field_f64):
+        B = empty((3, n))
+        field(P(dm), P(dw), 8e5, P(B))
+        out.append(host(B))
+    assert np.array_equal(out[0], out[1])
+    assert relerr(out[0], want) <= 1e-12
+    m32, w32, Bf = dev(m, np.float32), dev(msk, np.float32), empty((3, n), torch.float32)
+    d.field_f32(P(m32), P(w32), 8e5, P(Bf))
+    assert relerr(host(Bf), want) <= 2e-6
+    d.close()
