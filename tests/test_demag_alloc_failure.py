@@ -80,6 +80,10 @@ for N in {meshes!r}:
         for k in range(n):  # allocation k alone, where there is no retry
             d, err, _, launches = plan(N, k, k + 1)
             assert not d and err == 10004 and launches == 0, (N, k, err, launches)
+    else:
+        for k in range(n):  # ... and where the retry gets what it asks for
+            d, err, calls, _ = plan(N, k, k + 1)
+            assert d and not err and calls > n, (N, k, err, calls)
 print("fine")
 """
 

@@ -165,6 +165,10 @@ def test_every_fp32_pass_variant_matches_fp64(monkeypatch, N, pbc):
 # passes (fft_any.hpp): prime factors 7, 11 and 13, 25 = 5^2 (a 100-cell axis
 # pads to 200 = 8 * 25), an odd x length of a periodic axis (P2 = 9), a one-cell
 # x extent (P2 = 1), and such lengths next to compiled ones.
+# An open axis of such a length is padded to the next compiled one: of the cases
+# below only the one-cell and the periodic axes (P2 = 1 and 9, P1 = 9) run passes at
+# run-time lengths; tests/test_gpu_demag_runtime.py holds more of those, axis 0
+# among them.
 GENERIC = [
     ((11, 8, 8), (2e-9, 2e-9, 2e-9), (0, 0, 0)),       # P0 = 22
     ((7, 7, 14), (2e-9, 3e-9, 2e-9), (0, 0, 0)),       # P = 14, 14, 28 (row FFT of 14)
@@ -205,6 +209,7 @@ def test_generic_length_solves_alone_in_a_batch_and_vs_oracle():
     """An LLB-r batch on a mesh whose axis-0 pass runs at a run-time length
     (P0 = 14, the spectrum of all P0 rows held per solve): each solve equals
     its solve alone bit for bit, and the oracle after 6 RK4 steps."""
+    # (that axis is padded to 16 points by now; test_gpu_demag_runtime.py has batches at P0 = 7 and 11)
     from hotspin_amd import workloads as W
     from hotspin_amd.api import Batch, Solver
     N, cell = (7, 8, 10), (2e-9, 2e-9, 2e-9)

@@ -3,6 +3,7 @@ directly) against the FP64 oracle, at the sizes where its tiling can go wrong:
 plane counts below, at and beyond one axis-0 item (1..8 planes, then blocks of
 6 and 8 with a remainder), column counts that leave a partial tile, row counts
 that leave a partial row block, each length family, masks and batches.
+(Batches and slots: test_gpu_demag_folded.py.)
 
 Bars: FP64 1e-12 of max|B| (as the five-pass convolution); FP32 2e-6, the
 round-off of FP32 transforms of up to 2048 points and sums of up to 3 N0
@@ -26,6 +27,8 @@ def _gpu():
 
 
 # folded axis 1 (FP32 beyond 2048 points of N0 P1, FP64 beyond 1024): 2, 4, 8 and 16 ways
+# (the folds compiled are 2, 4 and 8, in FP64 2 and 4; more than 16 planes on compiled
+# lengths do not fold in FP32)
 SHAPES = ([(16, 128, 8), (64, 64, 16), (8, 256, 16), (20, 96, 12), (33, 80, 10), (3, 512, 8), (16, 512, 16)] +
           [(n0, 8, 16) for n0 in range(1, 10)] +           # planes per item, first of the blocked form
           [(10, 8, 16), (12, 4, 8), (13, 8, 8), (16, 16, 8), (17, 4, 16), (33, 8, 8)] +
