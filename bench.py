@@ -237,9 +237,10 @@ def serving_leg(nreq, plain_steps=20, check_steps=5, policy="sjf", inflight_cell
                  "oracle_check": "first request of each shape class solved alone in a slot for %d adaptive RK23 "
                                  "steps vs the FP64 oracle" % check_steps,
                  "latency_note": "latency = done - arrival, queue = admission - arrival, service = done - "
-                                 "admission; the stream offers ~3e11 cell-steps in 10 s, about 12x what the device "
-                                 "serves in that time: requests are admitted within a second and then share the "
-                                 "device, so service time, not queue wait, makes up the latency",
+                                 "admission; the stream offers ~3e11 cell-steps in 10 s, several times what the "
+                                 "device serves in that time.  sjf admits the request with the least work first "
+                                 "under a cap on running cells, so the larger ones wait in the queue; fifo admits "
+                                 "all and they share the device",
                  "plain_sample": "%d RK23 steps of one request per shape class through hs_solver_run" % plain_steps})
     return summ
 
@@ -534,9 +535,17 @@ def main():
     s.set_m(m)
     torch.cuda.synchronize()
     log("bench: set-up %.2f s" % (time.time() - t0))
-    tiles = (C.c_int * 6)()
-    _lib.lib().hs_demag_tiles(_lib.lib().hs_solver_demag(s._h), tiles)
-    log("bench: demag tiles (W,NT) rows %s cols %s z %s" % (tuple(tiles[0:2]), tuple(tiles[2:4]), tuple(tiles[4:6])))
+    tiles, form = (C.c_int * 6)(), (C.c_int * 2)()
+    plan = _lib.lib().hs_solver_demag(s._h)
+    _lib.lib().hs_demag_tiles(plan, tiles)
+    _lib.lib().hs_demag_form(plan, form)
+    fold = form[0]
+    if fold:
+        demag = {"form": "three kernels", "axis1_fold": fold}
+    else:
+        demag = {"form": "five passes",
+                 "tiles": {"rows": list(tiles[0:2]), "cols": list(tiles[2:4]), "z": list(tiles[4:6])}}
+    log("bench: demag %s" % demag)
     stage_variant = {0: "march", 1: "flat", 2: "pair", 3: "flatz"}.get(_lib.lib().hs_solver_stage_variant(s._h), "?")
     log("bench: stage kernel variant %s" % stage_variant)
     dt = 1e-15
@@ -562,8 +571,7 @@ def main():
     L.hs_prof_enable(0)
     names = ["F1", "F2", "F3K", "I2", "I1", "STAGE"]
     P = (32, 1024, 1024)
-    # no F2 launches: the plan takes the three-kernel convolution, folded 8 ways at this mesh
-    pb = demag_pass_bytes(w["N"], P) if cnt[1] else demag_fused_bytes(w["N"], P, 8)
+    pb = demag_fused_bytes(w["N"], P, fold) if fold else demag_pass_bytes(w["N"], P)
     per = {}
     for i, nme in enumerate(names):
         if cnt[i]:
@@ -593,7 +601,7 @@ def main():
         "dtype": "f32",
         "data": "synthetic",
         "config": {"workload": w["name"], "cells": ncell, "method": "rk23", "rejected": st.rejected,
-                   "demag_tiles": {"rows": list(tiles[0:2]), "cols": list(tiles[2:4]), "z": list(tiles[4:6])},
+                   "demag": demag,
                    "stage_kernel": stage_variant,
                    "state": "f64", "fields": "f32", "reductions": "f64", "final_dt": dt},
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",

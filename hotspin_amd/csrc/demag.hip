@@ -1558,6 +1558,13 @@ extern "C" int hs_demag_variant_count(const hs_demag* d, int* out3) {
     return 0;
 }
 
+extern "C" int hs_demag_form(const hs_demag* d, int out2[2]) {
+    if (!d || !out2) return HS_EINVAL;
+    out2[0] = d->fold32;
+    out2[1] = d->fold64;
+    return 0;
+}
+
 extern "C" int hs_demag_tiles(const hs_demag* d, int* out6) {
     if (!d || !out6) return HS_EINVAL;
     out6[0] = d->row32.W;

@@ -78,6 +78,9 @@ HS_API int hs_demag_kernel_f64(const hs_demag* d, double* host_out);
 /* max |imag| / max |real| of the transformed kernel (the reference panics
  * above 1e-12, maxwell_convolution.go:383-385) */
 HS_API double hs_demag_max_imag_ratio(const hs_demag* d);
+/* How the plan convolves, FP32 and FP64 fields: 0 in five passes, R >= 1 in
+ * three kernels, with axis 1 folded by R */
+HS_API int hs_demag_form(const hs_demag* d, int out2[2]);
 /* FP32 tile shapes the plan's autotuner picked: (W, NT) of the row passes
  * (F1/I1), the column passes (F2/I2) and the axis-0 product pass (F3K) of the
  * five-pass form; the first variant's, untimed, in a three-kernel plan */

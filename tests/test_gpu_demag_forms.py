@@ -159,3 +159,14 @@ def test_fp32_is_padded_where_fp64_stays_at_the_logic_size(N):
     d.field_f32(P(m32), P(w32), 8e5, P(Bf))
     assert relerr(host(Bf), want) <= 2e-6
     d.close()
+
+
+@pytest.mark.parametrize("N,pbc,form", [((16, 512, 512), (0, 0, 0), [8, 0]), ((8, 256, 256), (0, 0, 0), [4, 4]),
+                                        ((4, 8, 16), (0, 0, 0), [1, 1]), ((4, 8, 16), (1, 0, 0), [0, 0]),
+                                        ((33, 8, 16), (0, 0, 0), [0, 0]), ((24, 140, 110), (0, 0, 0), [4, 0])])
+def test_form_that_a_plan_reports(N, pbc, form):
+    import ctypes as C
+    from hotspin_amd._lib import lib
+    d, out = Demag(N, CELL, pbc), (C.c_int * 2)()
+    assert lib().hs_demag_form(d._h, out) == 0 and list(out) == form
+    d.close()
