@@ -880,7 +880,8 @@ fused::Form<T> fused_form(const hs_demag* d, int R) {
     const fused::Rows<T>& r = fused::rows_of<T>(d->M);
     const fused::Mids<T>& m = fused::mids_of<T>(d->P[1] / R);
     const int f = fused::fold_index(R);
-    return {r.fwd[f], r.inv[f], m.pick(d->N[0], R > 1), m.A, m.B};
+    const bool few = R == 1 && d->N[0] > 8 && fused::mid_nt(d->N[0], d->P[1], 1, fused::kFewIB) <= fused::kMidMax;
+    return {r.fwd[f], r.inv[f], m.pick(d->N[0], R > 1), few ? m.few : nullptr, m.A, m.B};
 }
 // values of the fused spectrum (per solve) and of its kernel table
 long fused_spectrum(const hs_demag* d, int R) { return 3L * d->N[0] * (R > 1 ? d->P[1] : d->N[1]) * d->H2p; }
@@ -912,7 +913,8 @@ int run_fused(hs_demag* d, const T* m, const T* msk, double srcMul, T* B, hipStr
     const int ncol = d->H2 * R;
     const fused::Mid<T> a{X,    kt,     N0, N1, ncol, fused::mid_cb(N0, Q, fm.A, fm.B, ncol, nsolve, sizeof(cpx<T>)),
                           nsolve, R, tw1, live};
-    fm.mid(a, st);
+    const long waves = (long)ncol * nsolve * (fused::mid_nt(N0, Q, 1) / 64);
+    (fm.few && a.CB == 1 && waves < fused::kFewWaves ? fm.few : fm.mid)(a, st);
     hs::prof_end(HS_PROF_F3K, st);
     hs::prof_begin(HS_PROF_I1, st);
     fm.inv(X, B, g, twM, twP2, tw1, st, lrows);

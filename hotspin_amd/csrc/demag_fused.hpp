@@ -84,8 +84,17 @@ struct Coef {
 };
 __device__ __forceinline__ float fmaT(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fmaT(double a, double b, double c) { return __builtin_fma(a, b, c); }
+// Planes per item of unfolded FP32 launches that leave the chip mostly idle (fewer
+// than kFewWaves waves with the usual items of 6 or 8, one a thread): twice the
+// threads share the N0^2 products.  The sums are formed in the same order, so a
+// solve's bits do not depend on it.  One field with the usual items / with four
+// planes: 32^3 (132 waves) 25.1 / 21.1 us, 16x16x32 23.9 / 18.2, 64x64x16 22.7 /
+// 19.1, 512x8x32 (513) 33.6 / 28.7, 512x32x16 (1026) 33.7 / 30.2, but 256x64x9
+// (1028) 23.6 / 24.9 and 512x64x9 (2052) 31.5 / 34.9.
+constexpr int kFewIB = 4;
+constexpr long kFewWaves = 1024;
 // axis-0 items per thread: 3 IB values each, at most 24 in all
-constexpr int mid_itm(int IB) { return 8 / IB; }
+constexpr int mid_itm(int IB, bool multi = false) { return multi && IB == kFewIB ? 1 : 8 / IB; }
 
 // Shape of a column's tile.
 template <int Q_, bool FOLD>
@@ -116,7 +125,7 @@ __device__ __forceinline__ const T* table_row(const Mid<T>& a, const G& g, int t
 // three components at one slot (MULTI: N0 > IB).
 template <typename T, int IB, bool MULTI, bool FOLD, typename G>
 __device__ __forceinline__ void axis0(const Mid<T>& a, const G& g, cpx<T>* lds, int col0, int ncb) {
-    constexpr int ITM = mid_itm(IB);
+    constexpr int ITM = mid_itm(IB, MULTI);
     const int tid = threadIdx.x, NT = blockDim.x, N0 = a.N0, PC = 3 * N0, PL = g.PL;
     const int NIB = MULTI ? (N0 + IB - 1) / IB : 1, items = ncb * NIB * g.Q;
     cpx<T> y[ITM][3][IB];
@@ -212,7 +221,7 @@ __device__ __forceinline__ void axis0(const Mid<T>& a, const G& g, cpx<T>* lds, 
 // One block: CB columns of one solve, 3 N0 pencils of Q points each, held in
 // LDS as lds[pencil * A (B+1) + k1 (B+1) + k2] (the odd row pitch keeps both
 // phases free of bank conflicts).  Axis 0 in items of IB planes (MULTI: N0 >
-// IB); blockDim.x gives a thread mid_itm(IB) items, 15 to 24 elements, rounded up
+// IB); blockDim.x gives a thread mid_itm(IB) items, 12 to 24 elements, rounded up
 // to whole waves (mid_nt).
 template <typename T, int Q, int IB, bool MULTI, bool FOLD>
 __global__ void __launch_bounds__(kMidMax) k_fmid(Mid<T> a) {
@@ -840,8 +849,9 @@ inline int mid_ib(int N0) {
     return (N0 + 5) / 6 * 6 < (N0 + 7) / 8 * 8 ? 6 : 8;
 }
 // threads of a block: mid_itm axis-0 items each
-inline int mid_nt(int N0, int Q, int CB) {
-    const int IB = mid_ib(N0), items = CB * ((N0 + IB - 1) / IB) * Q, itm = mid_itm(IB);
+inline int mid_nt(int N0, int Q, int CB, int IB = 0) {
+    if (!IB) IB = mid_ib(N0);
+    const int items = CB * ((N0 + IB - 1) / IB) * Q, itm = mid_itm(IB, N0 > IB);
     return ((items + itm - 1) / itm + 63) / 64 * 64;
 }
 // whether a column of the mesh fits one block
@@ -874,8 +884,8 @@ inline long mid_elems(size_t cs) { return kTile * 8 / (long)cs; }
 // than fold.  One field, folded / five passes: 64x64x24 30.3 / 27.2 us,
 // 96x96x24 39.5 / 35.1, 256x64x20 46.0 / 39.2, 128x128x32 62.4 / 52.8; RK4 steps
 // of batches are between 0.9 (64x256x20) and 1.14 (512x64x24) times as long.
-// Without folding, batches decide: one field of 32^3 takes 25.1 us against
-// 20.3, but a step of 64 solves 729 us against 945.  A plan at padded lengths has
+// Without folding, three kernels up to 32 planes: one field of 32^3 takes 21.1 us
+// against 20.3, a step of 64 solves 729 us against 945.  A plan at padded lengths has
 // untimed passes, and folds (96x96x30: a step of 8 solves 789 us against 893).
 template <typename F>
 int mid_fold(int N0, int P1, size_t cs, bool timed, F fits) {
@@ -921,6 +931,7 @@ template <typename T>
 struct Mids {
     mid_t<T> one[2][9] = {};    // [folded] N0 = 1..8 planes
     mid_t<T> multi[2][9] = {};  // more, in blocks of 6 or 8
+    mid_t<T> few = nullptr;     // more, in blocks of kFewIB, unfolded
     int A = 0, B = 0;
     mid_t<T> pick(int N0, bool fold) const {
         return N0 <= 8 ? one[fold][N0] : multi[fold][mid_ib(N0)];
@@ -934,6 +945,7 @@ struct Form {
     frows_t<T> fwd = nullptr;
     irows_t<T> inv = nullptr;
     mid_t<T> mid = nullptr;
+    mid_t<T> few = nullptr;  // mid for launches of few waves, null where it has none
     int A = 0, B = 0;  // split of the mid kernel's columns
 };
 // registries (demag.hip): the entry to fill at library load, and the entry of a
@@ -987,7 +999,7 @@ template <typename T, int Q, int IB, bool MULTI, bool FOLD>
 void launch_mid(const Mid<T>& m, hipStream_t st) {
     constexpr int A = split_even(Q).A, B = split_even(Q).B;
     const size_t lds = mid_lds(Q, A, B, m.N0, m.CB, sizeof(cpx<T>));
-    const int nt = mid_nt(m.N0, Q, m.CB);
+    const int nt = mid_nt(m.N0, Q, m.CB, IB);
     if (lds > 65536)
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fmid<T, Q, IB, MULTI, FOLD>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -1033,6 +1045,7 @@ void add_mid() {
         Mids<T>& m = add_mids_of<T>(Q);
         m.A = split_even(Q).A;
         m.B = split_even(Q).B;
+        if constexpr (sizeof(T) == 4 && Q <= kMidMax) m.few = &launch_mid<T, Q, kFewIB, true, false>;
         add_mid_fold<T, Q, false>(m);
         add_mid_fold<T, Q, true>(m);
     }

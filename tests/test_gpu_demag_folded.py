@@ -99,3 +99,27 @@ def test_plane_counts_match_oracle(N):
     # FP32 transforms of up to 256 points and sums of up to 96 products
     assert relerr(host(B), want) <= 2e-6
     d.close()
+
+
+# unfolded, more than eight planes: items of four planes in a launch of fewer than 1024 waves
+# (the solve alone), of six or eight beyond (the batch); plane counts that fill items of each
+# size and that do not
+@pytest.mark.parametrize("N,k", [((32, 32, 32), 9), ((24, 32, 16), 24), ((9, 16, 16), 64), ((13, 12, 10), 96),
+                                 ((20, 8, 16), 64), ((31, 10, 12), 96)])
+def test_small_and_large_launches_give_the_same_bits(N, k):
+    kw = W.llbr_params(T=300.0, seed=5, material=MAT)
+    T, m = _states(N, k)
+    seeds = np.arange(k, dtype=np.uint64) + 11
+    b = Batch(N, CELL, k, TMuls=T, seeds=seeds, **kw)
+    b.set_m(m)
+    _, h = b.rhs()
+    b.run("rk4", 1, 2e-15)
+    mb = b.get_m()
+    b.close()
+    for q in (0, k // 2, k - 1):
+        s = Solver(N, CELL, **dict(kw, TMul=float(T[q]), seed=int(seeds[q])))
+        s.set_m(m[q])
+        assert np.array_equal(s.rhs()[1], h[q]), q
+        s.run("rk4", 1, 2e-15)
+        assert np.array_equal(s.get_m(), mb[q]), q
+        s.close()
